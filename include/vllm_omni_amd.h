@@ -388,7 +388,7 @@ int mi_mask_logits_argmax(void* logits, int64_t* ids, int32_t num_tokens, int32_
  *                  (+ g * shared_out[t], g = sigmoid(x[t] . shared_gate_weight) or 1).
  * ---------------------------------------------------------------------- */
 enum { MI_MOE_PLAIN = 0, MI_MOE_GATED = 1, MI_MOE_RELU_SQUARED = 2 };
-int32_t mi_moe_rows_per_tile(int32_t num_tokens, int32_t top_k, int32_t num_experts); /* 32, 64 or (prefill chunks) 256 */
+int32_t mi_moe_rows_per_tile(int32_t num_tokens, int32_t top_k, int32_t num_experts); /* 32, 64 or 256 */
 int64_t mi_moe_max_rows(int32_t num_tokens, int32_t top_k, int32_t num_experts, int32_t rows_per_tile);
 int mi_moe_route(int32_t* topk_ids, float* topk_weights, int32_t* expert_counts, const void* router_logits,
                  const float* bias /* [num_experts], added to the logits, or NULL */, int32_t num_tokens, int32_t num_experts, int64_t logits_row_stride, int32_t top_k,

@@ -145,3 +145,40 @@ def test_align_groups_pairs_by_expert(dev, rpt, T, given_counts):
     assert torch.equal(rop_c[live].long(), live_rows)                                 # and row_of_pair is the inverse
     assert int((sp_c < 0).sum()) == n_tiles * rpt - T * k                             # everything else is -1 padding
     assert (te_c[1:] >= te_c[:-1]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k", [(128, 128), (384, 256), (640, 384), (1152, 4096)])   # weight tiles that hang over, 2 and 64 k blocks
+@pytest.mark.parametrize("form", ["gated", "plain", "relu_squared"])
+def test_tall_tiles_give_the_rows_of_low_ones(dev, dtype, n, k, form):
+    """An expert's row does not depend on the tile it is in, bit for bit: experts of 0 to 513 rows (every edge of the 64-row units a
+    tall tile counts) through tiles of 64, 128 and 256 rows against tiles of 32, gathered and plain, with a row's own factor."""
+    from vllm_omni_amd import _C, ops
+
+    lib = _C.lib
+    sizes = [1, 63, 64, 0, 65, 128, 129, 192, 193, 255, 256, 257, 513]
+    E, top = len(sizes), 3
+    pairs = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes))
+    pairs = torch.cat([pairs, torch.full((-len(pairs) % top,), 2)])
+    g = torch.Generator().manual_seed(n + k)
+    ids = pairs[torch.randperm(len(pairs), generator=g)].to(torch.int32).to(dev).view(-1, top)
+    T, f = ids.shape[0], {"gated": _C.MI_MOE_GATED, "plain": _C.MI_MOE_PLAIN, "relu_squared": _C.MI_MOE_RELU_SQUARED}[form]
+    w = (torch.randn(E, (2 if form == "gated" else 1) * n, k, generator=g) * k ** -0.5).to(dtype).to(dev)
+    x = torch.randn(T * top if form == "plain" else T, k, generator=g).to(dtype).to(dev)
+    pw = torch.rand(T * top, generator=g).to(dev) if form == "relu_squared" else None
+    got = []
+    for rpt in (32, 64, 128, 256):
+        rows = int(lib.mi_moe_max_rows(T, top, E, rpt))
+        sp, rop, te, nt = ops._moe_align(ids, E, rows, rpt)
+        a = x
+        if form == "plain":      # the grouped rows themselves
+            a = torch.zeros(rows, k, dtype=dtype, device=dev)
+            a[rop.long()] = x
+        out = torch.full((rows, n), float("nan"), dtype=dtype, device=dev)
+        ops.check("mi_moe_expert_gemm", lib.mi_moe_expert_gemm(
+            out.data_ptr(), a.data_ptr(), w.data_ptr(), sp.data_ptr(), te.data_ptr(), nt.data_ptr(), rows // rpt, f,
+            None if pw is None else pw.data_ptr(), n, k, top, a.stride(0), out.stride(0), w.stride(0), rpt, ops._dt(dtype),
+            torch.cuda.current_stream().cuda_stream))
+        got.append(out[rop.long()])
+    assert not got[0].isnan().any() and got[0].abs().max() > 0
+    assert all(torch.equal(got[0], o) for o in got[1:])

@@ -460,10 +460,10 @@ extern "C" int32_t mi_moe_rows_per_tile(int32_t num_tokens, int32_t top_k, int32
   // The fragments-from-global kernel (MI_MOE_GEMM=direct) is faster with 32-row tiles at every size measured.
   const char* e = getenv("MI_MOE_GEMM");
   if (e && strcmp(e, "direct") == 0) return 32;
-  // Prefill chunks (an expert sees hundreds of rows): 256-row tiles stream an expert's weights 4x less often than 64-row
-  // ones — 459 against 497 us at 8192 tokens, 277 / 294 at 4096, level at 2048, behind at 1024
-  // (profiles/r03w_moe_tall_tiles.log); the gain is small because K is short here (1024 / 384: 16 / 6 ring steps per tile)
-  if ((int64_t)num_tokens * top_k >= 256 * (int64_t)num_experts) return 256;
+  // Past 48 rows an expert, 256-row tiles (tall_gemm.hip counts a tile's live rows in units of 64): both products at 64 rows an
+  // expert 523 -> 362 us (4096 x 1536), 144 -> 124 (2048 x 768), 117 -> 97 (1024 x 384), at 128 rows 877 -> 400, 238 -> 138,
+  // 199 -> 113; at 48 rows 359 / 341, 107 / 117, 81 / 88.  128-row tiles are level up to 96 rows and behind from there.
+  if ((int64_t)num_tokens * top_k > 48 * (int64_t)num_experts) return 256;
   return (int64_t)num_tokens * top_k > 24 * (int64_t)num_experts ? 64 : 32;
 }
 
@@ -566,7 +566,13 @@ extern "C" int mi_moe_expert_gemm(void* out, const void* a_rows, const void* wei
       ga.rows_per_tile = rows_per_tile;
       ga.a_row_stride = a_row_stride; ga.out_row_stride = out_row_stride; ga.weight_expert_stride = weight_expert_stride;
       ga.dtype = dtype;
-      const int rc = launch_grouped_skinny(ga, s);
+      // Tall tiles on tall_gemm.hip; the ring kernel keeps them for k of an odd number of 64-blocks and operands past 32-bit
+      // offsets.  64-row tiles (24 to 48 rows an expert) are weight streaming: the tall kernel's 256-row weight tiles are ahead
+      // where an expert's product is large (4096 x 1536: 357 -> 335 us for both products), the ring's 128-row ones where it is
+      // small (2048 x 768: 105 against 115, 1024 x 384: 80 against 87)
+      const bool tall = rows_per_tile > 64 || (rows_per_tile == 64 && (int64_t)n_out * k >= (4 << 20));
+      int rc = tall ? launch_grouped_tall(ga, s) : MI_ERR_UNSUPPORTED;
+      if (rc == MI_ERR_UNSUPPORTED) rc = launch_grouped_skinny(ga, s);
       if (rc != MI_ERR_UNSUPPORTED) return rc;
     }
   }

@@ -560,8 +560,8 @@ int launch_skinny(const SkinnyParams& p_in, const SkinnyPlan& pl, bool gated, in
   return launch_status();
 }
 
-// MT: 16-row m-tiles of a tile's row image: 4 (<= 64 token rows per tile: decode batches), 8 / 16 (128 / 256 rows: prefill
-// chunks, where an expert sees hundreds of rows and a 64-row tile would stream its weights 8-16 times)
+// MT: 16-row m-tiles of a tile's row image: 4 (<= 64 token rows per tile: decode batches), 8 / 16 (128 / 256 rows: what
+// tall_gemm.hip does not take)
 template <typename Tag, bool GATED, int MT>
 int launch_grouped_t(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
   constexpr int MH = MT == 4 ? 1 : 2;

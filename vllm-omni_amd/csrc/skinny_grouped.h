@@ -23,5 +23,7 @@ struct GroupedGemmArgs {
 // MI_OK, or MI_ERR_UNSUPPORTED when the shape is outside the ring kernel's envelope (the caller then runs its
 // direct-from-global kernel).
 int launch_grouped_skinny(const GroupedGemmArgs& a, hipStream_t s);
+// Tiles of 64, 128 or 256 rows (tall_gemm.hip); MI_ERR_UNSUPPORTED outside its envelope.
+int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s);
 
 }  // namespace mi
