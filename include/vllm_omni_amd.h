@@ -603,6 +603,14 @@ int mi_linear_silu_mul(void* out, const void* x, const void* weight, int32_t m, 
 int mi_linear_clamped_glu(void* out, const void* x, const void* weight, int32_t m, int32_t inter,
                           int32_t k, int64_t x_row_stride, int64_t out_row_stride, float alpha,
                           float limit, int dtype, void* stream);
+/* y = x W^T (+ bias), or the gated form of mi_linear_silu_mul (n = inter), for
+ * any number of rows on 256 x 256 tiles (tall_gemm.hip): prefill chunks.  k a
+ * multiple of 128, n of 16; strides multiples of 8; x and the weight each under
+ * 4 GiB (MI_ERR_UNSUPPORTED past that).  The workspace (0 bytes: none) is scratch. */
+int64_t mi_linear_tall_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated);
+int mi_linear_tall(void* out, const void* x, const void* weight, const void* bias, int32_t m,
+                   int32_t n, int32_t k, int64_t x_row_stride, int64_t out_row_stride, int32_t gated,
+                   void* workspace, int64_t workspace_bytes, int dtype, void* stream);
 /* Tile plans measured for a deployment's shapes (tools/tune_linear_plans.py ->
  * vllm_omni_amd/tuned/linear_plans_gfx950.json), replacing the built-in heuristic of the
  * three entry points above for 16-bit operands — the counterpart of the TunableOp

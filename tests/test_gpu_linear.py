@@ -422,3 +422,46 @@ def test_in_launch_splitk_reduce_equals_the_reduce_launch_bit_for_bit(plan_regis
         monkeypatch.setattr(ops, "LINEAR_FUSED_REDUCE", True)
         torch.cuda.synchronize()
         assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,gated", [
+    (257, 3584, 9472, False),     # 28 tiles: every one cut along K, the last row tile holds one row
+    (300, 256, 18944, False), (1, 16, 128, False),
+    (520, 33024, 512, False),     # 387 tiles: 256 whole ones and a last round in pieces too short to cut
+    (700, 24576, 2048, False),    # 288 tiles: a whole round and 32 tiles in pieces, with a bias
+    (1030, 16448, 256, True), (640, 144, 384, True)])     # columns that hang over the last tile
+def test_tall_linear_matches_float64(dev, dtype, m, n, k, gated):
+    from vllm_omni_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(m + n)
+    new = lambda *s: torch.randn(*s, generator=g, device=dev)   # noqa: E731
+    x = new(m, k + 8).to(dtype)[:, :k]      # rows further apart than they are long
+    w = (new((2 if gated else 1) * n, k) * k ** -0.5).to(dtype)
+    b = new(n).to(dtype) if (m, gated) == (700, False) else None
+    got = ops.linear_tall(x, w, b, gated).double()
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11      # half a step of the type, relative
+    ref = x.double() @ w.double().t()
+    # sums of k products in 32 bits: k steps of 2^-24 of what has been summed, at most sum |x w|
+    near = (x.double().abs() @ w.double().abs().t()) * k * 2.0 ** -24
+    if not gated:
+        ref = ref + (0 if b is None else b.double())
+        assert ((got - ref).abs() <= eps * ref.abs() + near + 1e-6).all()
+        return
+    (gt, up), (ng, nu) = ref.split(n, 1), near.split(n, 1)
+    ref = gt * torch.sigmoid(gt) * up
+    # both products are rounded to the type first; silu's slope is at most 1.1
+    bound = 1.1 * (eps * gt.abs() + ng) * (up.abs() * (1 + eps) + nu) + gt.abs() * (eps * up.abs() + nu) + 1.01 * eps * ref.abs()
+    assert ((got - ref).abs() <= 1.05 * bound + 1e-5).all()
+
+
+def test_tall_linear_takes_what_it_is_ahead_on(monkeypatch):
+    from vllm_omni_amd import layers, tuned
+
+    monkeypatch.setattr(layers, "_LINEAR_MODE", "auto")
+    monkeypatch.setattr(tuned, "_done", True)
+    bf = torch.bfloat16
+    assert layers._tall_wins(257, 3584, 18944, bf) and layers._tall_wins(6719, 18944, 3584, bf, gated=True)
+    assert not layers._tall_wins(256, 3584, 18944, bf) and not layers._tall_wins(8192, 3584, 18944, bf)      # selected by measurement
+    assert not layers._tall_wins(768, 18944, 3584, bf, gated=True) and not layers._tall_wins(6719, 3584, 3584, bf)
+    assert not layers._tall_wins(300, 3584, 18944, torch.float32) and not layers._tall_wins(120_000, 3584, 18944, bf)

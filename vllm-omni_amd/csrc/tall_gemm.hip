@@ -1,5 +1,5 @@
-// Grouped matrix products whose row tiles are tall: an expert's rows times its weights where an expert sees dozens of rows or
-// more (prefill chunks, large decode batches).  y = x W^T in the swapped form of skinny_gemm.hip, D = W . x^T, on the same
+// Matrix products whose row tiles are tall: an expert's rows times its weights where an expert sees dozens of rows or more, and
+// plain linears of prefill chunks (with SiLU and the product with the up projection, or cut along K).  y = x W^T in the swapped form of skinny_gemm.hip, D = W . x^T, on the same
 // LDS image of 128-byte rows (16-byte chunk c of row r at c ^ ((r >> 1) & 7): conflict-free for 32-row fragments as well).
 //
 // What bounds it: the matrix cores, and through them the power limit (at 90 % of busy matrix cores the chip runs at 1.37 GHz).
@@ -16,7 +16,7 @@
 //   * A row tile's live rows are counted in units of 64: four code paths, so that an expert's last tile costs what it holds.
 // Experts' both products, 4096 x 1536, 64 experts, 8 chosen (relu squared): 8192 rows 2176 -> 1603 us, 1024 rows 877 -> 400 us;
 // gated, 6 chosen: 8192 rows 2289 -> 1819 us, 1365 rows 1213 -> 533 us; 1024 x 384, 128 experts, 8 chosen: 2048 rows 199 -> 113 us
-// (before: the ring kernel's 64- and 256-row tiles).
+// (before: the ring kernel's 64- and 256-row tiles).  Linears beside the library's: layers.py, _tall_wins.
 #include "mfma_attn_common.h"
 #include "skinny_grouped.h"
 #include "skinny_tile.h"
@@ -37,7 +37,17 @@ struct TallParams {
   const int32_t* num_tiles;     // [1]
   const float* pair_weights;    // RELU_SQUARED: the sums of a pair's row times this, in front of the activation
   int64_t ldx, ldo, w_expert_stride;
+  // DENSE: one weight matrix, all M rows.  The first `whole` tiles are items of their own; each of the others is cut along K into
+  // `split` items that leave fp32 sums in part [item][256][256]
+  int32_t M, whole, split, group;
+  const uint16_t* bias;
+  float* part;
 };
+
+// FORM of a dense product (the others are MI_MOE_*)
+constexpr int kTallDense = 16, kTallDenseGated = 17;
+constexpr bool tall_dense(int form) { return form >= kTallDense; }
+constexpr bool tall_gated(int form) { return form == MI_MOE_GATED || form == kTallDenseGated; }
 
 constexpr int kTallN = 256;       // weight rows of a tile
 constexpr int kTallStage = 64 * 1024;
@@ -45,11 +55,49 @@ constexpr int kTallStage = 64 * 1024;
 // the part of a work item that its place decides; row: the item's 8 x pieces' rows of a_rows, as the alignment's map has them
 struct TallItem {
   int row0, tile, expert, units;     // units: 64-row units of the row tile that hold live rows
+  int kb, n_it;                      // where the item starts along K (bytes) and its 64-wide blocks: an even number
+  int slab;                          // >= 0: fp32 sums into this slab
   int row[8];
 };
 
-__device__ __forceinline__ void tall_fetch(const TallParams& p, int item, TallItem& t) {
+// items of the XCD-th of eight workgroup sets: a range of the whole tiles, then a range of the pieces
+__device__ __forceinline__ int tall_items(const TallParams& p, bool dense, int xcd, int& lo, int& whole, int& tail) {
+  const int work = dense ? p.whole : p.num_tiles[0] * p.nx, each = (work + 7) >> 3;
+  lo = xcd * each;
+  whole = max(min(each, work - lo), 0);
+  tail = 0;
+  if (dense && p.split > 1) {
+    const int pieces = (((p.M + 255) >> 8) * p.nx - p.whole) * p.split, per = (pieces + 7) >> 3;
+    tail = xcd * per;
+    return whole + max(min(per, pieces - tail), 0);
+  }
+  return whole;
+}
+
+template <int FORM>
+__device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo, int whole, int tail, TallItem& t) {
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  t.kb = 0;
+  t.n_it = p.K >> 6;
+  t.slab = -1;
+  if constexpr (tall_dense(FORM)) {
+    int at = lo + item;
+    if (item >= whole) {
+      t.slab = tail + item - whole;
+      const int s = t.slab % p.split, nb = p.K >> 7, b0 = s * nb / p.split;
+      at = p.whole + t.slab / p.split;
+      t.kb = b0 * 256;
+      t.n_it = 2 * ((s + 1) * nb / p.split - b0);
+    }
+    // `group` row tiles by the weight tiles, rows first: what an XCD's 32 workgroups read at a time
+    const int tiles = (p.M + 255) >> 8, g = at / (p.group * p.nx), in = at - g * p.group * p.nx, rows = min(p.group, tiles - p.group * g);
+    t.tile = in / rows;
+    t.row0 = (p.group * g + in - t.tile * rows) * 256;
+    t.units = min((p.M - t.row0 + 63) >> 6, 4);
+    t.expert = 0;
+    return;
+  }
+  item += lo;
   const int row_tile = item / p.nx;      // the weight tiles of a row tile in a row: its rows through one L2
   t.tile = item - row_tile * p.nx;
   t.row0 = row_tile * p.rpt;
@@ -67,12 +115,17 @@ __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, TallIt
 }
 
 // byte offsets of a lane's 8 x pieces
+template <int FORM>
 __device__ __forceinline__ void tall_rows(const TallParams& p, const TallItem& t, uint32_t (&x)[8]) {
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int row = 8 * (wid + 4 * i) + (lane >> 3);
     const int lc = (lane & 7) ^ ((row >> 1) & 7);
+    if constexpr (tall_dense(FORM)) {     // a row past the last one repeats it and is never stored
+      x[i] = (uint32_t)min(t.row0 + row, p.M - 1) * (uint32_t)(2 * p.ldx) + 16 * lc;
+      continue;
+    }
     uint32_t m = t.row[i] < 0 ? 0u : (uint32_t)t.row[i];
     if (p.gather_div > 1) m = __umulhi(m, p.div_magic);      // / gather_div
     x[i] = m * (uint32_t)(2 * p.ldx) + 16 * lc;
@@ -112,13 +165,13 @@ template <typename Tag, int FORM, int HM>
 __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s1, char* so, const TallItem& t, uint32_t (&x)[8],
                                           const uint32_t (&wo)[8], const TallItem& nt, bool more) {
   using E = Elem<Tag>;
-  constexpr bool GATED = FORM == MI_MOE_GATED;
+  constexpr bool GATED = tall_gated(FORM);
   constexpr int NM = 8 * HM;                 // products of half a step
   constexpr int PPL = 8 + 2 * HM;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wid & 1, wn = wid >> 1;
-  const int n_it = p.K >> 6;
+  const int n_it = t.n_it;
   const int r32 = lane & 31, half = lane >> 5;
   int frag[4];
 #pragma unroll
@@ -173,7 +226,7 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     __builtin_amdgcn_s_waitcnt(kLgkm0);
     barrier();                                   // everybody has read this stage
     // (loads spread over the step: a wave that finds the memory pipe's queue full issues no product either)
-    const int kb = KIND == 0 ? (it + 2) * 128 : (KIND - 1) * 128;
+    const int kb = KIND == 0 ? t.kb + (it + 2) * 128 : nt.kb + (KIND - 1) * 128;
     if (KIND == 0 || more) tall_issue_w(wo, wr, kb, cur);
     if (KIND == 2) {
       if (more) tall_issue_x<8>(p, x, kb, cur);
@@ -221,7 +274,7 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     step(K0{}, it + 1, s1, s0);
   }
   if (more) {
-    tall_rows(p, nt, x);
+    tall_rows<FORM>(p, nt, x);
     wr = tall_weights<GATED>(p, nt);
   }
   step(K1{}, n_it - 2, s0, s1);
@@ -230,6 +283,21 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
   // Lane: row r32 of x tile j, columns 8 q + 4 half + 0 .. 3 of W tile g in registers 4 q .. 4 q + 3.  A wave turns 32 rows at a
   // time in its 8 KB of LDS and stores whole row segments (16-byte chunk c of row r at c ^ (r & 7)).
   constexpr int CW = GATED ? 64 : 128;           // columns of a wave
+  if constexpr (FORM == kTallDense) {
+    if (t.slab >= 0) {
+      float* const to = p.part + (int64_t)t.slab * 65536 + wn * 128 + 4 * half;
+#pragma unroll
+      for (int j = 0; j < HM; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4_t*>(to + (32 * (wm * HM + j) + r32) * 256 + 32 * g + 8 * q) =
+                f32x4_t{acc[g][j][4 * q], acc[g][j][4 * q + 1], acc[g][j][4 * q + 2], acc[g][j][4 * q + 3]};
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      return;
+    }
+  }
   char* const mine = so + wid * 8192;
   const int n0 = t.tile * (2 * CW) + wn * CW;
 #pragma unroll
@@ -246,14 +314,21 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     for (int g = 0; g < 4; ++g) {
 #pragma unroll
       for (int q = 0; q < (GATED ? 2 : 4); ++q) {
-        float v[4];
+        float v[4], bv[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (FORM == kTallDense) {
+          if (p.bias) {
+            const int n = n0 + 32 * g + 8 * q + 4 * half;
+            const uint2 w = *reinterpret_cast<const uint2*>(p.bias + (n < p.N ? n : 0));
+            bv[0] = E::lo(w.x), bv[1] = E::hi(w.x), bv[2] = E::lo(w.y), bv[3] = E::hi(w.y);
+          }
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           if constexpr (GATED) {      // a W tile is 16 gate rows and the up rows of the same columns
             const float gt = E::from_bits(E::to_bits(acc[g][j][4 * q + r])), up = E::from_bits(E::to_bits(acc[g][j][8 + 4 * q + r]));
             v[r] = gt / (1.f + __expf(-gt)) * up;
           } else {
-            v[r] = acc[g][j][4 * q + r];
+            v[r] = acc[g][j][4 * q + r] + bv[r];
             if constexpr (FORM == MI_MOE_RELU_SQUARED) {
               v[r] = fmaxf(v[r] * pw, 0.f);
               v[r] *= v[r];
@@ -271,28 +346,28 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
       const int at = 64 * i + lane, r = at / per, c = at % per;
       const u32x4_t o = *reinterpret_cast<const u32x4_t*>(mine + r * (2 * CW) + ((c ^ (r & 7)) << 4));
       const int n = n0 + 8 * c;
-      if (n < p.N) *reinterpret_cast<u32x4_t*>(p.out + (int64_t)(m0 + r) * p.ldo + n) = o;
+      if (n < p.N && (!tall_dense(FORM) || m0 + r < p.M)) *reinterpret_cast<u32x4_t*>(p.out + (int64_t)(m0 + r) * p.ldo + n) = o;
     }
   }
-  // the next item's two stages came before the stores (which a wave past the last column does not issue)
+  // the next item's two stages came before the stores (which a wave past the last column or row does not issue)
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  if (n0 + CW <= p.N) __builtin_amdgcn_s_waitcnt(vmcnt_imm(CW / 16 * HM));
+  if (n0 + CW <= p.N && (!tall_dense(FORM) || t.row0 + 64 * HM <= p.M)) __builtin_amdgcn_s_waitcnt(vmcnt_imm(CW / 16 * HM));
   else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 }
 
 template <typename Tag, int FORM>
 __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
   scalar_cache_acquire();
-  constexpr bool GATED = FORM == MI_MOE_GATED;
+  constexpr bool GATED = tall_gated(FORM);
   __shared__ __attribute__((aligned(1024))) char s0[kTallStage];
   __shared__ __attribute__((aligned(1024))) char s1[kTallStage];
   __shared__ __attribute__((aligned(1024))) char so[32768];
   // every XCD has a contiguous range of the items, its workgroups take them in turn
-  const int work = p.num_tiles[0] * p.nx, each = (work + 7) >> 3;
-  const int hi = min((int)((blockIdx.x & 7) + 1) * each, work), stride = gridDim.x >> 3;
-  int item = (blockIdx.x & 7) * each + (blockIdx.x >> 3);
-  if (item >= hi) return;
+  int lo, whole, tail;
+  const int items = tall_items(p, tall_dense(FORM), blockIdx.x & 7, lo, whole, tail), stride = gridDim.x >> 3;
+  int item = blockIdx.x >> 3;
+  if (item >= items) return;
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t x[8], wo[8];
 #pragma unroll
@@ -302,14 +377,14 @@ __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
     wo[i] = (uint32_t)n * (uint32_t)(2 * p.K) + 16 * ((lane & 7) ^ ((row >> 1) & 7));
   }
   TallItem t, nt;
-  tall_fetch(p, item, t);
-  tall_rows(p, t, x);
+  tall_fetch<FORM>(p, item, lo, whole, tail, t);
+  tall_rows<FORM>(p, t, x);
   {
     const __amdgpu_buffer_rsrc_t wr = tall_weights<GATED>(p, t);
-    tall_issue_w(wo, wr, 0, s0);
-    tall_issue_x<8>(p, x, 0, s0);
-    tall_issue_w(wo, wr, 128, s1);
-    tall_issue_x<8>(p, x, 128, s1);
+    tall_issue_w(wo, wr, t.kb, s0);
+    tall_issue_x<8>(p, x, t.kb, s0);
+    tall_issue_w(wo, wr, t.kb + 128, s1);
+    tall_issue_x<8>(p, x, t.kb + 128, s1);
   }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   while (true) {
@@ -317,9 +392,9 @@ __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     item += stride;
-    const bool more = item < hi;
+    const bool more = item < items;
     nt = t;
-    if (more) tall_fetch(p, item, nt);
+    if (more) tall_fetch<FORM>(p, item, lo, whole, tail, nt);
     if (t.units >= 4) tall_tile<Tag, FORM, 4>(p, s0, s1, so, t, x, wo, nt, more);
     else if (t.units == 3) tall_tile<Tag, FORM, 3>(p, s0, s1, so, t, x, wo, nt, more);
     else if (t.units == 2) tall_tile<Tag, FORM, 2>(p, s0, s1, so, t, x, wo, nt, more);
@@ -327,6 +402,31 @@ __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
     if (!more) break;
     t = nt;
   }
+}
+
+// the pieces' sums of a tile cut along K, in order (+ bias); a workgroup has 8 rows of a tile, a thread 8 columns
+template <typename Tag>
+__global__ __launch_bounds__(256) void tall_reduce_kernel(const TallParams p) {
+  scalar_cache_acquire();
+  using E = Elem<Tag>;
+  const int cut = blockIdx.x >> 5, at = p.whole + cut;
+  const int tiles = (p.M + 255) >> 8, g = at / (p.group * p.nx), in = at - g * p.group * p.nx, rows = min(p.group, tiles - p.group * g);
+  const int tile = in / rows, r = 8 * (blockIdx.x & 31) + (threadIdx.x >> 5), c = 8 * (threadIdx.x & 31);
+  const int m = (p.group * g + in - tile * rows) * 256 + r, n = tile * kTallN + c;
+  if (m >= p.M || n >= p.N) return;
+  f32x4_t v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
+  const float* from = p.part + (int64_t)cut * p.split * 65536 + r * 256 + c;
+  for (int s = 0; s < p.split; ++s, from += 65536) {
+    v0 += *reinterpret_cast<const f32x4_t*>(from);
+    v1 += *reinterpret_cast<const f32x4_t*>(from + 4);
+  }
+  if (p.bias) {
+    const uint4 b = *reinterpret_cast<const uint4*>(p.bias + n);
+    v0 += f32x4_t{E::lo(b.x), E::hi(b.x), E::lo(b.y), E::hi(b.y)};
+    v1 += f32x4_t{E::lo(b.z), E::hi(b.z), E::lo(b.w), E::hi(b.w)};
+  }
+  *reinterpret_cast<uint4*>(p.out + (int64_t)m * p.ldo + n) =
+      make_uint4(E::pack(v0[0], v0[1]), E::pack(v0[2], v0[3]), E::pack(v1[0], v1[1]), E::pack(v1[2], v1[3]));
 }
 
 template <typename Tag>
@@ -346,7 +446,7 @@ int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s) {
   // 32-bit byte offsets into the rows (a gathered row's number is at most its pair's) and into one expert's weights
   const int64_t rows = (int64_t)a.max_tiles * a.rows_per_tile, lim = (int64_t)1 << 32;
   if (rows >= 1 << 28 || rows * a.a_row_stride * 2 >= lim || (int64_t)(gated ? 2 : 1) * a.n_out * a.k * 2 >= lim) return MI_ERR_UNSUPPORTED;
-  TallParams p;
+  TallParams p{};
   p.x = reinterpret_cast<const uint16_t*>(a.a_rows);
   p.w = reinterpret_cast<const uint16_t*>(a.weights);
   p.out = reinterpret_cast<uint16_t*>(a.out);
@@ -369,3 +469,76 @@ int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s) {
   return a.dtype == MI_DTYPE_BF16 ? launch_tall<bf16_tag>(p, a.form, grid, s) : launch_tall<f16_tag>(p, a.form, grid, s);
 }
 }  // namespace mi
+
+namespace {
+// Tiles of one round more than fill the 256 CUs but not a whole number of rounds: the last round's tiles are cut along K so that it
+// takes a fraction of a round, at the price of fp32 sums written and read.
+struct TallCut {
+  int tiles, whole, split;
+};
+TallCut tall_cut(int32_t m, int32_t n, int32_t k, bool gated) {
+  TallCut c;
+  const int cols = gated ? mi::kTallN / 2 : mi::kTallN;
+  c.tiles = ((m + 255) / 256) * ((n + cols - 1) / cols);
+  const int last = c.tiles % 256;
+  c.split = last && !gated ? 256 / last : 1;
+  if (c.split > k / 512) c.split = k / 512;      // at least eight blocks a piece
+  if (c.split > 8) c.split = 8;
+  if (c.split < 2) c.split = 1;
+  c.whole = c.split > 1 ? c.tiles - last : c.tiles;
+  return c;
+}
+bool tall_linear_ok(int32_t m, int32_t n, int32_t k, int64_t ldx, bool gated, int dtype) {
+  const int64_t lim = (int64_t)1 << 32;
+  return k % 128 == 0 && n % 16 == 0 && (dtype == MI_DTYPE_BF16 || dtype == MI_DTYPE_F16) && (int64_t)m * ldx * 2 < lim &&
+         (int64_t)(gated ? 2 : 1) * n * k * 2 < lim;
+}
+}  // namespace
+
+extern "C" int64_t mi_linear_tall_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated) {
+  if (m <= 0 || n <= 0 || k <= 0) return 0;
+  const TallCut c = tall_cut(m, n, k, gated != 0);
+  return c.split > 1 ? (int64_t)(c.tiles - c.whole) * c.split * 65536 * 4 : 0;
+}
+
+extern "C" int mi_linear_tall(void* out, const void* x, const void* weight, const void* bias, int32_t m, int32_t n, int32_t k,
+                              int64_t x_row_stride, int64_t out_row_stride, int32_t gated, void* workspace, int64_t workspace_bytes,
+                              int dtype, void* stream) {
+  using namespace mi;
+  if (m == 0) return MI_OK;
+  if (!out || !x || !weight || m < 0 || n <= 0 || k <= 0 || (gated && bias)) return MI_ERR_INVALID_ARG;
+  if (x_row_stride < k || out_row_stride < n || x_row_stride % 8 || out_row_stride % 8) return MI_ERR_INVALID_ARG;
+  if (((uintptr_t)out | (uintptr_t)x | (uintptr_t)weight | (uintptr_t)bias | (uintptr_t)workspace) & 15) return MI_ERR_INVALID_ARG;
+  if (!tall_linear_ok(m, n, k, x_row_stride, gated != 0, dtype)) return MI_ERR_UNSUPPORTED;
+  const TallCut c = tall_cut(m, n, k, gated != 0);
+  if (workspace_bytes < mi_linear_tall_workspace_bytes(m, n, k, gated) || (c.split > 1 && !workspace)) return MI_ERR_INVALID_ARG;
+  TallParams p{};
+  p.x = reinterpret_cast<const uint16_t*>(x);
+  p.w = reinterpret_cast<const uint16_t*>(weight);
+  p.out = reinterpret_cast<uint16_t*>(out);
+  p.bias = reinterpret_cast<const uint16_t*>(bias);
+  p.part = reinterpret_cast<float*>(workspace);
+  p.M = m;
+  p.N = n;
+  p.K = k;
+  p.rpt = 256;
+  p.nx = (n + (gated ? kTallN / 2 : kTallN) - 1) / (gated ? kTallN / 2 : kTallN);
+  p.whole = c.whole;
+  p.split = c.split;
+  p.group = 8;
+  p.ldx = x_row_stride;
+  p.ldo = out_row_stride;
+  const int64_t items = c.whole + (int64_t)(c.tiles - c.whole) * c.split;
+  const dim3 grid(items < 256 ? (int)((items + 7) / 8 * 8) : 256), block(256);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+#define MI_TALL(TAG)                                                                                     \
+  do {                                                                                                   \
+    if (gated) hipLaunchKernelGGL((tall_gemm_kernel<TAG, kTallDenseGated>), grid, block, 0, s, p);       \
+    else hipLaunchKernelGGL((tall_gemm_kernel<TAG, kTallDense>), grid, block, 0, s, p);                  \
+    if (c.split > 1) hipLaunchKernelGGL((tall_reduce_kernel<TAG>), dim3(32 * (c.tiles - c.whole)), block, 0, s, p); \
+  } while (0)
+  if (dtype == MI_DTYPE_BF16) MI_TALL(bf16_tag);
+  else MI_TALL(f16_tag);
+#undef MI_TALL
+  return launch_status();
+}

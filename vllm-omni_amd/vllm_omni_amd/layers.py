@@ -377,6 +377,24 @@ def _streaming_kernel_wins(m: int, n: int, k: int) -> bool:
     return m <= 256 and n <= 2048 and k <= 4096 and k > 2 * n and n * k >= (1 << 20)
 
 
+def _tall_wins(m: int, n: int, k: int, dtype: torch.dtype, gated: bool = False) -> bool:
+    """Whether a prefill chunk's product runs on ``ops.linear_tall`` instead of the library.  Measured at the talker's shapes, 257 to
+    8192 rows: the library's default choice for a long K behind few columns is slow (3584 x 18944: 257 rows 97 us against 75, 512 rows
+    179 / 82, 2500 rows 528 / 348, 6719 rows 1191 / 679), and the gate with SiLU in the same launch is ahead from two rounds of tiles on
+    (18944 x 3584, 1000 rows 316 / 253, 6719 rows 1497 / 1403; 512 rows 148 / 167).  Where the library's solution was selected by
+    measurement at exactly this row count it keeps the shape (3584 x 18944, 8192 rows 794 / 853), and so it does elsewhere (3584 x 3584,
+    6719 rows 129 / 165; 4096 x 16384 0.9 to 2.1 times as fast)."""
+    from .tuned import has_tuned_gemm
+
+    if m <= 256 or _LINEAR_MODE != "auto" or not ops.linear_tall_supported(m, n, k, dtype, gated):
+        return False
+    if has_tuned_gemm(m, 2 * n if gated else n, k, dtype):
+        return False
+    if gated:
+        return k >= 2048 and -(-m // 256) * -(-n // 128) >= 512
+    return n >= 2048 and k >= 8192 and k > 4 * n
+
+
 def fused_gate_up_silu(layer, x: torch.Tensor, clamped: Optional[tuple[float, float]] = None) -> Optional[torch.Tensor]:
     """``act_fn(gate_up_proj(x))`` in one launch (``ops.linear_silu_mul``) when the policy picks the streaming kernel
     for this shape, else None (the caller runs the GEMM and ``SiluAndMul`` apart).  Column-parallel, no bias, 16-bit
@@ -401,6 +419,8 @@ def fused_gate_up_silu(layer, x: torch.Tensor, clamped: Optional[tuple[float, fl
     w = layer.weight
     m = x.numel() // x.shape[-1]
     n, k = w.shape
+    if clamped is None and n % 2 == 0 and _tall_wins(m, n // 2, k, x.dtype, gated=True):
+        return ops.linear_tall(x, w, gated=True)
     if n % 32 or not ops.linear_supported(m, n // 2, k, x.dtype):
         return None
     e = _tuned(m, n // 2, k, gated=True)
@@ -463,6 +483,8 @@ def _apply_linear(layer, x: torch.Tensor, bias: Optional[torch.Tensor], defer_re
     if _LINEAR_MODE != "library" and x.is_cuda:
         m = x.numel() // x.shape[-1]
         n, k = w.shape
+        if _tall_wins(m, n, k, x.dtype):
+            return ops.linear_tall(x, w, bias)
         e = _tuned(m, n, k) if ops.linear_supported(m, n, k, x.dtype) else None
         if e is not None and e.get("full"):
             # measured at this shape: the cheapest of {library, kernel + its reduce launch, partials reduced downstream}

@@ -871,6 +871,31 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor, clamped: Optional[tup
     return out.view(*x.shape[:-1], inter)
 
 
+def linear_tall_supported(m: int, n: int, k: int, dtype: torch.dtype, gated: bool = False) -> bool:
+    """Shape envelope of ``mi_linear_tall``: x and the weight each under 4 GiB"""
+    return (k % 128 == 0 and n % 16 == 0 and dtype in (torch.bfloat16, torch.float16) and m * k < 1 << 31
+            and (2 if gated else 1) * n * k < 1 << 31)
+
+
+def linear_tall(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, gated: bool = False) -> torch.Tensor:
+    """``linear`` (``gated``: ``linear_silu_mul``) for the rows of a prefill chunk: the 256 x 256 tiles of csrc/tall_gemm.hip"""
+    _gpu(x, weight, bias)
+    x2 = x.reshape(-1, x.shape[-1])
+    if x2.stride(-1) != 1 or x2.stride(0) % 8:
+        x2 = x2.contiguous()
+    m, k = x2.shape
+    n = weight.shape[0] // 2 if gated else weight.shape[0]
+    if weight.shape[1] != k or (gated and weight.shape[0] % 2) or not weight.is_contiguous() or weight.dtype != x.dtype:
+        raise ValueError("weight must be a contiguous [n, k] (gated: [2 n, k]) tensor of x's dtype")
+    if bias is not None and (bias.shape != (n,) or bias.dtype != x.dtype or not bias.is_contiguous()):
+        raise ValueError("bias must be a contiguous [n] tensor of x's dtype")
+    out = torch.empty(m, n, dtype=x.dtype, device=x.device)
+    need = int(lib.mi_linear_tall_workspace_bytes(m, n, k, int(gated)))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check("mi_linear_tall", lib.mi_linear_tall(_p(out), _p(x2), _p(weight), _p(bias), m, n, k, x2.stride(0), out.stride(0), int(gated),
+                                               _p(ws), need, _dt(x.dtype), _stream()))
+    return out.view(*x.shape[:-1], n)
+
 
 INT8_TILE_ROWS = 512   # rows one launch of the tiled W8A8 kernel takes
 

@@ -3,7 +3,10 @@ tools/tune_gemms.py).  Loading them only changes WHICH hipBLASLt / rocBLAS solut
 runs; tuning itself is off at run time, and shapes not in the file use the library default."""
 from __future__ import annotations
 
+import functools
 import os
+
+import torch
 
 _DIR = os.path.dirname(os.path.abspath(__file__))
 RESULTS = os.path.join(_DIR, "tunableop_gfx950.csv")
@@ -30,3 +33,21 @@ def enable_tuned_gemms() -> bool:
         return _done
     except Exception:  # noqa: BLE001 - an older torch or a validator mismatch: library defaults
         return False
+
+
+@functools.lru_cache(maxsize=1)
+def _selected() -> frozenset:
+    """(type, n, m, k) of the y[m, n] = x W^T products in the file"""
+    names, found = {"BFloat16": torch.bfloat16, "Half": torch.float16}, set()
+    with open(RESULTS) as f:
+        for line in f:
+            op, shape = (line.split(",") + [""])[:2]
+            parts = shape.split("_")
+            if op.startswith("GemmTunableOp_") and op.endswith("_TN") and parts[0] == "tn" and len(parts) >= 4:
+                found.add((names.get(op.split("_")[1]), *map(int, parts[1:4])))
+    return frozenset(found)
+
+
+def has_tuned_gemm(m: int, n: int, k: int, dtype: torch.dtype) -> bool:
+    """Whether the library's product of exactly this shape runs a solution selected by measurement."""
+    return _done and (dtype, n, m, k) in _selected()
