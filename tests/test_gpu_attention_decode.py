@@ -302,6 +302,46 @@ def test_fused_merge_equals_the_two_kernel_merge_bit_for_bit(dev):
         assert torch.equal(out, want), step
 
 
+@pytest.mark.parametrize("form", ["plain", "rope", "biased"])
+@pytest.mark.parametrize("d,ps,parts", [(128, 64, 2), (128, 32, 5), (64, 32, 8), (64, 96, 3)])
+def test_partitions_merged_in_their_workgroup_equal_the_two_launches_bit_for_bit(dev, d, ps, parts, form):
+    """A bound of at most five (head_dim 64: eight) partitions merges inside the workgroup when the batch covers half the chip
+    or the contexts are short; nine partitions of the same size, the last of them empty, take the merge launch: the same sums
+    in the same order.  Sequences end on, before and behind every partition's edge, and two are empty."""
+    from vllm_omni_amd import ops
+    from vllm_omni_amd.layers import build_cos_sin_cache
+
+    nkv, bs, dtype = 2, 16, torch.bfloat16
+    for nq, S in ((2, 65), (14, 128), (32, 2)):
+        edges = [1, ps - 1, ps, ps + 1, parts * ps - 1, parts * ps, (parts - 1) * ps, (parts - 1) * ps + 1, 17]
+        if S == 2 and parts * ps * d > 256 * 128:
+            continue
+        lens = [parts * ps, 0] if S == 2 else [edges[i % len(edges)] for i in range(S - 2)] + [0, 0]
+        _, kb, vb, table, q, _ = _mk_case(S, nq, nkv, d, bs, [max(n, 1) for n in lens], dtype, seed=3)
+        kb, vb, seq_lens = kb.to(dev), vb.to(dev), torch.tensor(lens, dtype=torch.int32, device=dev)
+        table, q = table.to(dev), q.reshape(S, nq * d).to(dev)
+        g = torch.Generator().manual_seed(4)
+        new = torch.randn(S, 2 * nkv * d, generator=g).to(dtype).to(dev)
+        pos = torch.tensor([max(n - 1, 0) for n in lens], device=dev)
+        slots = torch.tensor([int(table[i, (n - 1) // bs]) * bs + (n - 1) % bs if n > 0 else -1 for i, n in enumerate(lens)], device=dev)
+        slopes, sinks = torch.rand(nq, generator=g).to(dev) * 0.1, torch.randn(nq, generator=g).to(dev)
+        outs = []
+        for msl in (parts * ps, 9 * ps):
+            kc, vc = kb.clone(), vb.clone()
+            out = torch.full((S, nq * d), float("nan"), dtype=dtype, device=dev)
+            if form == "rope":
+                ops.rope_cache_paged_attn_decode(out, q, new[:, : nkv * d], new[:, nkv * d:], pos, build_cos_sin_cache(d, 8192, 1e6, device=dev),
+                                                 kc, vc, slots, table, seq_lens, msl, d ** -0.5, partition_size=ps)
+            else:
+                bias = {"slopes": slopes, "sinks": sinks} if form == "biased" else {}
+                ops.paged_attn_decode(out, q, kc, vc, table, seq_lens, msl, d ** -0.5, partition_size=ps, **bias)
+            torch.cuda.synchronize()
+            outs.append((out, kc, vc))
+        for one, two in zip(*outs):
+            assert torch.equal(one, two), (nq, S)
+        assert not torch.isnan(outs[0][0].float()).any() and not outs[0][0][-1].any()      # empty sequences: zeros
+
+
 @pytest.mark.parametrize("bs,d,lens", [(32, 128, [4500, 2047, 2049, 4096]),      # windows of 2048 tokens
                                          (64, 64, [8200, 4095, 4097, 4096]),       # windows of 4096 tokens, head_dim 64
                                          (16, 64, [3000, 1025, 2048, 1024])])

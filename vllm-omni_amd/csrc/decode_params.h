@@ -43,9 +43,12 @@ struct DecodeParams {
   const float* slopes = nullptr;
   const float* sinks = nullptr;
   float out_scale = 1.f;   // the output times this (matrix-core kernel and the merge)
+  bool group_parts = false;   // matrix-core kernel: the partitions are the waves of a workgroup and merge there
 };
 
 // paged_attn_decode_mfma.hip
+// whether to set p.group_parts; groups = sequences x head groups
+bool decode_mfma_groups(int64_t groups, int num_parts, int head_dim, int max_seq_len);
 int launch_decode_mfma(const DecodeParams& p, int heads_per_wave, int head_dim, int dtype, bool nontemporal,
                        bool split_p, hipStream_t stream);
 // the same launch with RoPE + KV write inside (p.k_new etc. set); nontemporal + split-P form only

@@ -21,6 +21,7 @@
 //   * tiles of 16 tokens, register double-buffered: the loads of tile t+1 are in
 //     flight while tile t is computed (8 KiB per wave in flight).
 //   * partitions of the context are merged by `decode_reduce_kernel`.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -486,8 +487,12 @@ extern "C" int32_t mi_paged_attn_decode_auto_partition(int32_t num_seqs, int32_t
   // pipeline fill), an fp32 partial write and its share of the merge launch, so take the FEWEST partitions that still
   // leave >= 512 waves (two per CU) — ONE when (sequences x KV heads) >= 512: direct output, no partials, no merge
   // (B 256 / ctx 4096: 315 us against 340 with four partitions of 1024; fewer than 512 waves loses: 256 waves run at
-  // 55 % of that rate).  Never below 256 tokens, never above 8192 (a bound on the tail when ONE sequence of a batch is
+  // 55 % of that rate).  Never above 8192 (a bound on the tail when ONE sequence of a batch is
   // far longer than the rest: one wave streams its whole partition).
+  // Three partitions or more go below 256 tokens, to an eighth of the context or 64: a wave takes about 0.95 us per 32 tokens
+  // whatever the others do, so a small batch's launch lasts as long as its longest partition.  28 / 4 heads, cold KV, at least 256 |
+  // this: 1 x 150 9.0 | 6.8 us, 1 x 1000 14.3 | 10.9, 8 x 1000 15.1 | 11.8, 23 x up to 800 16.4 | 14.2, 32 x up to 150 9.7 | 8.7; two of
+  // 64 lose to one (120 x up to 120: 11.1 against 10.4), and more than eight make the merge longer than what they save.
   // head_dim 64: a wave's ring holds half the bytes, so twice the waves (>= 1024: 128 sequences x 2 heads x ctx 4096 run
   // 46.6 us in four partitions against 54.5 in two; 512 x 2 heads stay at ONE: profiles/r03zb_decode_parts_d64.log)
   if (num_seqs <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 256;
@@ -495,7 +500,8 @@ extern "C" int32_t mi_paged_attn_decode_auto_partition(int32_t num_seqs, int32_t
   const int64_t want = head_dim > 0 && head_dim <= 64 ? 1024 : 512;
   const int64_t parts = (want + pairs - 1) / pairs;
   int64_t ps = mi::round_up((int32_t)((max_seq_len + parts - 1) / parts), 32);
-  if (ps < 256) ps = 256;
+  const int64_t least = parts < 3 ? 256 : std::min(256, std::max(64, mi::round_up((int32_t)(((int64_t)max_seq_len + 7) / 8), 32)));
+  if (ps < least) ps = least;
   if (ps > 8192) ps = 8192;
   if (ps > mi::round_up(max_seq_len, 32)) ps = mi::round_up(max_seq_len, 32);
   return (int32_t)ps;  // kernels that keep a partition's block ids in ONE register cap it at 64 blocks (below)
@@ -602,6 +608,8 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
                   (int64_t)num_seqs * num_q_heads * (int64_t)sizeof(int32_t) <= MI_DECODE_COUNTER_BYTES)
                      ? reinterpret_cast<int32_t*>(workspace)
                      : nullptr;
+  p.group_parts = use_mfma && decode_mfma_groups((int64_t)num_seqs * (num_q_heads / G), num_parts, head_dim, max_seq_len);
+  if (p.group_parts) p.part_count = nullptr;
   p.num_seqs = num_seqs;
   p.num_q_heads = num_q_heads;
   p.kv_group = kv_group;
@@ -650,7 +658,7 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
                          : dispatch_group<f16_tag, 64>(p, G, packed, s);
   }
   if (rc != MI_OK) return rc;
-  if (p.part_count) return MI_OK;   // merged inside the launch
+  if (p.part_count || p.group_parts) return MI_OK;   // merged inside the launch
   if (flags & MI_DECODE_SKIP_MERGE) return MI_OK;   // measurement of the attention kernel alone
   if (dtype == MI_DTYPE_BF16)
     return head_dim == 128 ? launch_reduce<bf16_tag, 128>(p, s) : launch_reduce<bf16_tag, 64>(p, s);

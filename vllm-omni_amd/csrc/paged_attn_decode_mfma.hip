@@ -129,8 +129,30 @@ __device__ __forceinline__ float item_sumsq(const uint4& xr, const uint4& yr) {
 
 // BIAS: a distance bias and a sink.  The bias is the MFMA's C operand — S^T = K . Q^T + slope / scale * (key - position) — so
 // the softmax does not know of it; the sink is what partition 0 starts its running maximum and sum from.
-template <typename Tag, int HD, int AUX, bool SPLIT, int NS, bool ROPE = false, bool NORM = false, bool BIAS = false>
-__global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p, const int gh) {
+// GROUP: the context partitions of a sequence's head group are the waves of ONE workgroup, each with a ring of its own, and merge
+// through LDS with decode_reduce_kernel's arithmetic (the same bits): no partials in memory, no merge launch behind this one (4.8 us in a
+// graph).  The waves of a group share one CU's loads, though (it sustains about 40 GB/s of these rows), where single-wave workgroups spread
+// over the chip; decode_mfma_groups holds the line between the two.
+constexpr int kCUs = 256, kLdsBytes = 160 * 1024;
+template <int HD>
+constexpr int ring_bytes = (HD == 128 ? 2 : MI_DECODE_NS64) * 2 * kStep * HD * 2;
+template <int HD>
+constexpr int group_parts_max = kLdsBytes / ring_bytes<HD> < 8 ? kLdsBytes / ring_bytes<HD> : 8;   // head_dim 128: five; 64: eight
+// The rings' LDS: static for a lone wave, whose DMA destinations are then constants.  The addresses of both start at 0.
+using lds_float = __attribute__((address_space(3))) float;
+using lds_char = __attribute__((address_space(3))) char;   // a generic pointer costs a null check at each DMA's cast
+template <bool GROUP, int BYTES>
+__device__ __forceinline__ lds_char* ring_base() {
+  if constexpr (GROUP) {
+    extern __shared__ __attribute__((aligned(1024))) char rings[];      // [waves][BYTES]
+    return (lds_char*)rings;
+  } else {
+    __shared__ __attribute__((aligned(1024))) char ring[BYTES];
+    return (lds_char*)ring;
+  }
+}
+template <typename Tag, int HD, int AUX, bool SPLIT, int NS, bool ROPE = false, bool NORM = false, bool BIAS = false, bool GROUP = false>
+__global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void decode_mfma_kernel(const DecodeParams p, const int gh) {
   scalar_cache_acquire();
   using E = Elem<Tag>;
   constexpr int ROWB = HD * 2;        // bytes per token row of one head
@@ -141,11 +163,12 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
   constexpr int IPS = 16 / RPI;       // DMA instructions per 16-row sub-tile: 4 / 2
   constexpr int IMG = kStep * ROWB;   // one K or V image of a stage (8 KiB)
   constexpr int STAGE = 2 * IMG;      // K image + V image
-  __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
-
-  const int lane = threadIdx.x;
-  const int wave = blockIdx.x;
-  const int part = wave % p.num_parts;
+  const int lane = GROUP ? threadIdx.x & 63 : threadIdx.x;
+  const int wid = GROUP ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  lds_char* const rings = ring_base<GROUP, NS * STAGE>();
+  lds_char* const smem = rings + wid * (NS * STAGE);
+  const int wave = GROUP ? blockIdx.x * p.num_parts + wid : blockIdx.x;
+  const int part = GROUP ? wid : wave % p.num_parts;
   const int hw = (wave / p.num_parts) % (p.num_q_heads / gh);
   const int seq = wave / (p.num_parts * (p.num_q_heads / gh));
   const int qh0 = hw * gh;
@@ -176,6 +199,40 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
   uint16_t* const out16 = reinterpret_cast<uint16_t*>(p.out);
   float* const out32 = reinterpret_cast<float*>(p.out);
 
+  // GROUP: the partitions' (m, l, O^T) lie in their waves' rings; heads are dealt to the waves.  decode_reduce_kernel's arithmetic.
+  const auto merge_group = [&]() {
+    __syncthreads();
+    constexpr int DPL = HD / 64;
+    const int np = min(p.num_parts, (steps_total + part_steps - 1) / part_steps);   // partitions that hold tokens
+    for (int hh = wid; hh < gh; hh += p.num_parts) {
+      float mm = -3.0e38f;
+      for (int i = 0; i < np; ++i) mm = fmaxf(mm, ((const lds_float*)(rings + i * (NS * STAGE)))[16 * HD + 2 * hh]);
+      float L = 0.f, a[DPL];
+#pragma unroll
+      for (int d = 0; d < DPL; ++d) a[d] = 0.f;
+      for (int i = 0; i < np; ++i) {
+        const lds_float* of = (const lds_float*)(rings + i * (NS * STAGE));
+        const float w = fast_exp2(of[16 * HD + 2 * hh] - mm);
+        L += w * of[16 * HD + 2 * hh + 1];
+#pragma unroll
+        for (int d = 0; d < DPL; ++d) a[d] += w * of[hh * HD + (((lane * DPL) >> 2) ^ hh) * 4 + ((lane * DPL) & 3) + d];
+      }
+      const float inv = np > 0 ? p.out_scale / L : 0.f;
+      const int64_t o = (int64_t)seq * p.out_stride + (int64_t)(qh0 + hh) * HD + lane * DPL;
+#pragma unroll
+      for (int d = 0; d < DPL; ++d) {
+        const float r = a[d] * inv;
+        if (p.out_f32) out32[o + d] = r;
+        else out16[o + d] = E::to_bits(r);
+      }
+    }
+  };
+  if constexpr (GROUP) {
+    if (t_begin >= t_end) {
+      merge_group();
+      return;
+    }
+  }
   if (t_begin >= t_end) {
     // Empty partition.  seq_len == 0 has no partition at all: the direct launch and, with the fused merge, the wave of
     // partition 0 write the zeros (without the fused merge decode_reduce_kernel does).
@@ -269,7 +326,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
   const int sw_h = swz_k<HD>(h);
   uint32_t k_rd[KS];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) k_rd[s] = (uint32_t)(h * ROWB + (((4 * s + g) ^ sw_h) * 16));
+  for (int s = 0; s < KS; ++s) k_rd[s] = (uint32_t)(wid * (NS * STAGE) + h * ROWB + (((4 * s + g) ^ sw_h) * 16));
   // V transposed read (A operand of PV): group g, lane i = 4q + pp supplies row 4g + q (+16 j),
   // dims 16n + 4pp .. +3  -> logical chunk 2n + (pp>>1), 8 B half (pp&1)
   const int q4 = (lane & 15) >> 2, pp = lane & 3;
@@ -278,7 +335,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
   uint32_t v_rd[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n)
-    v_rd[n] = (uint32_t)(IMG + v_row * ROWB + (((2 * n + (pp >> 1)) ^ sw_v) * 16) + 8 * (pp & 1));
+    v_rd[n] = (uint32_t)(wid * (NS * STAGE) + IMG + v_row * ROWB + (((2 * n + (pp >> 1)) ^ sw_v) * 16) + 8 * (pp & 1));
 
   const char* const kbase_b = reinterpret_cast<const char*>(p.k_cache);
   const char* const vbase_b = reinterpret_cast<const char*>(p.v_cache);
@@ -309,7 +366,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
       const char* src = kbase_b + subtile_base(t * kStep + 16 * j);
 #pragma unroll
       for (int ii = 0; ii < IPS; ++ii) {
-        char* kdst = smem + st * STAGE + (16 * j + RPI * ii) * ROWB;
+        lds_char* kdst = smem + st * STAGE + (16 * j + RPI * ii) * ROWB;
         __builtin_amdgcn_global_load_lds((gbl_void*)(src + src_off_k[ii]), (lds_void*)kdst, 16, 0, AUX);
         src += grp_bytes;
       }
@@ -323,7 +380,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
         const char* src = vbase_b + subtile_base(t * kStep + 16 * j);
 #pragma unroll
         for (int ii = 0; ii < IPS; ++ii) {
-          char* vdst = smem + st * STAGE + IMG + (16 * j + RPI * ii) * ROWB;
+          lds_char* vdst = smem + st * STAGE + IMG + (16 * j + RPI * ii) * ROWB;
           __builtin_amdgcn_global_load_lds((gbl_void*)(src + src_off_v[ii]), (lds_void*)vdst, 16, 0, AUX);
           src += grp_bytes;
         }
@@ -335,7 +392,7 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
       for (int j = 0; j < 2; ++j) {
 #pragma unroll
         for (int ii = 0; ii < IPS; ++ii) {
-          char* vdst = smem + st * STAGE + IMG + (16 * j + RPI * ii) * ROWB;
+          lds_char* vdst = smem + st * STAGE + IMG + (16 * j + RPI * ii) * ROWB;
           const int row0 = t * kStep + 16 * j + RPI * ii;
           const int tok = min(row0 + lane / LPR, limit - 1);              // per lane
           const int blk_u = min(row0, limit - 1) >> p.bs_log2;              // wave-uniform
@@ -550,6 +607,19 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
 
   // ---- epilogue ---------------------------------------------------------------------------------
   l = rows_allreduce_sum(l);
+  if constexpr (GROUP) {      // the ring has no reader and no load in flight any more
+    if (head_ok) {
+      lds_float* const po = (lds_float*)smem;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) *(__attribute__((address_space(3))) f32x4_t*)(po + h * HD + (((4 * n + g) ^ h) * 4)) = acc[n];   // 16-byte chunks
+      if (g == 0) {
+        po[16 * HD + 2 * h] = m;
+        po[16 * HD + 2 * h + 1] = l;
+      }
+    }
+    merge_group();
+    return;
+  }
   if (direct) {
     if (!head_ok) return;
     const float inv = p.out_scale / l;
@@ -633,64 +703,62 @@ __global__ __launch_bounds__(64, 2) void decode_mfma_kernel(const DecodeParams p
   }
 }
 
+// one wave a workgroup, or (group) the partitions of a sequence's head group as the waves of one
+template <typename Tag, int HD, int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool BIAS = false>
+int launch_form(const DecodeParams& p, int gh, hipStream_t stream) {
+  constexpr int NS = HD == 128 ? 2 : MI_DECODE_NS64, ring = ring_bytes<HD>;
+  static_assert(ring >= (16 * HD + 32) * 4, "a wave's partial takes its ring's place");
+  const int64_t groups = (int64_t)p.num_seqs * (p.num_q_heads / gh);
+  if (groups * p.num_parts > INT32_MAX) return MI_ERR_UNSUPPORTED;
+  if (p.group_parts) {
+    auto kern = decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, true>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       group_parts_max<HD> * ring);
+    if (attr != hipSuccess) return MI_ERR_LAUNCH;
+    hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(64 * p.num_parts), p.num_parts * ring, stream, p, gh);
+  } else {
+    hipLaunchKernelGGL((decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS>), dim3((unsigned)(groups * p.num_parts)), dim3(64), 0,
+                       stream, p, gh);
+  }
+  return launch_status();
+}
+template <int AUX, bool SPLIT, bool ROPE = false, bool NORM = false>
+int launch_types(const DecodeParams& p, int gh, int head_dim, int dtype, hipStream_t stream) {
+  if (dtype == MI_DTYPE_BF16)
+    return head_dim == 128 ? launch_form<bf16_tag, 128, AUX, SPLIT, ROPE, NORM>(p, gh, stream) : launch_form<bf16_tag, 64, AUX, SPLIT, ROPE, NORM>(p, gh, stream);
+  return head_dim == 128 ? launch_form<f16_tag, 128, AUX, SPLIT, ROPE, NORM>(p, gh, stream) : launch_form<f16_tag, 64, AUX, SPLIT, ROPE, NORM>(p, gh, stream);
+}
+
 }  // namespace
+
+// Whether the partitions merge inside their workgroup.  Only while every group is resident at once (an idle wave of a group, its partition
+// past the sequence's end, holds its LDS until the group ends), and where the spread over the CUs that a group gives up is not worth the merge
+// launch: with half the CUs holding a group anyway, or contexts short enough for one CU (256 tokens of 128 dims, as bytes).  Two launches | one,
+// us, 28 / 4 heads of 128 with the KV cold: 64 x 2048 in 2 parts 51.4 | 49.8, 48 x up to 500 in 3 15.5 | 13.2, 120 x up to 700 in 2
+// 30.4 | 28.5, 1 x 150 in 3 7.3 | 6.8; past the line 1 x 1500 in 4 17.5 | 21.7, 8 x 1000 in 4 14.9 | 18.1, 23 x up to 2000 in 5
+// 20.7 | 30.6; 16 / 2 heads of 64: 30 x up to 300 in 5 8.7 | 8.5, 128 x 1000 in 4 18.3 | 16.9.
+bool decode_mfma_groups(int64_t groups, int num_parts, int head_dim, int max_seq_len) {
+  const int ring = head_dim == 128 ? ring_bytes<128> : ring_bytes<64>, most = head_dim == 128 ? group_parts_max<128> : group_parts_max<64>;
+  return num_parts > 1 && num_parts <= most && groups <= (int64_t)kCUs * (kLdsBytes / (num_parts * ring)) &&
+         (2 * groups >= kCUs || (int64_t)max_seq_len * head_dim <= 256 * 128);
+}
 
 // Launch the MFMA decode kernel.  Caller guarantees: head_dim in {64, 128}, block_size >= 16,
 // partition a multiple of 32 tokens (any number of blocks: the block-id window is reloaded every 64 blocks).
 int launch_decode_mfma(const DecodeParams& p, int gh, int head_dim, int dtype, bool nt, bool split_p,
                        hipStream_t stream) {
-  const int64_t waves = (int64_t)p.num_seqs * (p.num_q_heads / gh) * p.num_parts;
-  if (waves > INT32_MAX) return MI_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)waves), block(64);
   if (p.slopes || p.sinks) {
     if (dtype != MI_DTYPE_BF16 || !split_p) return MI_ERR_UNSUPPORTED;
-    if (head_dim == 128) hipLaunchKernelGGL((decode_mfma_kernel<bf16_tag, 128, 2, true, 2, false, false, true>), grid, block, 0, stream, p, gh);
-    else hipLaunchKernelGGL((decode_mfma_kernel<bf16_tag, 64, 2, true, MI_DECODE_NS64, false, false, true>), grid, block, 0, stream, p, gh);
-    return launch_status();
+    return head_dim == 128 ? launch_form<bf16_tag, 128, 2, true, false, false, true>(p, gh, stream)
+                           : launch_form<bf16_tag, 64, 2, true, false, false, true>(p, gh, stream);
   }
-#define MI_LAUNCH_NS(TAG, HDIM, NS_)                                                                        \
-  do {                                                                                                      \
-    if (split_p) {                                                                                          \
-      if (nt) hipLaunchKernelGGL((decode_mfma_kernel<TAG, HDIM, 2, true, NS_>), grid, block, 0, stream, p, gh);  \
-      else hipLaunchKernelGGL((decode_mfma_kernel<TAG, HDIM, 0, true, NS_>), grid, block, 0, stream, p, gh);     \
-    } else {                                                                                                \
-      if (nt) hipLaunchKernelGGL((decode_mfma_kernel<TAG, HDIM, 2, false, NS_>), grid, block, 0, stream, p, gh); \
-      else hipLaunchKernelGGL((decode_mfma_kernel<TAG, HDIM, 0, false, NS_>), grid, block, 0, stream, p, gh);    \
-    }                                                                                                       \
-  } while (0)
-#define MI_LAUNCH(TAG, HDIM) MI_LAUNCH_NS(TAG, HDIM, 2)
-  if (dtype == MI_DTYPE_BF16) {
-    if (head_dim == 128) MI_LAUNCH(bf16_tag, 128); else MI_LAUNCH_NS(bf16_tag, 64, MI_DECODE_NS64);
-  } else {
-    if (head_dim == 128) MI_LAUNCH(f16_tag, 128); else MI_LAUNCH_NS(f16_tag, 64, MI_DECODE_NS64);
-  }
-#undef MI_LAUNCH
-#undef MI_LAUNCH_NS
-  return launch_status();
+  if (split_p) return nt ? launch_types<2, true>(p, gh, head_dim, dtype, stream) : launch_types<0, true>(p, gh, head_dim, dtype, stream);
+  return nt ? launch_types<2, false>(p, gh, head_dim, dtype, stream) : launch_types<0, false>(p, gh, head_dim, dtype, stream);
 }
 
 int launch_decode_mfma_rope(const DecodeParams& p, int gh, int head_dim, int dtype, hipStream_t stream) {
-  const int64_t waves = (int64_t)p.num_seqs * (p.num_q_heads / gh) * p.num_parts;
-  if (waves > INT32_MAX) return MI_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)waves), block(64);
-  if (p.q_norm_w) {   // per-head q / k RMSNorm in front of the rotation (Qwen3 family)
-    if (dtype == MI_DTYPE_BF16) {
-      if (head_dim == 128) hipLaunchKernelGGL((decode_mfma_kernel<bf16_tag, 128, 2, true, 2, true, true>), grid, block, 0, stream, p, gh);
-      else hipLaunchKernelGGL((decode_mfma_kernel<bf16_tag, 64, 2, true, MI_DECODE_NS64, true, true>), grid, block, 0, stream, p, gh);
-    } else {
-      if (head_dim == 128) hipLaunchKernelGGL((decode_mfma_kernel<f16_tag, 128, 2, true, 2, true, true>), grid, block, 0, stream, p, gh);
-      else hipLaunchKernelGGL((decode_mfma_kernel<f16_tag, 64, 2, true, MI_DECODE_NS64, true, true>), grid, block, 0, stream, p, gh);
-    }
-    return launch_status();
-  }
-  if (dtype == MI_DTYPE_BF16) {
-    if (head_dim == 128) hipLaunchKernelGGL((decode_mfma_kernel<bf16_tag, 128, 2, true, 2, true>), grid, block, 0, stream, p, gh);
-    else hipLaunchKernelGGL((decode_mfma_kernel<bf16_tag, 64, 2, true, MI_DECODE_NS64, true>), grid, block, 0, stream, p, gh);
-  } else {
-    if (head_dim == 128) hipLaunchKernelGGL((decode_mfma_kernel<f16_tag, 128, 2, true, 2, true>), grid, block, 0, stream, p, gh);
-    else hipLaunchKernelGGL((decode_mfma_kernel<f16_tag, 64, 2, true, MI_DECODE_NS64, true>), grid, block, 0, stream, p, gh);
-  }
-  return launch_status();
+  // (with per-head q / k RMSNorm in front of the rotation: Qwen3 family)
+  return p.q_norm_w ? launch_types<2, true, true, true>(p, gh, head_dim, dtype, stream) : launch_types<2, true, true>(p, gh, head_dim, dtype, stream);
 }
 
 }  // namespace mi

@@ -617,10 +617,11 @@ class GPUARModelRunner:
                                                            hidden_size=self.config.hidden_size, hs_dtype=self.dtype)
 
     def _alloc_decode_workspace(self, shapes) -> None:
-        """the largest need of any batch size, over the layers' (query heads, kv heads, head size)"""
-        nbytes = max(ops.decode_workspace_bytes(b, nq, hd, self.max_model_len,
-                                                ops.decode_auto_partition(b, nkv, self.max_model_len, self.block_size, head_dim=hd))
-                     for nq, nkv, hd in shapes for b in range(1, self.max_num_reqs + 1))
+        """the largest need of any batch size and context, over the layers' (query heads, kv heads, head size)"""
+        # below 2048 tokens a bound just under the largest may be cut finer (into eighths of a multiple of 256)
+        bounds = {self.max_model_len, *(min(c, self.max_model_len) for c in range(512, 2049, 256))}
+        nbytes = max(ops.decode_workspace_bytes(b, nq, hd, c, ops.decode_auto_partition(b, nkv, c, self.block_size, head_dim=hd))
+                     for nq, nkv, hd in shapes for c in bounds for b in range(1, self.max_num_reqs + 1))
         if torch.device(self.device).type == "cuda":
             self._decode_ws = ops.new_decode_workspace(nbytes, self.device)   # zeroed counters: fused partition merge
         else:
