@@ -264,6 +264,18 @@ int mi_rope_cache_paged_attn_decode(void* out, const void* q, const void* k, con
                                     int64_t cache_token_stride, int64_t cache_head_stride,
                                     int32_t partition_size, void* workspace, int64_t workspace_bytes,
                                     int dtype, int out_dtype, int32_t flags, void* stream);
+
+/* The same launch fed by the fp32 split-K partials [split][num_seqs][(num_q_heads + 2 num_kv_heads) * head_dim] of qkv_proj
+ * (mi_linear_partials) and its bias (may be NULL) instead of 16-bit q / k / v rows: bit-identical to mi_linear in front of it. */
+int mi_rope_cache_paged_attn_decode_splitk(void* out, const void* partials, int32_t split, const void* qkv_bias,
+                                           const int64_t* positions, const float* cos_sin_cache, int32_t max_position, int32_t rot_dim,
+                                           const void* q_norm_weight, const void* k_norm_weight, float norm_eps, void* k_cache,
+                                           void* v_cache, const int64_t* slot_mapping, const int32_t* block_table,
+                                           const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                           int32_t head_dim, int32_t block_size, int32_t block_table_stride, int32_t max_seq_len,
+                                           float scale, int64_t out_token_stride, int64_t cache_block_stride, int64_t cache_token_stride,
+                                           int64_t cache_head_stride, int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                           int dtype, int out_dtype, int32_t flags, void* stream);
 /* Partition size the auto heuristic picks: the fewest partitions that leave >= 512 waves (>= 1024 at
  * head_dim <= 64) — ONE (direct output, no workspace, no merge launch) once num_seqs * num_kv_heads
  * reaches that; 256..8192 tokens. */

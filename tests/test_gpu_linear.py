@@ -5,6 +5,8 @@ accumulates in fp32 in a different order than a library GEMM (k permuted inside 
 so results are compared to a float64-accumulated reference rounded to the output type, within 1 output ulp + 1e-3 of
 the row's magnitude.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -465,3 +467,68 @@ def test_tall_linear_takes_what_it_is_ahead_on(monkeypatch):
     assert not layers._tall_wins(256, 3584, 18944, bf) and not layers._tall_wins(8192, 3584, 18944, bf)      # selected by measurement
     assert not layers._tall_wins(768, 18944, 3584, bf, gated=True) and not layers._tall_wins(6719, 3584, 3584, bf)
     assert not layers._tall_wins(300, 3584, 18944, torch.float32) and not layers._tall_wins(120_000, 3584, 18944, bf)
+
+
+@pytest.mark.parametrize("m,n,k,bias", [
+    (33, 4608, 3584, True), (64, 3584, 4096, False), (128, 4592, 3584, True),       # 64-column tiles, few slices; a ragged last tile
+    (96, 6144, 3072, False), (65, 2304, 3584, True), (128, 8192, 512, False),       # 96 columns; many slices; two slices of 256
+])
+def test_narrow_tiles_match_float64(plan_registry, m, n, k, bias):
+    """the plans of 33 to 128 rows that are not 128 columns wide, on both sides of their row blocks and with partials"""
+    from vllm_omni_amd import _C, ops
+    buf = (ctypes.c_int32 * 3)()
+    assert _C.lib.mi_linear_plan_get(_C.MI_LINEAR_PLAN_FULL, m, n, k, buf) == _C.MI_OK and buf[0] <= 128 and buf[1] in (64, 96), list(buf)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) * k ** -0.5).bfloat16()
+    b = torch.randn(n, device="cuda", generator=g).bfloat16() if bias else None
+    ref = _ref(x, w, b)
+    tol = ref.abs() * 2.0 ** -8 + 1e-3 * ref.abs().amax(dim=1, keepdim=True).clamp_min(1.0)
+    y = ops.linear(x, w, b)
+    assert bool(((y.double() - ref).abs() <= tol).all())
+    part = ops.linear_partials(x, w, b)
+    if part is not None:
+        assert bool(((part.materialize().double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("qk_norm", [False, True])
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float16, 64)])
+@pytest.mark.parametrize("S,split,bias", [(1, 2, True), (3, 3, False), (70, 4, True), (2, 5, True), (130, 9, False)])
+def test_decode_attention_from_qkv_partials_is_bit_identical(plan_registry, S, split, bias, dtype, d, qk_norm):
+    """Slabs of qkv_proj summed inside the decode attention launch against the reduce launch in front of it: the output and both
+    caches, over one and several partitions, short ones whose wave writes the token's row before it reads, and empty sequences."""
+    from vllm_omni_amd import _C, ops
+    from vllm_omni_amd.layers import build_cos_sin_cache
+    k, bs, dev = 1024, 16, "cuda"
+    g = torch.Generator(device=dev).manual_seed(S + split)
+    for nq, nkv, ctx, ps in ((14, 2, 200, 64), (16, 1, 90, 0), (5, 5, 700, 96)):
+        n = (nq + 2 * nkv) * d
+        assert _C.lib.mi_linear_plan_set(_C.MI_LINEAR_PLAN_PARTIALS, 0, 256, n, k, 64, 64, split) == _C.MI_OK
+        x = torch.randn(S, k, device=dev, generator=g).to(dtype)
+        w = (torch.randn(n, k, device=dev, generator=g) * k ** -0.5).to(dtype)
+        b = torch.randn(n, device=dev, generator=g).to(dtype) if bias else None
+        lens = [ctx, 0, 33, 65, 64, 1, ctx - 1]
+        lens = [lens[i % len(lens)] for i in range(S)]
+        blocks = -(-ctx // bs)
+        table = (1 + torch.randperm(S * blocks, device=dev, generator=g).view(S, blocks)).int()
+        kv = torch.randn(S * blocks + 1, 2, bs, nkv, d, device=dev, generator=g).to(dtype)
+        slots = torch.tensor([int(table[i, (t - 1) // bs]) * bs + (t - 1) % bs if t else -1 for i, t in enumerate(lens)], device=dev)
+        pos = torch.tensor([max(t - 1, 0) for t in lens], device=dev)
+        seq_lens = torch.tensor(lens, dtype=torch.int32, device=dev)
+        csc = build_cos_sin_cache(d, 2048, 1e6, device=dev)
+        norm = {}
+        if qk_norm:
+            norm = {f"{c}_norm_weight": (1 + 0.1 * torch.randn(d, device=dev, generator=g)).to(dtype) for c in "qk"}
+        part = ops.linear_partials(x, w, b)
+        assert part.split == split
+        row = part.materialize()
+        q, kn, vn = row.split([nq * d, nkv * d, nkv * d], dim=-1)
+        one, two = kv.clone(), kv.clone()
+        want = torch.full((S, nq * d), float("nan"), dtype=dtype, device=dev)
+        ops.rope_cache_paged_attn_decode(want, q, kn, vn, pos, csc, one[:, 0], one[:, 1], slots, table, seq_lens, ctx, d ** -0.5,
+                                         partition_size=ps, **norm)
+        got = ops.rope_cache_paged_attn_decode_splitk(part, nq, nkv, d, pos, csc, two[:, 0], two[:, 1], slots, table, seq_lens, ctx, d ** -0.5,
+                                                      partition_size=ps, **norm)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(one, two) and not torch.equal(one, kv), (nq, nkv)
+        _C.lib.mi_linear_plan_clear()

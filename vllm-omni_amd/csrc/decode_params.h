@@ -43,6 +43,11 @@ struct DecodeParams {
   const float* slopes = nullptr;
   const float* sinks = nullptr;
   float out_scale = 1.f;   // the output times this (matrix-core kernel and the merge)
+  // the rope form fed by the fp32 slabs [num_slabs][num_seqs][slab_row] of a split-K qkv_proj instead of q / k_new / v_new
+  const float* slabs = nullptr;
+  const void* qkv_bias = nullptr;   // [slab_row] of the dtype, or null
+  int32_t num_slabs = 0;
+  int64_t slab_stride = 0, slab_row = 0;
   bool group_parts = false;   // matrix-core kernel: the partitions are the waves of a workgroup and merge there
 };
 

@@ -550,6 +550,9 @@ struct RopeFusion {
   const void* q_norm_w;
   const void* k_norm_w;
   float norm_eps;
+  const float* slabs;      // split-K partials of qkv_proj in the place of q, k and v
+  int32_t num_slabs;
+  const void* qkv_bias;
 };
 
 int decode_call(void* out, const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
@@ -646,6 +649,9 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
     p.cos_sin = rope->cos_sin; p.max_position = rope->max_position;
     p.kn_stride = rope->k_stride; p.vn_stride = rope->v_stride;
     p.q_norm_w = rope->q_norm_w; p.k_norm_w = rope->k_norm_w; p.norm_eps = rope->norm_eps;
+    p.slabs = rope->slabs; p.num_slabs = rope->num_slabs; p.qkv_bias = rope->qkv_bias;
+    p.slab_row = (int64_t)(num_q_heads + 2 * num_kv_heads) * head_dim;
+    p.slab_stride = num_seqs * p.slab_row;
     rc = launch_decode_mfma_rope(p, G, head_dim, dtype, s);
   } else if (use_mfma) {
     rc = launch_decode_mfma(p, G, head_dim, dtype, (flags & MI_DECODE_NONTEMPORAL) != 0,
@@ -719,9 +725,35 @@ extern "C" int mi_rope_cache_paged_attn_decode(void* out, const void* q, const v
   if (k_token_stride % 8 || v_token_stride % 8 || (((uintptr_t)k | (uintptr_t)v | (uintptr_t)cos_sin_cache) & 15))
     return MI_ERR_INVALID_ARG;
   const RopeFusion rf{k, v, positions, slot_mapping, cos_sin_cache, max_position, k_token_stride, v_token_stride,
-                      q_norm_weight, k_norm_weight, norm_eps};
+                      q_norm_weight, k_norm_weight, norm_eps, nullptr, 0, nullptr};
   return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
                      block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
                      cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
                      workspace_bytes, dtype, out_dtype, flags, stream, &rf);
+}
+
+extern "C" int mi_rope_cache_paged_attn_decode_splitk(void* out, const void* partials, int32_t split, const void* qkv_bias,
+                                                      const int64_t* positions, const float* cos_sin_cache,
+                                                      int32_t max_position, int32_t rot_dim, const void* q_norm_weight,
+                                                      const void* k_norm_weight, float norm_eps, void* k_cache, void* v_cache,
+                                                      const int64_t* slot_mapping, const int32_t* block_table,
+                                                      const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads,
+                                                      int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                                      int32_t block_table_stride, int32_t max_seq_len, float scale,
+                                                      int64_t out_token_stride, int64_t cache_block_stride,
+                                                      int64_t cache_token_stride, int64_t cache_head_stride,
+                                                      int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                                      int dtype, int out_dtype, int32_t flags, void* stream) {
+  if (num_seqs == 0) return MI_OK;
+  if (!partials || !positions || !cos_sin_cache || !slot_mapping || max_position <= 0 || split < 1) return MI_ERR_INVALID_ARG;
+  if (rot_dim != head_dim) return MI_ERR_UNSUPPORTED;
+  if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return MI_ERR_INVALID_ARG;
+  if (((uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight | (uintptr_t)partials | (uintptr_t)qkv_bias | (uintptr_t)cos_sin_cache) & 15)
+    return MI_ERR_INVALID_ARG;
+  const RopeFusion rf{nullptr, nullptr, positions, slot_mapping, cos_sin_cache, max_position, 0, 0, q_norm_weight, k_norm_weight,
+                      norm_eps, static_cast<const float*>(partials), split, qkv_bias};
+  return decode_call(out, partials, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                     block_size, block_table_stride, max_seq_len, scale, 0, out_token_stride, cache_block_stride,
+                     cache_token_stride, cache_head_stride, partition_size, workspace, workspace_bytes, dtype, out_dtype, flags,
+                     stream, &rf);
 }

@@ -138,6 +138,8 @@ template <int HD>
 constexpr int ring_bytes = (HD == 128 ? 2 : MI_DECODE_NS64) * 2 * kStep * HD * 2;
 template <int HD>
 constexpr int group_parts_max = kLdsBytes / ring_bytes<HD> < 8 ? kLdsBytes / ring_bytes<HD> : 8;   // head_dim 128: five; 64: eight
+// PART (with ROPE): the qkv row is the sum of the fp32 slabs of a split-K qkv_proj (skinny_gemm.hip) and its bias, in skinny_reduce_kernel's
+// order and rounding: each wave sums the columns of its own query heads, the wave that owns the token's row those of its k and v.
 // The rings' LDS: static for a lone wave, whose DMA destinations are then constants.  The addresses of both start at 0.
 using lds_float = __attribute__((address_space(3))) float;
 using lds_char = __attribute__((address_space(3))) char;   // a generic pointer costs a null check at each DMA's cast
@@ -151,7 +153,8 @@ __device__ __forceinline__ lds_char* ring_base() {
     return (lds_char*)ring;
   }
 }
-template <typename Tag, int HD, int AUX, bool SPLIT, int NS, bool ROPE = false, bool NORM = false, bool BIAS = false, bool GROUP = false>
+template <typename Tag, int HD, int AUX, bool SPLIT, int NS, bool ROPE = false, bool NORM = false, bool BIAS = false, bool GROUP = false,
+          bool PART = false>
 __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void decode_mfma_kernel(const DecodeParams p, const int gh) {
   scalar_cache_acquire();
   using E = Elem<Tag>;
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
 
   // ---- Q^T fragments (B operand): lane (head h, dims 32s + 8g ..) ------------------------
   uint4 qf[KS];
-  {
+  if constexpr (!PART) {
     const uint16_t* qb = reinterpret_cast<const uint16_t*>(p.q) + (int64_t)seq * p.q_stride +
                          (int64_t)(qh0 + (head_ok ? h : 0)) * HD + 8 * g;
 #pragma unroll
@@ -276,15 +279,32 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
     rope_row = p.cos_sin + pos * HD;   // rot_dim == head_dim
     kv_owner = t_end == steps_total && qh0 % p.kv_group == 0;   // wave-uniform
   }
+  // PART: the 16-bit rows [gh query heads | k | v], in the last stage's V image until its DMA is issued
+  lds_char* const qkv_lds = smem + (NS - 1) * STAGE + IMG;
+  using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
+  const auto lds_row16 = [&](int off) -> uint4 {
+    const u32x4 v = *(const __attribute__((address_space(3))) u32x4*)(qkv_lds + off);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+  };
+  static_assert(18 * ROWB <= IMG, "sixteen query heads, k and v");
+  int64_t new_slot = 0;
+  if constexpr (PART) new_slot = p.slot_mapping[seq];   // beside the slabs' loads, not behind them
   auto kv_write = [&]() {
-    const int64_t slot = p.slot_mapping[seq];
+    const int64_t slot = PART ? new_slot : p.slot_mapping[seq];
     if (slot < 0) return;
     const int64_t crow = (slot >> p.bs_log2) * p.blk_stride + (slot & bs_mask_of(p.bs_log2)) * p.tok_stride +
                          (int64_t)kvh * p.head_stride;
     constexpr int RI = HD / 16;   // rotate-items of one k head: lane j < RI = dims [8 j, 8 j + 8) and their partners
     if (lane < RI) {
-      const uint16_t* kn = reinterpret_cast<const uint16_t*>(p.k_new) + (int64_t)seq * p.kn_stride + kvh * HD;
-      uint4 x = *reinterpret_cast<const uint4*>(kn + 8 * lane), y = *reinterpret_cast<const uint4*>(kn + HD / 2 + 8 * lane);
+      uint4 x, y;
+      if constexpr (PART) {
+        x = lds_row16(gh * ROWB + 16 * lane);
+        y = lds_row16(gh * ROWB + ROWB / 2 + 16 * lane);
+      } else {
+        const uint16_t* kn = reinterpret_cast<const uint16_t*>(p.k_new) + (int64_t)seq * p.kn_stride + kvh * HD;
+        x = *reinterpret_cast<const uint4*>(kn + 8 * lane);
+        y = *reinterpret_cast<const uint4*>(kn + HD / 2 + 8 * lane);
+      }
       if constexpr (NORM) {   // the RI lanes of the head: rope_cache_kernel's reduction, lane for lane
         float ss = item_sumsq<Tag>(x, y);
         ss += dpp_f32<kDppQuadXor1>(ss);
@@ -299,13 +319,79 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
       *reinterpret_cast<uint4*>(kc + HD / 2 + 8 * lane) = y;
     } else if (lane < RI + HD / 8) {
       const int j = lane - RI;
-      const uint16_t* vn = reinterpret_cast<const uint16_t*>(p.v_new) + (int64_t)seq * p.vn_stride + kvh * HD;
       uint16_t* vc = reinterpret_cast<uint16_t*>(const_cast<void*>(p.v_cache)) + crow;
-      *reinterpret_cast<uint4*>(vc + 8 * j) = *reinterpret_cast<const uint4*>(vn + 8 * j);
+      if constexpr (PART) {
+        *reinterpret_cast<uint4*>(vc + 8 * j) = lds_row16((gh + 1) * ROWB + 16 * j);
+      } else {
+        const uint16_t* vn = reinterpret_cast<const uint16_t*>(p.v_new) + (int64_t)seq * p.vn_stride + kvh * HD;
+        *reinterpret_cast<uint4*>(vc + 8 * j) = *reinterpret_cast<const uint4*>(vn + 8 * j);
+      }
     }
   };
   const bool kv_early = kv_owner && t_end - t_begin <= NS;
-  if constexpr (ROPE) {
+  // PART: 4 columns a lane and step, the loads of 5 steps and 4 slabs in flight together (28 / 4 heads: all of q in 4 steps, k and v in
+  // one more).  A loop of few instructions: every wave runs it once, and at a small batch its instruction fetches would be what is waited for.
+  const auto sum_slabs = [&]() {
+    constexpr int IT = 5, SL = 4;
+    using lds_u32x2 = __attribute__((address_space(3))) u32x2_t;
+    const int nkv = p.num_q_heads / p.kv_group;
+    const int nq4 = gh * (HD / 4), n4 = nq4 + (kv_owner ? HD / 2 : 0);
+    const float* const row = p.slabs + (int64_t)seq * p.slab_row;
+#pragma unroll 1
+    for (int base = 0; base < n4; base += 64 * IT) {
+      int col[IT];
+      float4 a[IT];
+      uint2 b[IT];
+#pragma unroll
+      for (int t = 0; t < IT; ++t) {
+        const int i = min(base + 64 * t + lane, n4 - 1), r = i - nq4;
+        col[t] = r < 0 ? qh0 * HD + 4 * i : (p.num_q_heads + (r < HD / 4 ? 0 : nkv - 1) + kvh) * HD + 4 * r;
+        a[t] = make_float4(-0.f, -0.f, -0.f, -0.f);      // x + -0 is x, for 0 and -0 too
+        b[t] = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(p.qkv_bias ? p.qkv_bias : p.slabs) + col[t]);
+      }
+#pragma unroll 1
+      for (int s0 = 0; s0 < p.num_slabs; s0 += SL) {
+        float4 v[SL][IT];
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {      // past the last slab: that slab again, dropped
+          const float* const slab = row + (int64_t)min(s0 + i, p.num_slabs - 1) * p.slab_stride;
+#pragma unroll
+          for (int t = 0; t < IT; ++t) v[i][t] = *reinterpret_cast<const float4*>(slab + col[t]);
+        }
+#pragma unroll
+        for (int i = 0; i < SL; ++i)
+          if (s0 + i < p.num_slabs) {
+#pragma unroll
+            for (int t = 0; t < IT; ++t) {
+              a[t].x += v[i][t].x;
+              a[t].y += v[i][t].y;
+              a[t].z += v[i][t].z;
+              a[t].w += v[i][t].w;
+            }
+          }
+      }
+#pragma unroll
+      for (int t = 0; t < IT; ++t) {
+        if (p.qkv_bias) {
+          a[t].x += E::lo(b[t].x);
+          a[t].y += E::hi(b[t].x);
+          a[t].z += E::lo(b[t].y);
+          a[t].w += E::hi(b[t].y);
+        }
+        if (base + 64 * t + lane < n4)
+          *(lds_u32x2*)(qkv_lds + 8 * (base + 64 * t + lane)) = u32x2_t{E::pack(a[t].x, a[t].y), E::pack(a[t].z, a[t].w)};
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      qf[s] = head_ok ? lds_row16(h * ROWB + 64 * s + 16 * g) : make_uint4(0, 0, 0, 0);
+    if (kv_owner) {
+      kv_write();
+      wait_vmcnt<0>();
+    }
+    lds_wait_all();   // the rows are in registers: their place may be filled
+  };
+  if constexpr (ROPE && !PART) {
     if (kv_early) {
       kv_write();
       wait_vmcnt<0>();   // acknowledged before the prologue DMA below can fetch the row
@@ -540,12 +626,25 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
     win_b = bt_row[min(first_blk + 64 + lane, p.block_table_stride - 1)];
     asm volatile("" : "+v"(win_b));
   }
+  const auto fill = [&]() {
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    if (t_begin + i < t_end) {
-      issue_k(t_begin + i, i);
-      issue_v(t_begin + i, i);
+    for (int i = 0; i < NS; ++i) {
+      if (t_begin + i < t_end) {
+        issue_k(t_begin + i, i);
+        if (!PART || i < NS - 1) issue_v(t_begin + i, i);
+      }
     }
+  };
+  if constexpr (PART) {
+    // the sums ride under the DMA, or stand in front of it where it fetches the token's row.  One copy of either's code
+#pragma unroll 1
+    for (int turn = 0; turn < 2; ++turn) {
+      if ((turn == 0) == kv_early) sum_slabs();
+      else fill();
+    }
+    if (t_begin + NS - 1 < t_end) issue_v(t_begin + NS - 1, NS - 1);
+  } else {
+    fill();
   }
   if constexpr (ROPE) {
     // q: dims 32 s + 8 g .. of head h pair with dims + HD / 2 = fragment s + KS / 2 of the same lane
@@ -570,7 +669,7 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
     }
 #pragma unroll
     for (int s = 0; s < KS / 2; ++s) rope_rotate8<Tag>(qf[s], qf[s + KS / 2], rope_row, 32 * s + 8 * g, HD / 2);
-    if (kv_owner && !kv_early) {
+    if (!PART && kv_owner && !kv_early) {
       kv_write();
       // Acknowledged before the loop can issue the DMA of the row's step (it may do so in its very first step: a
       // counted wait only bounds the operations outstanding, it does not order three young stores).  The prologue's
@@ -704,29 +803,31 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
 }
 
 // one wave a workgroup, or (group) the partitions of a sequence's head group as the waves of one
-template <typename Tag, int HD, int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool BIAS = false>
+template <typename Tag, int HD, int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool BIAS = false, bool PART = false>
 int launch_form(const DecodeParams& p, int gh, hipStream_t stream) {
   constexpr int NS = HD == 128 ? 2 : MI_DECODE_NS64, ring = ring_bytes<HD>;
   static_assert(ring >= (16 * HD + 32) * 4, "a wave's partial takes its ring's place");
   const int64_t groups = (int64_t)p.num_seqs * (p.num_q_heads / gh);
   if (groups * p.num_parts > INT32_MAX) return MI_ERR_UNSUPPORTED;
   if (p.group_parts) {
-    auto kern = decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, true>;
+    auto kern = decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, true, PART>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        group_parts_max<HD> * ring);
     if (attr != hipSuccess) return MI_ERR_LAUNCH;
     hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(64 * p.num_parts), p.num_parts * ring, stream, p, gh);
   } else {
-    hipLaunchKernelGGL((decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS>), dim3((unsigned)(groups * p.num_parts)), dim3(64), 0,
+    hipLaunchKernelGGL((decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, false, PART>), dim3((unsigned)(groups * p.num_parts)), dim3(64), 0,
                        stream, p, gh);
   }
   return launch_status();
 }
-template <int AUX, bool SPLIT, bool ROPE = false, bool NORM = false>
+template <int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool PART = false>
 int launch_types(const DecodeParams& p, int gh, int head_dim, int dtype, hipStream_t stream) {
   if (dtype == MI_DTYPE_BF16)
-    return head_dim == 128 ? launch_form<bf16_tag, 128, AUX, SPLIT, ROPE, NORM>(p, gh, stream) : launch_form<bf16_tag, 64, AUX, SPLIT, ROPE, NORM>(p, gh, stream);
-  return head_dim == 128 ? launch_form<f16_tag, 128, AUX, SPLIT, ROPE, NORM>(p, gh, stream) : launch_form<f16_tag, 64, AUX, SPLIT, ROPE, NORM>(p, gh, stream);
+    return head_dim == 128 ? launch_form<bf16_tag, 128, AUX, SPLIT, ROPE, NORM, false, PART>(p, gh, stream)
+                           : launch_form<bf16_tag, 64, AUX, SPLIT, ROPE, NORM, false, PART>(p, gh, stream);
+  return head_dim == 128 ? launch_form<f16_tag, 128, AUX, SPLIT, ROPE, NORM, false, PART>(p, gh, stream)
+                         : launch_form<f16_tag, 64, AUX, SPLIT, ROPE, NORM, false, PART>(p, gh, stream);
 }
 
 }  // namespace
@@ -758,6 +859,9 @@ int launch_decode_mfma(const DecodeParams& p, int gh, int head_dim, int dtype, b
 
 int launch_decode_mfma_rope(const DecodeParams& p, int gh, int head_dim, int dtype, hipStream_t stream) {
   // (with per-head q / k RMSNorm in front of the rotation: Qwen3 family)
+  if (p.slabs)
+    return p.q_norm_w ? launch_types<2, true, true, true, true>(p, gh, head_dim, dtype, stream)
+                      : launch_types<2, true, true, false, true>(p, gh, head_dim, dtype, stream);
   return p.q_norm_w ? launch_types<2, true, true, true>(p, gh, head_dim, dtype, stream) : launch_types<2, true, true>(p, gh, head_dim, dtype, stream);
 }
 

@@ -625,6 +625,22 @@ int forced_split() {   // MI_LINEAR_SPLIT=<S>: tuning override of the split-K fa
 }  // namespace
 
 namespace {
+// Narrow tiles.  At 33 to 128 rows a workgroup waits for its share of K and not for the rows that narrow tiles read again, and few slices of
+// 64-column tiles leave fewer slabs to sum than many of 128 columns.  Where 64 columns fill 84 % of the CUs (96 columns: 95 %) with at most
+// 1536 of K each (cold weights, 128-column tiles | this, us: 4608 x 3584, 64 rows 15.7 | 14.7, 128 rows 20.7 | 19.0; 4096 x 4096 15.9 | 14.3
+// and 21.2 | 17.8; 2048 x 8192 16.1 | 14.1 and 22.2 | 18.6; 6144 x 3072, 96 columns, 16.5 | 15.6 and 22.1 | 21.6); a longer share wants the
+// wide tile (3584 x 18944, 64 rows 30.5 | 33.2), and so does a fuller round (10368 x 4096, 96 columns on 84 %, 22.8 | 24.9).  Up to 32 rows
+// the two are level, launch and reduce (4608 x 3584, 24 rows 12.3 | 12.0) or in the consumer (9.4 | 9.7).
+bool narrow_plan(int m, int n, int k, mi::SkinnyPlan* pl) {
+  if (m <= 32 || m > 128) return false;
+  for (int ns = 2; ns <= 3; ++ns) {
+    const int t = (n + 32 * ns - 1) / (32 * ns), split = std::min(16, 256 / t);
+    if (split < 2 || t * split < (ns == 2 ? 215 : 243) || k > 1536 * split || k < 256 * split) continue;
+    mi::plan_fill(pl, m <= 64 ? 4 : 8, ns, split, n, false);
+    return true;
+  }
+  return false;
+}
 // 16-bit plan for up to 512 rows: 257-512 rows run as two row blocks per weight tile (grid.y), with the split halved so
 // the grid still fits one round — the same arrangement as the W8A8 entry points below
 mi::SkinnyPlan linear_plan(int m, int n, int k, int purpose = MI_LINEAR_PLAN_FULL) {
@@ -632,6 +648,7 @@ mi::SkinnyPlan linear_plan(int m, int n, int k, int purpose = MI_LINEAR_PLAN_FUL
   if (mi::plan_override("MI_LINEAR_PLAN", n, false, k, &reg)) return reg;
   if (purpose == MI_LINEAR_PLAN_PARTIALS && mi::plan_lookup(MI_LINEAR_PLAN_PARTIALS, m, n, k, &reg)) return reg;
   if (mi::plan_lookup(MI_LINEAR_PLAN_FULL, m, n, k, &reg)) return reg;
+  if (forced_split() <= 0 && narrow_plan(m, n, k, &reg)) return reg;
   mi::SkinnyPlan pl = mi::skinny_plan(m > 256 ? 256 : m, n, k, forced_split());
   if (m > 256 && forced_split() <= 0) pl.split = pl.split > 1 ? (pl.split + 1) / 2 : 1;
   return pl;

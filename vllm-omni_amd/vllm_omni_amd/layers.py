@@ -257,7 +257,7 @@ class Attention:
     def rope_decode_fusable(self, rope: RotaryEmbedding, positions: torch.Tensor, q_norm_weight=None) -> bool:
         """Whether this step's RoPE + KV write run inside the paged-attention launch (``ops.rope_cache_paged_attn_decode``):
         a pure-decode step on the production decode kernel, plain positions (q/k-norm rides along), not a single-block sequence
-        (those have their own fused launch).  qkv_proj then hands over a 16-bit row, not split-K partials."""
+        (those have their own fused launch).  qkv_proj then hands over a 16-bit row or, at some batch sizes, split-K partials."""
         md = get_forward_context().attn_metadata
         if md is None or md.single_block or positions.dim() != 1:
             return False
@@ -303,7 +303,7 @@ class Attention:
     def forward_fused_rope_partials(self, rope: RotaryEmbedding, positions: torch.Tensor, qkv: "ops.SplitKPartials",
                                     q_norm_weight=None, k_norm_weight=None, norm_eps: float = 1e-6) -> torch.Tensor:
         """``forward_fused_rope`` when qkv_proj handed over split-K partials: their reduction (+ bias) happens inside
-        the RoPE + KV-write launch; same result bit for bit."""
+        the RoPE + KV-write launch, or the decode attention launch that this is part of; same result bit for bit."""
         md = get_forward_context().attn_metadata
         if (md.single_block and rope._section(positions) is None and _BLOCK_ATTENTION
                 and ops.block_attention_supported(self.num_heads, self.num_kv_heads, self.head_size, self._kb.shape[1],
@@ -313,6 +313,11 @@ class Attention:
                                                       rope.cos_sin_cache, self._kb, self._vb, md.block_table[:, 0], self.scale,
                                                       q_norm_weight=q_norm_weight, k_norm_weight=k_norm_weight,
                                                       norm_eps=norm_eps, max_position_bound=md.max_seq_len - 1)
+        if self.rope_decode_fusable(rope, positions, q_norm_weight):
+            return ops.rope_cache_paged_attn_decode_splitk(
+                qkv, self.num_heads, self.num_kv_heads, self.head_size, positions, rope.cos_sin_cache, self._kb, self._vb,
+                md.slot_mapping, md.block_table, md.seq_lens, md.max_seq_len, self.scale, partition_size=md.decode_partition_size,
+                workspace=md.decode_workspace, q_norm_weight=q_norm_weight, k_norm_weight=k_norm_weight, norm_eps=norm_eps)
         q = ops.rope_neox_and_cache_splitk(qkv, self.num_heads, self.num_kv_heads, self.head_size, positions,
                                            rope.cos_sin_cache, self._kb, self._vb, md.slot_mapping,
                                            mrope_section=rope._section(positions), q_norm_weight=q_norm_weight,
@@ -457,6 +462,21 @@ def _deferred_qkv_wins(m: int, n: int, k: int) -> bool:
     return m <= 256 and n * k >= (1 << 23) and _DEFER_QKV
 
 
+def _narrow_kernel_wins(m: int, n: int, k: int) -> bool:
+    # 33 to 128 rows of a K that splits into few slices (narrow_plan in skinny_gemm.hip).  Library | kernel, us, cold weights: 4608 x 3584,
+    # 64 rows 19.0 | 14.7, 128 rows 22.9 | 19.0; 5120 x 4096 17.6 | 15.6 and 25.2 | 19.8; 4096 x 4096 15.2 | 14.3 and 24.4 | 17.8; 10368 x 4096
+    # 26.8 | 22.8 and 31.0 | 27.5.  K 3072 is level (6144 x 3072, 128 rows 21.1 | 21.6), K 2048 behind (8192 x 2048, 64 rows 13.6 | 15.0), and at
+    # 256 rows whole decode steps are behind, 1.5 to 3 %
+    return 32 < m <= 128 and 3584 <= n <= 12288 and 3584 <= k <= 4096
+
+
+def _attn_qkv_wins(m: int, n: int, k: int) -> bool:
+    # qkv_proj (4608 x 3584) with its split-K reduce (+ bias) inside the decode attention launch.  Both launches, us, library | kernel
+    # and its reduce | this: 64 x 2048 tokens 68.6 | 64.1 | 61.9, 120 x up to 700 47.7 | 47.2 | 46.1, 128 x 2048 113 | 111 | 107; up to 32
+    # rows the wait for the slabs costs what the reduce launch does (1 x 150 21.2 | 17.8 | 18.8, 23 x up to 1700 31.1 | 30.4 | 30.9)
+    return _narrow_kernel_wins(m, n, k)
+
+
 def _fused_gate_up_wins(m: int, inter: int, k: int) -> bool:
     # same measurements: ahead at I 18944 and 9472 per rank (>= ~120 tiles in one launch), not at 4736
     if m <= 256 and inter >= 8192:
@@ -496,18 +516,22 @@ def _apply_linear(layer, x: torch.Tensor, bias: Optional[torch.Tensor], defer_re
             defer_us = _DEFERRED_REDUCE_US
             if part and e.get("tp") == 0 and _DEFER_TRAFFIC:
                 defer_us += int(part["split"]) * m * n * 4 / 3.0e6
-            if defer_reduce and _DEFER_REDUCE and part and part["us"] + defer_us < best_direct and (
+            if defer_reduce and defer_reduce != "attn" and _DEFER_REDUCE and part and part["us"] + defer_us < best_direct and (
                     defer_reduce != "rope" or _DEFER_QKV_TUNED):
                 pr = ops.linear_partials(x, w, bias)
                 if pr is not None:
                     return pr
             return ops.linear(x, w, bias) if e["full"]["us"] < e["library_us"] else F.linear(x, w, bias)
         if ops.linear_supported(m, n, k, x.dtype):
-            wins = (_LINEAR_MODE == "kernel" or _streaming_kernel_wins(m, n, k)
+            wins = (_LINEAR_MODE == "kernel" or _streaming_kernel_wins(m, n, k) or _narrow_kernel_wins(m, n, k)
                     or (_LINEAR_MODE in ("mlp", "mlp+o") and getattr(layer, "_is_down_proj", False))
                     or (_LINEAR_MODE == "mlp+o" and getattr(layer, "_is_o_proj", False)))
-            if defer_reduce and _DEFER_REDUCE and (
-                    wins or (_deferred_qkv_wins(m, n, k) if defer_reduce == "rope" else _deferred_kernel_wins(m, n, k))):
+            if defer_reduce == "attn":
+                defer = _attn_qkv_wins(m, n, k)
+            else:
+                defer = defer_reduce and (
+                    wins or (_deferred_qkv_wins(m, n, k) if defer_reduce == "rope" else _deferred_kernel_wins(m, n, k)))
+            if defer and _DEFER_REDUCE:
                 part = ops.linear_partials(x, w, bias)
                 if part is not None:
                     return part
@@ -561,7 +585,8 @@ class ColumnParallelLinear:
 
     def __call__(self, x: torch.Tensor, defer_reduce=False):
         """``defer_reduce="rope"`` (qkv_proj): the caller runs the fused RoPE + KV-write kernel next, which can take the
-        split-K partials of the streaming kernel directly (``ops.rope_neox_and_cache_splitk``)."""
+        split-K partials of the streaming kernel directly (``ops.rope_neox_and_cache_splitk``); ``"attn"``: the decode
+        attention launch that RoPE and the KV write are part of (``ops.rope_cache_paged_attn_decode_splitk``)."""
         y = _apply_linear(self, x, self.bias, defer_reduce if not self.gather_output else False)
         if self.gather_output:
             y = tensor_model_parallel_all_gather(y)

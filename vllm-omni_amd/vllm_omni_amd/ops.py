@@ -471,6 +471,47 @@ def rope_cache_paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k: torch.Te
     return out
 
 
+def rope_cache_paged_attn_decode_splitk(part: "SplitKPartials", num_q_heads: int, num_kv_heads: int, head_dim: int,
+                                        positions: torch.Tensor, cos_sin_cache: torch.Tensor, k_cache: torch.Tensor,
+                                        v_cache: torch.Tensor, slot_mapping: torch.Tensor, block_table: torch.Tensor,
+                                        seq_lens: torch.Tensor, max_seq_len: int, scale: float, partition_size: int = 0,
+                                        workspace: Optional[torch.Tensor] = None, q_norm_weight: Optional[torch.Tensor] = None,
+                                        k_norm_weight: Optional[torch.Tensor] = None, norm_eps: float = 1e-6) -> torch.Tensor:
+    """``rope_cache_paged_attn_decode`` fed by the split-K partials of ``qkv_proj`` (``linear_partials``): returns the
+    attention output [S, nq*d].  Bit-identical to ``linear`` + ``rope_cache_paged_attn_decode``."""
+    _gpu(positions, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, seq_lens, workspace, q_norm_weight, k_norm_weight)
+    part._live()
+    if part.n != (num_q_heads + 2 * num_kv_heads) * head_dim:
+        raise ValueError("partials row is not [q heads | k heads | v heads]")
+    if (q_norm_weight is None) != (k_norm_weight is None):
+        raise ValueError("q_norm_weight and k_norm_weight come together")
+    nb, bs, hkv, d = k_cache.shape
+    if (hkv, d) != (num_kv_heads, head_dim):
+        raise ValueError("the cache's heads are not the partials' ones")
+    if block_table.dtype != torch.int32 or seq_lens.dtype != torch.int32:
+        raise TypeError("block_table and seq_lens must be int32")
+    if positions.dtype != torch.int64 or slot_mapping.dtype != torch.int64 or cos_sin_cache.dtype != torch.float32:
+        raise TypeError("positions / slot_mapping must be int64 and cos_sin_cache float32")
+    if positions.dim() != 1 or block_table.stride(1) != 1:
+        raise ValueError("1-D positions and contiguous block_table rows required")
+    s = part.m
+    out = torch.empty(s, num_q_heads * head_dim, dtype=part.dtype, device=part.device)
+    max_pos, rot_dim = cos_sin_cache.shape
+    cb, ct, ch = _cache_strides(k_cache, v_cache)
+    partition_size = decode_auto_partition(s, hkv, max_seq_len, bs, partition_size, None, False, head_dim=d)
+    need = decode_workspace_bytes(s, num_q_heads, d, max_seq_len, partition_size)
+    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
+        workspace = new_decode_workspace(need, part.device)
+    fused_merge = DECODE_FUSED_MERGE and _decode_ws_ready(workspace)
+    check("mi_rope_cache_paged_attn_decode_splitk", lib.mi_rope_cache_paged_attn_decode_splitk(
+        _p(out), _p(part.part), part.split, _p(part.bias), _p(positions), _p(cos_sin_cache), max_pos, rot_dim, _p(q_norm_weight),
+        _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache), _p(slot_mapping), _p(block_table), _p(seq_lens), s, num_q_heads,
+        hkv, d, bs, block_table.stride(0), int(max_seq_len), float(scale), out.stride(0), cb, ct, ch, int(partition_size),
+        _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(part.dtype), _dt(out.dtype),
+        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0), _stream()))
+    return out
+
+
 # --------------------------------------------------------------------------- A6
 _PREFILL_WS: dict = {}   # device -> grow-only fp32 workspace of the split-context prefill (never captured in a graph)
 
