@@ -626,25 +626,31 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
     win_b = bt_row[min(first_blk + 64 + lane, p.block_table_stride - 1)];
     asm volatile("" : "+v"(win_b));
   }
-  const auto fill = [&]() {
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      if (t_begin + i < t_end) {
-        issue_k(t_begin + i, i);
-        if (!PART || i < NS - 1) issue_v(t_begin + i, i);
-      }
-    }
-  };
   if constexpr (PART) {
     // the sums ride under the DMA, or stand in front of it where it fetches the token's row.  One copy of either's code
 #pragma unroll 1
     for (int turn = 0; turn < 2; ++turn) {
-      if ((turn == 0) == kv_early) sum_slabs();
-      else fill();
+      if ((turn == 0) == kv_early) {
+        sum_slabs();
+      } else {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+          if (t_begin + i < t_end) {
+            issue_k(t_begin + i, i);
+            if (i < NS - 1) issue_v(t_begin + i, i);
+          }
+        }
+      }
     }
     if (t_begin + NS - 1 < t_end) issue_v(t_begin + NS - 1, NS - 1);
   } else {
-    fill();
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      if (t_begin + i < t_end) {
+        issue_k(t_begin + i, i);
+        issue_v(t_begin + i, i);
+      }
+    }
   }
   if constexpr (ROPE) {
     // q: dims 32 s + 8 g .. of head h pair with dims + HD / 2 = fragment s + KS / 2 of the same lane
