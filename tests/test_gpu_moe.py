@@ -182,3 +182,57 @@ def test_tall_tiles_give_the_rows_of_low_ones(dev, dtype, n, k, form):
         got.append(out[rop.long()])
     assert not got[0].isnan().any() and got[0].abs().max() > 0
     assert all(torch.equal(got[0], o) for o in got[1:])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k,E,rpt,form", [
+    (4096, 320, 9, 32, "plain"),           # an odd number of k blocks; 144 tiles: quarters
+    (8192, 256, 33, 32, "plain"),          # the fewest k blocks; 32 tiles and halves
+    (640, 448, 5, 64, "gated"),            # a last tile that hangs over; fewer tiles than workgroups
+    (1920, 1024, 41, 64, "relu_squared"),  # 41 x 8 tiles, one round and quarters
+    (2944, 576, 64, 64, "gated"),          # several rounds
+])
+def test_streamed_experts_match_float64(dev, dtype, n, k, E, rpt, form):
+    """experts of a few rows (none, one, a whole tile) against float64; rows without a pair are not written"""
+    from vllm_omni_amd import _C, ops
+
+    lib, top = _C.lib, 2
+    pairs = torch.cat([torch.full(((rpt, 0, 1, 2 * rpt - 31, 33, 7)[e % 6],), e) for e in range(E)])
+    pairs = torch.cat([pairs, torch.full((-len(pairs) % top,), E - 1)])
+    g = torch.Generator().manual_seed(n + k)
+    ids = pairs[torch.randperm(len(pairs), generator=g)].to(torch.int32).to(dev).view(-1, top)
+    T, f = ids.shape[0], {"gated": _C.MI_MOE_GATED, "plain": _C.MI_MOE_PLAIN, "relu_squared": _C.MI_MOE_RELU_SQUARED}[form]
+    w = (torch.randn(E, (2 if form == "gated" else 1) * n, k, generator=g) * k ** -0.5).to(dtype).to(dev)
+    x = torch.randn(T * top if form == "plain" else T, k, generator=g).to(dtype).to(dev)
+    pw = torch.rand(T * top, generator=g).to(dev) if form == "relu_squared" else None
+    rows = int(lib.mi_moe_max_rows(T, top, E, rpt))
+    sp, rop, te, nt = ops._moe_align(ids, E, rows, rpt)
+    a = x
+    if form == "plain":
+        a = torch.full((rows, k), float("nan"), dtype=dtype, device=dev)
+        a[rop.long()] = x
+    out = torch.full((rows, n), float("nan"), dtype=dtype, device=dev)
+    ops.check("mi_moe_expert_gemm", lib.mi_moe_expert_gemm(
+        out.data_ptr(), a.data_ptr(), w.data_ptr(), sp.data_ptr(), te.data_ptr(), nt.data_ptr(), rows // rpt, f,
+        None if pw is None else pw.data_ptr(), n, k, top, a.stride(0), out.stride(0), w.stride(0), rpt, ops._dt(dtype),
+        torch.cuda.current_stream().cuda_stream))
+    got, e_of = out[rop.long()], ids.flatten().long()
+    ref = torch.empty(T * top, n, dtype=torch.float64, device=dev)
+    for e in range(E):
+        p = (e_of == e).nonzero().flatten()
+        if len(p) == 0:
+            continue
+        y = (x[p] if form == "plain" else x[p // top]).double() @ w[e].double().t()
+        if form == "gated":
+            gate, up = y[:, :n].to(dtype).double(), y[:, n:].to(dtype).double()
+            y = gate / (1 + torch.exp(-gate)) * up
+        elif form == "relu_squared":
+            y = torch.relu(y * pw[p, None].double()) ** 2
+        ref[p] = y
+    # an output ulp, and for the gated form the two factors' own ulps of rounding to the dtype (fp32 sums may land on the other side)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    tol = ref.abs() * ulp * (3 if form == "gated" else 1) + 1e-3 * ref.abs().amax(dim=1, keepdim=True).clamp_min(1.0)
+    assert bool(((got.double() - ref).abs() <= tol).all())
+    dead = torch.ones(rows, dtype=torch.bool, device=dev)
+    dead[rop.long()] = False
+    assert out[dead].isnan().all()

@@ -567,11 +567,13 @@ extern "C" int mi_moe_expert_gemm(void* out, const void* a_rows, const void* wei
       ga.a_row_stride = a_row_stride; ga.out_row_stride = out_row_stride; ga.weight_expert_stride = weight_expert_stride;
       ga.dtype = dtype;
       // Tall tiles on tall_gemm.hip; the ring kernel keeps them for k of an odd number of 64-blocks and operands past 32-bit
-      // offsets.  64-row tiles (24 to 48 rows an expert) are weight streaming: the tall kernel's 256-row weight tiles are ahead
-      // where an expert's product is large (4096 x 1536: 357 -> 335 us for both products), the ring's 128-row ones where it is
-      // small (2048 x 768: 105 against 115, 1024 x 384: 80 against 87)
-      const bool tall = rows_per_tile > 64 || (rows_per_tile == 64 && (int64_t)n_out * k >= (4 << 20));
-      int rc = tall ? launch_grouped_tall(ga, s) : MI_ERR_UNSUPPORTED;
+      // offsets.  Up to 64 rows it is weight streaming, and expert_stream.hip is ahead of the ring where its tiles fill the chip for
+      // several rounds or a round is short.  Down, us, ring | stream: 4096 x 1536, 64 experts, 8 chosen, 1 token 27 | 20, 7 tokens 94 | 89, 64
+      // 162 | 139, 200 176 | 144, 6 chosen, 32 tokens 146 | 130; 1024 x 384, 128 experts, 512 tokens 27 | 26, but 1 token (32 tiles)
+      // 6.7 | 7.2.  Up, 64-row tiles: 1536 x 4096, 200 tokens 174 | 154, gated 400 tokens 317 | 313, 384 x 1024 gated 44 | 42; 32-row
+      // tiles of a long k end in a round that is mostly idle: 64 tokens 162 | 173, gated 5 tokens 127 | 156, 32 tokens 254 | 262
+      const bool stream = form == MI_MOE_PLAIN ? rows_per_tile <= 64 && (int64_t)max_tiles * n_out >= 128 * 256 : rows_per_tile == 64;
+      int rc = rows_per_tile > 64 ? launch_grouped_tall(ga, s) : stream ? launch_grouped_stream(ga, s) : MI_ERR_UNSUPPORTED;
       if (rc == MI_ERR_UNSUPPORTED) rc = launch_grouped_skinny(ga, s);
       if (rc != MI_ERR_UNSUPPORTED) return rc;
     }

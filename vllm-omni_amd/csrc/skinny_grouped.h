@@ -23,7 +23,9 @@ struct GroupedGemmArgs {
 // MI_OK, or MI_ERR_UNSUPPORTED when the shape is outside the ring kernel's envelope (the caller then runs its
 // direct-from-global kernel).
 int launch_grouped_skinny(const GroupedGemmArgs& a, hipStream_t s);
-// Tiles of 64, 128 or 256 rows (tall_gemm.hip); MI_ERR_UNSUPPORTED outside its envelope.
+// Tiles of 32 or 64 rows (expert_stream.hip); MI_ERR_UNSUPPORTED outside its envelope.
+int launch_grouped_stream(const GroupedGemmArgs& a, hipStream_t s);
+// Tiles of 128 or 256 rows (tall_gemm.hip); MI_ERR_UNSUPPORTED outside its envelope.
 int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s);
 
 }  // namespace mi

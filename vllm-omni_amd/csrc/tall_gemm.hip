@@ -441,7 +441,7 @@ int launch_tall(const TallParams& p, int form, const dim3 grid, hipStream_t s) {
 
 int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s) {
   const bool gated = a.form == MI_MOE_GATED;
-  if (a.rows_per_tile != 64 && a.rows_per_tile != 128 && a.rows_per_tile != 256) return MI_ERR_UNSUPPORTED;
+  if (a.rows_per_tile != 128 && a.rows_per_tile != 256) return MI_ERR_UNSUPPORTED;
   if (a.k % 128 || a.n_out % 16 || a.out_row_stride % 8 || ((uintptr_t)a.out & 15) || (a.dtype != MI_DTYPE_BF16 && a.dtype != MI_DTYPE_F16)) return MI_ERR_UNSUPPORTED;
   // 32-bit byte offsets into the rows (a gathered row's number is at most its pair's) and into one expert's weights
   const int64_t rows = (int64_t)a.max_tiles * a.rows_per_tile, lim = (int64_t)1 << 32;
