@@ -498,7 +498,10 @@ extern "C" int32_t mi_paged_attn_decode_auto_partition(int32_t num_seqs, int32_t
   if (num_seqs <= 0 || num_kv_heads <= 0 || max_seq_len <= 0) return 256;
   const int64_t pairs = (int64_t)num_seqs * num_kv_heads;
   const int64_t want = head_dim > 0 && head_dim <= 64 ? 1024 : 512;
-  const int64_t parts = (want + pairs - 1) / pairs;
+  // head_dim 128, between five and seven waves a CU: five are resident (LDS), and a second round of so few would run on a part of the chip;
+  // three partitions each make it a stream of shorter waves (an odd number: see the kernel).  8 KV heads, one | three, us: 161 x 2048 263 | 231,
+  // up to 2048 156 | 145; 200 x 3001 431 | 409, up to 3001 283 | 264; 180 x 1200 169 | 159; past it 230 x 2500 389 | 397, 256 x 4096 698 | 712
+  const int64_t parts = head_dim > 64 && pairs > 1280 && pairs <= 1792 && max_seq_len > 1024 ? 3 : (want + pairs - 1) / pairs;
   int64_t ps = mi::round_up((int32_t)((max_seq_len + parts - 1) / parts), 32);
   const int64_t least = parts < 3 ? 256 : std::min(256, std::max(64, mi::round_up((int32_t)(((int64_t)max_seq_len + 7) / 8), 32)));
   if (ps < least) ps = least;

@@ -171,7 +171,10 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
   lds_char* const rings = ring_base<GROUP, NS * STAGE>();
   lds_char* const smem = rings + wid * (NS * STAGE);
   const int wave = GROUP ? blockIdx.x * p.num_parts + wid : blockIdx.x;
-  const int part = GROUP ? wid : wave % p.num_parts;
+  // Lone waves: a sequence's partitions side by side, turned by one every eight sequences' heads: without the turn an even number of them
+  // gives an XCD the same partitions of all sequences, and where those end in different ones half of the XCDs the emptier (200 x up to 3001
+  // tokens, 8 heads of 128: two partitions 314 us, three 263, four 333).
+  const int part = GROUP ? wid : p.num_parts == 1 ? 0 : (wave + wave / (8 * p.num_parts)) % p.num_parts;
   const int hw = (wave / p.num_parts) % (p.num_q_heads / gh);
   const int seq = wave / (p.num_parts * (p.num_q_heads / gh));
   const int qh0 = hw * gh;

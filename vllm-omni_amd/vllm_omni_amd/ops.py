@@ -298,7 +298,8 @@ def decode_auto_partition(num_seqs: int, num_kv_heads: int, max_seq_len: int, bl
                           requested: int = 0, packed_pv: Optional[bool] = None, force_valu: bool = False,
                           head_dim: int = 128) -> int:
     """Partition size a decode call will really use: ``requested``, or the auto choice — the fewest partitions that
-    leave >= 512 waves (1024 at head_dim 64), ONE (direct output, no merge launch) once sequences x KV heads reach that;
+    leave >= 512 waves (1024 at head_dim 64), ONE (direct output, no merge launch) once sequences x KV heads reach that,
+    three where those alone are a little more than the chip holds at once;
     any multiple of 32 tokens for the matrix-core kernel, capped at 64 blocks for the VALU kernel (``packed_pv`` False /
     ``force_valu``)."""
     return int(lib.mi_paged_attn_decode_effective_partition(num_seqs, num_kv_heads, max_seq_len, head_dim, block_size,
