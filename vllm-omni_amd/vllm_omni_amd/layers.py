@@ -389,10 +389,10 @@ def _tall_wins(m: int, n: int, k: int, dtype: torch.dtype, gated: bool = False) 
     (18944 x 3584, 1000 rows 316 / 253, 6719 rows 1497 / 1403; 512 rows 148 / 167).  Where the library's solution was selected by
     measurement at exactly this row count it keeps the shape (3584 x 18944, 8192 rows 794 / 853), and so it does elsewhere (3584 x 3584,
     6719 rows 129 / 165; 4096 x 16384 0.9 to 2.1 times as fast)."""
-    from .tuned import has_tuned_gemm
-
     if m <= 256 or _LINEAR_MODE != "auto" or not ops.linear_tall_supported(m, n, k, dtype, gated):
         return False
+    from .tuned import has_tuned_gemm
+
     if has_tuned_gemm(m, 2 * n if gated else n, k, dtype):
         return False
     if gated:
@@ -503,7 +503,7 @@ def _apply_linear(layer, x: torch.Tensor, bias: Optional[torch.Tensor], defer_re
     if _LINEAR_MODE != "library" and x.is_cuda:
         m = x.numel() // x.shape[-1]
         n, k = w.shape
-        if _tall_wins(m, n, k, x.dtype):
+        if m > 256 and _tall_wins(m, n, k, x.dtype):
             return ops.linear_tall(x, w, bias)
         e = _tuned(m, n, k) if ops.linear_supported(m, n, k, x.dtype) else None
         if e is not None and e.get("full"):
@@ -523,7 +523,7 @@ def _apply_linear(layer, x: torch.Tensor, bias: Optional[torch.Tensor], defer_re
                     return pr
             return ops.linear(x, w, bias) if e["full"]["us"] < e["library_us"] else F.linear(x, w, bias)
         if ops.linear_supported(m, n, k, x.dtype):
-            wins = (_LINEAR_MODE == "kernel" or _streaming_kernel_wins(m, n, k) or _narrow_kernel_wins(m, n, k)
+            wins = (_LINEAR_MODE == "kernel" or _streaming_kernel_wins(m, n, k) or (m <= 128 and _narrow_kernel_wins(m, n, k))
                     or (_LINEAR_MODE in ("mlp", "mlp+o") and getattr(layer, "_is_down_proj", False))
                     or (_LINEAR_MODE == "mlp+o" and getattr(layer, "_is_o_proj", False)))
             if defer_reduce == "attn":
