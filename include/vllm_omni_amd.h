@@ -228,10 +228,18 @@ int mi_rope_cache_attend_block_splitk(void* out, const void* partials, int32_t s
  * context is left out — `out` is then NOT written, unless the partitions merge inside the attention launch (few of
  * them, as the waves of one workgroup).  Never set by the product. */
 #define MI_DECODE_SKIP_MERGE 32
+/* MI_DECODE_SEQ_ORDER: seq_lens is what mi_decode_seq_order wrote for this call's sequences and sizes: their lengths, then the order that the
+ * launch takes them in (matrix-core kernel; the others run them as they are).  Speed only: outputs keep their bits. */
+#define MI_DECODE_SEQ_ORDER 64
 #define MI_DECODE_COUNTER_BYTES (1 << 20)
 int64_t mi_paged_attn_decode_workspace_bytes(int32_t num_seqs, int32_t num_q_heads,
                                              int32_t head_dim, int32_t max_seq_len,
                                              int32_t partition_size);
+/* lens_and_order [2 * num_seqs]: a copy of seq_lens, then the order in which a decode launch of these sizes (and flags) should take the
+ * sequences: for calls with MI_DECODE_SEQ_ORDER of one step, whose lengths are the same in every layer.  MI_ERR_UNSUPPORTED: such a launch
+ * gains nothing from an order (nothing is written). */
+int mi_decode_seq_order(int32_t* lens_and_order, const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                        int32_t head_dim, int32_t block_size, int32_t max_seq_len, int32_t partition_size, int32_t flags, void* stream);
 int mi_paged_attn_decode(void* out, const void* q, const void* k_cache, const void* v_cache,
                          const int32_t* block_table, const int32_t* seq_lens,
                          int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
@@ -928,6 +936,16 @@ int mi_paged_attn_decode_biased(void* out, const void* q, const void* k_cache, c
                                 int64_t cache_block_stride, int64_t cache_token_stride,
                                 int64_t cache_head_stride, int32_t partition_size, void* workspace,
                                 int64_t workspace_bytes, int dtype, void* stream);
+/* ... with flags: MI_DECODE_SEQ_ORDER or 0 */
+int mi_paged_attn_decode_biased_ordered(void* out, const void* q, const void* k_cache, const void* v_cache,
+                                        const int32_t* block_table, const int32_t* seq_lens,
+                                        const float* slopes, const float* sinks, float out_scale,
+                                        int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                        int32_t block_size, int32_t block_table_stride, int32_t max_seq_len,
+                                        float scale, int64_t q_token_stride, int64_t out_token_stride,
+                                        int64_t cache_block_stride, int64_t cache_token_stride,
+                                        int64_t cache_head_stride, int32_t partition_size, void* workspace,
+                                        int64_t workspace_bytes, int dtype, int32_t flags, void* stream);
 int mi_paged_attn_prefill_biased(void* out, const void* q, const void* k_cache, const void* v_cache,
                                  const int32_t* block_table, const int32_t* seq_lens,
                                  const int32_t* query_start_loc, const float* slopes,

@@ -49,12 +49,20 @@ struct DecodeParams {
   int32_t num_slabs = 0;
   int64_t slab_stride = 0, slab_row = 0;
   bool group_parts = false;   // matrix-core kernel: the partitions are the waves of a workgroup and merge there
+  const int32_t* seq_order = nullptr;   // ... [num_seqs]: the sequence of every place in the launch (decode_seq_order), nullptr: as they are
   int32_t turn = 0;           // ... lone waves: the order of a head group's partitions moves by one every so many waves (0: it does not)
 };
 
 // paged_attn_decode_mfma.hip
 // whether to set p.group_parts; groups = sequences x head groups
 bool decode_mfma_groups(int64_t groups, int num_parts, int head_dim, int max_seq_len);
+// How the sequences of a launch are ordered: `per` of them make a round of workgroups (0: not ordered), the odd ones of the first `turned`
+// rounds run the other way
+struct DecodeOrder {
+  int32_t per, turned;
+};
+DecodeOrder decode_mfma_order(int num_seqs, int groups_per_seq, int num_parts, bool group_parts, int head_dim, int max_seq_len);
+int launch_decode_order(int32_t* lens_and_order, const int32_t* seq_lens, int num_seqs, DecodeOrder order, hipStream_t stream);
 // p.turn of a launch of lone waves
 int32_t decode_mfma_turn(int64_t groups, int num_parts);
 int launch_decode_mfma(const DecodeParams& p, int heads_per_wave, int head_dim, int dtype, bool nontemporal,

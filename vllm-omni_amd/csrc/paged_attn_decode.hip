@@ -639,6 +639,7 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
   p.group_parts = use_mfma && decode_mfma_groups((int64_t)num_seqs * (num_q_heads / G), num_parts, head_dim, max_seq_len);
   if (p.group_parts) p.part_count = nullptr;
   p.turn = decode_mfma_turn((int64_t)num_seqs * (num_q_heads / G), num_parts);
+  if (use_mfma && (flags & MI_DECODE_SEQ_ORDER)) p.seq_order = seq_lens + num_seqs;
   p.num_seqs = num_seqs;
   p.num_q_heads = num_q_heads;
   p.kv_group = kv_group;
@@ -715,6 +716,36 @@ extern "C" int mi_paged_attn_decode(void* out, const void* q, const void* k_cach
                      workspace_bytes, dtype, out_dtype, flags, stream, nullptr);
 }
 
+extern "C" int mi_decode_seq_order(int32_t* lens_and_order, const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                   int32_t head_dim, int32_t block_size, int32_t max_seq_len, int32_t partition_size, int32_t flags, void* stream) {
+  using namespace mi;
+  if (!lens_and_order || !seq_lens || num_seqs <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || max_seq_len <= 0 || num_q_heads % num_kv_heads != 0)
+    return MI_ERR_INVALID_ARG;
+  if (head_dim != 64 && head_dim != 128) return MI_ERR_UNSUPPORTED;
+  const int32_t ps = mi_paged_attn_decode_effective_partition(num_seqs, num_kv_heads, max_seq_len, head_dim, block_size, partition_size, flags);
+  if (!(flags & MI_DECODE_PACKED_PV) || (flags & MI_DECODE_FORCE_VALU) || block_size < 16 || ps <= 0 || ps % 32) return MI_ERR_UNSUPPORTED;
+  const int parts = (max_seq_len + ps - 1) / ps, groups = num_q_heads / heads_per_wave(num_q_heads / num_kv_heads, 16);
+  const DecodeOrder o = decode_mfma_order(num_seqs, groups, parts, decode_mfma_groups((int64_t)num_seqs * groups, parts, head_dim, max_seq_len),
+                                          head_dim, max_seq_len);
+  if (!o.per) return MI_ERR_UNSUPPORTED;
+  return launch_decode_order(lens_and_order, seq_lens, num_seqs, o, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int mi_paged_attn_decode_biased_ordered(void* out, const void* q, const void* k_cache, const void* v_cache,
+                                                   const int32_t* block_table, const int32_t* seq_lens, const float* slopes,
+                                                   const float* sinks, float out_scale, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                                   int32_t head_dim, int32_t block_size, int32_t block_table_stride,
+                                                   int32_t max_seq_len, float scale, int64_t q_token_stride,
+                                                   int64_t out_token_stride, int64_t cache_block_stride,
+                                                   int64_t cache_token_stride, int64_t cache_head_stride, int32_t partition_size,
+                                                   void* workspace, int64_t workspace_bytes, int dtype, int32_t flags, void* stream) {
+  return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                     block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
+                     cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
+                     workspace_bytes, dtype, dtype, MI_DECODE_PACKED_PV | MI_DECODE_NONTEMPORAL | (flags & MI_DECODE_SEQ_ORDER), stream, nullptr, slopes,
+                     sinks, out_scale);
+}
+
 extern "C" int mi_paged_attn_decode_biased(void* out, const void* q, const void* k_cache, const void* v_cache,
                                            const int32_t* block_table, const int32_t* seq_lens, const float* slopes,
                                            const float* sinks, float out_scale, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
@@ -723,11 +754,10 @@ extern "C" int mi_paged_attn_decode_biased(void* out, const void* q, const void*
                                            int64_t out_token_stride, int64_t cache_block_stride,
                                            int64_t cache_token_stride, int64_t cache_head_stride, int32_t partition_size,
                                            void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
-  return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                     block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
-                     cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
-                     workspace_bytes, dtype, dtype, MI_DECODE_PACKED_PV | MI_DECODE_NONTEMPORAL, stream, nullptr, slopes,
-                     sinks, out_scale);
+  return mi_paged_attn_decode_biased_ordered(out, q, k_cache, v_cache, block_table, seq_lens, slopes, sinks, out_scale, num_seqs, num_q_heads,
+                                             num_kv_heads, head_dim, block_size, block_table_stride, max_seq_len, scale, q_token_stride,
+                                             out_token_stride, cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
+                                             workspace_bytes, dtype, 0, stream);
 }
 
 extern "C" int mi_rope_cache_paged_attn_decode(void* out, const void* q, const void* k, const void* v,

@@ -28,6 +28,7 @@ MI_DECODE_NONTEMPORAL = 4
 MI_DECODE_ROUNDED_P = 8
 MI_DECODE_FUSED_MERGE = 16
 MI_DECODE_SKIP_MERGE = 32
+MI_DECODE_SEQ_ORDER = 64
 MI_DECODE_COUNTER_BYTES = 1 << 20
 MI_ALLREDUCE_MAX_RANKS, MI_ALLREDUCE_HANDLE_BYTES = 8, 64
 
@@ -212,6 +213,9 @@ SIGNATURES = {
                              c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, _P]),
     "mi_paged_attn_decode_biased": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_float, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
                                             c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, _P]),
+    "mi_paged_attn_decode_biased_ordered": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_float, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
+                                                    c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, c_int32, _P]),
+    "mi_decode_seq_order": (c_int, [_P, _P, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, _P]),
     "mi_paged_attn_prefill_biased": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, c_float, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
                                              c_int32, c_int32, c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int32,
                                              c_int32, _P, c_int64, _P]),

@@ -57,7 +57,18 @@ class AttentionMetadata:
     # matrix its attention runs on (64-row aligned)
     prefill_ctx: dict = field(default_factory=dict)
     step_cache: dict = field(default_factory=dict)   # what layers of one step share (gathered contexts)
+    # sizes -> ops.decode_seq_order of the decode rows; a dict of ONE forward pass (the runner makes it), None: launches take the rows as they are
+    decode_orders: Optional[dict] = None
     prev_slots: Optional[torch.Tensor] = None   # int32 [num_tokens], device: slot a row leaves its token in (a request's last row), else -1
+
+    def decode_order(self, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int) -> Optional[torch.Tensor]:
+        """the order the pass's decode attention launches of these sizes take the rows in: made by the first of them"""
+        if self.decode_orders is None:
+            return None
+        key = (num_q_heads, num_kv_heads, head_dim, block_size)
+        if key not in self.decode_orders:
+            self.decode_orders[key] = ops.decode_seq_order(self.seq_lens[:self.num_decodes], *key, self.max_seq_len, self.decode_partition_size)
+        return self.decode_orders[key]
 
 
 @dataclass
@@ -230,12 +241,15 @@ class Attention:
         self.kv_cache = layer_kv
         self._kb, self._vb = pair
 
+    def _order(self, md: AttentionMetadata) -> Optional[torch.Tensor]:
+        return md.decode_order(self.num_heads, self.num_kv_heads, self.head_size, self._kb.shape[1])
+
     def _attend(self, q: torch.Tensor, md: AttentionMetadata, out: torch.Tensor) -> torch.Tensor:
         nd = md.num_decodes
         if nd > 0:
             ops.paged_attn_decode(out[:nd], q[:nd], self._kb, self._vb, md.block_table[:nd], md.seq_lens[:nd],
                                   md.max_seq_len, self.scale, partition_size=md.decode_partition_size,
-                                  workspace=md.decode_workspace)
+                                  workspace=md.decode_workspace, order=self._order(md))
         if nd < md.num_reqs:
             t0 = nd  # decodes come first and have one token each
             ops.paged_attn_prefill(out[t0:md.num_actual_tokens], q[t0:md.num_actual_tokens], self._kb, self._vb,
@@ -293,7 +307,7 @@ class Attention:
                                              self._vb, md.slot_mapping[:nd], md.block_table[:nd], md.seq_lens[:nd],
                                              md.max_seq_len, self.scale, partition_size=md.decode_partition_size,
                                              workspace=md.decode_workspace, q_norm_weight=q_norm_weight,
-                                             k_norm_weight=k_norm_weight, norm_eps=norm_eps)
+                                             k_norm_weight=k_norm_weight, norm_eps=norm_eps, order=self._order(md))
             return out
         ops.rope_neox_and_cache(q, k, v, positions, rope.cos_sin_cache, self.head_size, self._kb, self._vb,
                                 md.slot_mapping, mrope_section=sec, q_norm_weight=q_norm_weight,
@@ -317,7 +331,8 @@ class Attention:
             return ops.rope_cache_paged_attn_decode_splitk(
                 qkv, self.num_heads, self.num_kv_heads, self.head_size, positions, rope.cos_sin_cache, self._kb, self._vb,
                 md.slot_mapping, md.block_table, md.seq_lens, md.max_seq_len, self.scale, partition_size=md.decode_partition_size,
-                workspace=md.decode_workspace, q_norm_weight=q_norm_weight, k_norm_weight=k_norm_weight, norm_eps=norm_eps)
+                workspace=md.decode_workspace, q_norm_weight=q_norm_weight, k_norm_weight=k_norm_weight, norm_eps=norm_eps,
+                order=self._order(md))
         q = ops.rope_neox_and_cache_splitk(qkv, self.num_heads, self.num_kv_heads, self.head_size, positions,
                                            rope.cos_sin_cache, self._kb, self._vb, md.slot_mapping,
                                            mrope_section=rope._section(positions), q_norm_weight=q_norm_weight,

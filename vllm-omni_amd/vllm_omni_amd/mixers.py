@@ -452,7 +452,8 @@ class KeyValueAttention:
         else:
             if nd:
                 ops.paged_attn_decode(out[:nd], q[:nd], kc, vc, md.block_table[:nd], md.seq_lens[:nd], md.max_seq_len, c.scale,
-                                      workspace=md.decode_workspace, sinks=self.sinks)
+                                      workspace=md.decode_workspace, sinks=self.sinks,
+                                      order=md.decode_order(c.heads, kc.shape[2], self.head_dim, kc.shape[1]))
             if nd < n:      # the portions' row offsets count from the step's first row, so q and out go whole
                 ops.paged_attn_prefill(out, q, kc, vc, md.block_table[nd:n], md.seq_lens[nd:n], md.query_start_loc[nd:n + 1],
                                        md.max_query_len, c.scale, max_seq_len=md.max_seq_len, sinks=self.sinks)
@@ -731,7 +732,8 @@ class SinkAttention(Sublayer):
             return
         if nd:
             ops.paged_attn_decode(out[:nd], q[:nd], kc, vc, md.block_table[:nd], md.seq_lens[:nd], md.max_seq_len, c.scale,
-                                  workspace=md.decode_workspace, **bias)
+                                  workspace=md.decode_workspace, **bias,
+                                  order=md.decode_order(c.heads, kc.shape[2], self.head_dim, kc.shape[1]))
         if nd < md.num_reqs:      # the portions' row offsets count from the step's first row, so q and out go whole
             ops.paged_attn_prefill(out, q, kc, vc, md.block_table[nd:md.num_reqs], md.seq_lens[nd:md.num_reqs],
                                    md.query_start_loc[nd:md.num_reqs + 1], md.max_query_len, c.scale, max_seq_len=md.max_seq_len, **bias)

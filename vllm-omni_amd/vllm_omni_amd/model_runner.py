@@ -1107,6 +1107,7 @@ class GPUARModelRunner:
     # ------------------------------------------------------------------- forward
     def _forward(self, n: int, total: int, md: AttentionMetadata):
         """Model forward + logits + fused mask/argmax on the static buffers."""
+        md.decode_orders = {}      # this pass's own: a captured pass has to make its orders inside the graph
         with set_forward_context(md):
             if self._token_ids:
                 ids = self.last_token_ids.gpu[:n] if md.num_decodes == n == total else self.input_ids.gpu[:total]

@@ -361,7 +361,7 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                       packed_pv: Optional[bool] = None, force_valu: bool = False,
                       nontemporal: Optional[bool] = None, rounded_p: bool = False,
                       fused_merge: Optional[bool] = None, _skip_merge: bool = False, slopes: Optional[torch.Tensor] = None,
-                      sinks: Optional[torch.Tensor] = None, out_scale: float = 1.0) -> torch.Tensor:
+                      sinks: Optional[torch.Tensor] = None, out_scale: float = 1.0, order: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[s, h] = softmax(q[s,h] . K^T * scale) . V over the paged cache (one query per sequence).
 
     q, out: [S, nq*d] (or [S, nq, d]); block_table int32 [S, max_blocks]; seq_lens int32 [S].
@@ -375,8 +375,9 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     wave of each (sequence, head group) instead of a second kernel — same bits.  Returns ``out``.
     ``slopes`` / ``sinks`` (fp32 [nq]): a distance bias (score - slope * (position - key position)) and one more term
     exp(sink) of the softmax's denominator, and the output times ``out_scale``; bf16 and the default mode only.
+    ``order``: ``decode_seq_order`` of these lengths and sizes (speed only: same bits).
     """
-    _gpu(out, q, k_cache, v_cache, block_table, seq_lens, workspace, slopes, sinks)
+    _gpu(out, q, k_cache, v_cache, block_table, seq_lens, workspace, slopes, sinks, order)
     nb, bs, hkv, d = k_cache.shape
     s = q.shape[0]
     nq = q.numel() // (s * d) if s else 0
@@ -396,19 +397,20 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         fused_merge = DECODE_FUSED_MERGE and ready
     elif fused_merge and not ready:
         raise ValueError("fused_merge needs a workspace from ops.new_decode_workspace (zeroed arrival counters)")
+    lens, ordered = _ordered_lens(seq_lens, order, s)
     if slopes is None and sinks is None and out_scale != 1.0:
         raise ValueError("out_scale goes with a distance bias or a sink")
     if slopes is not None or sinks is not None:
         _head_vectors(nq, slopes, sinks)
         if force_valu or rounded_p or packed_pv is False or out.dtype != q.dtype:
             raise ValueError("a distance bias or a sink runs in the default mode only")
-        check("mi_paged_attn_decode_biased", lib.mi_paged_attn_decode_biased(
-            _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(seq_lens), _p(slopes), _p(sinks), float(out_scale), s, nq, hkv, d, bs,
+        check("mi_paged_attn_decode_biased_ordered", lib.mi_paged_attn_decode_biased_ordered(
+            _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(lens), _p(slopes), _p(sinks), float(out_scale), s, nq, hkv, d, bs,
             block_table.stride(0), int(max_seq_len), float(scale), q.stride(0), out.stride(0), cb, ct, ch, int(partition_size),
-            _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(q.dtype), _stream()))
+            _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(q.dtype), ordered, _stream()))
         return out
     check("mi_paged_attn_decode", lib.mi_paged_attn_decode(
-        _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(seq_lens), s, nq, hkv, d, bs,
+        _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(lens), s, nq, hkv, d, bs,
         block_table.stride(0), int(max_seq_len), float(scale), q.stride(0), out.stride(0), cb, ct, ch,
         int(partition_size), _p(workspace),
         workspace.numel() * workspace.element_size() if workspace is not None else 0,
@@ -417,10 +419,40 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         | (_C.MI_DECODE_FORCE_VALU if force_valu else 0)
         | (_C.MI_DECODE_ROUNDED_P if rounded_p else 0)
         | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0)
+        | ordered
         | (_C.MI_DECODE_SKIP_MERGE if _skip_merge else 0)   # bench.py's kernel-only timing; never set by the product
         | (_C.MI_DECODE_NONTEMPORAL if (DECODE_NONTEMPORAL if nontemporal is None else nontemporal) else 0),
         _stream()))
     return out
+
+
+def decode_seq_order(seq_lens: torch.Tensor, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int, max_seq_len: int,
+                     partition_size: int = 0) -> Optional[torch.Tensor]:
+    """int32 [2, S] on the device: the lengths, and the order in which the decode attention launches of one step (the default mode, these
+    sizes) should take the sequences — longest first.  For their ``order`` as long as ``seq_lens`` holds these values.  None where a
+    launch gains nothing from it."""
+    _gpu(seq_lens)
+    _i32(seq_lens)
+    s = seq_lens.numel()
+    if s == 0 or not DECODE_PACKED_PV or not seq_lens.is_contiguous():
+        return None
+    partition_size = decode_auto_partition(s, num_kv_heads, max_seq_len, block_size, partition_size, head_dim=head_dim)
+    out = torch.empty(2, s, dtype=torch.int32, device=seq_lens.device)
+    code = lib.mi_decode_seq_order(_p(out), _p(seq_lens), s, num_q_heads, num_kv_heads, head_dim, block_size, int(max_seq_len),
+                                   int(partition_size), _C.MI_DECODE_PACKED_PV, _stream())
+    if code == _C.MI_ERR_UNSUPPORTED:
+        return None
+    check("mi_decode_seq_order", code)
+    return out
+
+
+def _ordered_lens(seq_lens: torch.Tensor, order: Optional[torch.Tensor], s: int):
+    """(what a decode launch of s sequences reads as their lengths, its flag)"""
+    if order is None:
+        return seq_lens, 0
+    if order.dtype != torch.int32 or tuple(order.shape) != (2, s) or not order.is_contiguous():
+        raise ValueError("order: decode_seq_order of this call's sequences")
+    return order, _C.MI_DECODE_SEQ_ORDER
 
 
 def rope_decode_fusable(q: torch.Tensor, k_cache: torch.Tensor, positions: torch.Tensor, rot_dim: int,
@@ -440,12 +472,12 @@ def rope_cache_paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k: torch.Te
                                  seq_lens: torch.Tensor, max_seq_len: int, scale: float, partition_size: int = 0,
                                  workspace: Optional[torch.Tensor] = None, _skip_merge: bool = False,
                                  q_norm_weight: Optional[torch.Tensor] = None, k_norm_weight: Optional[torch.Tensor] = None,
-                                 norm_eps: float = 1e-6) -> torch.Tensor:
+                                 norm_eps: float = 1e-6, order: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``rope_neox_and_cache`` + ``paged_attn_decode`` of a pure-decode step in ONE launch (same bits): q is rotated in
     registers (the tensor keeps its un-rotated values), the token's rotated k and its v are written to the cache by the
     wave that owns the sequence's last context partition.  q [S, nq*d], k / v [S, nkv*d]: views of the qkv row."""
     _gpu(out, q, k, v, positions, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, seq_lens, workspace,
-         q_norm_weight, k_norm_weight)
+         q_norm_weight, k_norm_weight, order)
     if (q_norm_weight is None) != (k_norm_weight is None):
         raise ValueError("q_norm_weight and k_norm_weight come together")
     nb, bs, hkv, d = k_cache.shape
@@ -466,13 +498,14 @@ def rope_cache_paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k: torch.Te
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = new_decode_workspace(need, q.device)
     fused_merge = DECODE_FUSED_MERGE and _decode_ws_ready(workspace)
+    lens, ordered = _ordered_lens(seq_lens, order, s)
     check("mi_rope_cache_paged_attn_decode", lib.mi_rope_cache_paged_attn_decode(
         _p(out), _p(q), _p(k), _p(v), _p(positions), _p(cos_sin_cache), max_pos, rot_dim, _p(q_norm_weight),
         _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache),
-        _p(slot_mapping), _p(block_table), _p(seq_lens), s, nq, hkv, d, bs, block_table.stride(0), int(max_seq_len),
+        _p(slot_mapping), _p(block_table), _p(lens), s, nq, hkv, d, bs, block_table.stride(0), int(max_seq_len),
         float(scale), q.stride(0), k.stride(0), v.stride(0), out.stride(0), cb, ct, ch, int(partition_size), _p(workspace),
         workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(q.dtype), _dt(out.dtype),
-        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0)
+        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | ordered | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0)
         | (_C.MI_DECODE_SKIP_MERGE if _skip_merge else 0), _stream()))
     return out
 
@@ -482,10 +515,11 @@ def rope_cache_paged_attn_decode_splitk(part: "SplitKPartials", num_q_heads: int
                                         v_cache: torch.Tensor, slot_mapping: torch.Tensor, block_table: torch.Tensor,
                                         seq_lens: torch.Tensor, max_seq_len: int, scale: float, partition_size: int = 0,
                                         workspace: Optional[torch.Tensor] = None, q_norm_weight: Optional[torch.Tensor] = None,
-                                        k_norm_weight: Optional[torch.Tensor] = None, norm_eps: float = 1e-6) -> torch.Tensor:
+                                        k_norm_weight: Optional[torch.Tensor] = None, norm_eps: float = 1e-6,
+                                        order: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``rope_cache_paged_attn_decode`` fed by the split-K partials of ``qkv_proj`` (``linear_partials``): returns the
     attention output [S, nq*d].  Bit-identical to ``linear`` + ``rope_cache_paged_attn_decode``."""
-    _gpu(positions, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, seq_lens, workspace, q_norm_weight, k_norm_weight)
+    _gpu(positions, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, seq_lens, workspace, q_norm_weight, k_norm_weight, order)
     part._live()
     if part.n != (num_q_heads + 2 * num_kv_heads) * head_dim:
         raise ValueError("partials row is not [q heads | k heads | v heads]")
@@ -511,12 +545,13 @@ def rope_cache_paged_attn_decode_splitk(part: "SplitKPartials", num_q_heads: int
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = new_decode_workspace(need, part.device)
     fused_merge = DECODE_FUSED_MERGE and _decode_ws_ready(workspace)
+    lens, ordered = _ordered_lens(seq_lens, order, s)
     check("mi_rope_cache_paged_attn_decode_splitk", lib.mi_rope_cache_paged_attn_decode_splitk(
         _p(out), _p(part.part), part.split, _p(part.bias), _p(positions), _p(cos_sin_cache), max_pos, rot_dim, _p(q_norm_weight),
-        _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache), _p(slot_mapping), _p(block_table), _p(seq_lens), s, num_q_heads,
+        _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache), _p(slot_mapping), _p(block_table), _p(lens), s, num_q_heads,
         hkv, d, bs, block_table.stride(0), int(max_seq_len), float(scale), out.stride(0), cb, ct, ch, int(partition_size),
         _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(part.dtype), _dt(out.dtype),
-        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0), _stream()))
+        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | ordered | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0), _stream()))
     return out
 
 
