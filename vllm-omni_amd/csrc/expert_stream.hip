@@ -13,10 +13,12 @@
 //   * Rows without a pair, weight rows past the last one and stages past the last tile are loads past the end of a buffer: they count,
 //     but read nothing.  Rows without a pair are not stored.
 //   * Stores at a tile's end count like loads: the next tile's first two waits allow for them.
+//   * Weight rows a multiple of 4096 bytes apart: every tile's k blocks begin with another one (StreamParams::turn), or all workgroups, which keep step
+//     with each other, read from the same few channels at a time.  4096 x 1536, 200 tokens, 8 of 64, up 149 | 126 us; 2048 x 768 44.5 | 35.7.
 //   * Tiles that would leave half of an XCD's workgroups idle or more in its last round are cut into halves or quarters of their weight
 //     rows (expert_stream_items.h: an item of them that begins past the last column reads, multiplies and stores nothing).
-// Cold weights, us, the ring kernel before | this: 64 experts of 4096 x 1536, 8 of them a token, 200 tokens, up with relu squared 172 | 143, down
-// 177 | 142 (5.6 and 5.7 TB/s); 6 a token, 32 tokens, down 154 | 123; 128 experts of 1024 x 384, 512 tokens, down 27 | 23.
+// Cold weights, us, the ring kernel before | this: 64 experts of 4096 x 1536, 8 of them a token, 200 tokens, up with relu squared 172 | 126, down
+// 177 | 142 (6.4 and 5.7 TB/s); 6 a token, 32 tokens, down 154 | 123; 128 experts of 1024 x 384, 512 tokens, down 27 | 23.
 #include "expert_stream_items.h"
 #include "mfma_attn_common.h"
 #include "skinny_grouped.h"
@@ -32,6 +34,7 @@ struct StreamParams {
   int32_t N, K;
   int32_t rpt, gather_div;      // rows per tile; > 0: source row = pair index / gather_div, else the row itself
   int32_t nx;                   // weight tiles of a row tile
+  int32_t turn;                 // a tile's k blocks begin with grouped_first_block and go round
   uint32_t div_magic;           // 2^32 / gather_div, rounded up: exact for pair indices below 2^28
   uint32_t map_bytes;
   const int32_t* row_map;       // [max_rows] pair index or -1; the pairs of a tile in front
@@ -123,6 +126,7 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
   StreamItem lt;
   __amdgpu_buffer_rsrc_t wr = x_r;
   uint32_t xo[2], xn[2];
+  int w_first = 0, x_first = 0, xn_first = 0;      // the blocks that the tiles begin with
   int pieces = 0, n_loaded = 0;      // n_loaded: tiles taken up so far
   const auto take = [&]() {
     const int i = item + n_loaded * per;
@@ -153,15 +157,17 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
     const StreamRange r = stream_range(lt.col, lt.cut, p.N, p.K, GATED);
     wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w + (int64_t)lt.expert * p.w_expert_stride + r.first), 0, (int)r.bytes, 0x00020000);
     pieces = r.pieces;
+    if (p.turn) w_first = xn_first = grouped_first_block(GATED, lt.expert, lt.col, p.N, n_it);
     ++n_loaded;
     if (item + n_loaded * per < items) load_map(item + n_loaded * per, n_loaded % 3);
   };
   int w_it = 0, w_slot = 0, x_it = 0, x_slot = 0;
   const auto issue_w = [&]() {
+    const int kb = 128 * (w_it + w_first - (w_it + w_first < n_it ? 0 : n_it));
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(lds + w_slot * kWStage + (wid + 4 * i) * 1024), 16, i < pieces ? wo[i] : kDead,
-                                               w_it * 128, 0, MI_SKINNY_W_AUX);
+                                               kb, 0, MI_SKINNY_W_AUX);
     w_slot = (w_slot + 1) & 3;
     if (++w_it == n_it) {
       w_it = 0;
@@ -169,14 +175,16 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
     }
   };
   const auto issue_x = [&]() {
+    const int kb = 128 * (x_it + x_first - (x_it + x_first < n_it ? 0 : n_it));
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_r, (lds_void*)(lds + kXRing + x_slot * kXStage + (wid + 4 * i) * 1024), 16, xo[i], x_it * 128, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_r, (lds_void*)(lds + kXRing + x_slot * kXStage + (wid + 4 * i) * 1024), 16, xo[i], kb, 0, 0);
     x_slot = x_slot == 2 ? 0 : x_slot + 1;
     if (++x_it == n_it) {
       x_it = 0;
       xo[0] = xn[0];
       xo[1] = xn[1];
+      x_first = xn_first;
     }
   };
 
@@ -185,6 +193,7 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
   take();
   xo[0] = xn[0];
   xo[1] = xn[1];
+  x_first = xn_first;
   StreamItem t = lt;
   issue_w();
   issue_x();
@@ -348,6 +357,7 @@ int launch_grouped_stream(const GroupedGemmArgs& a, hipStream_t s) {
   p.w_expert_stride = a.weight_expert_stride;
   const int cols = gated ? kStreamRows / 2 : kStreamRows;
   p.nx = (a.n_out + cols - 1) / cols;
+  p.turn = grouped_turn(a.k);
   const dim3 grid(256);
   return a.dtype == MI_DTYPE_BF16 ? launch_stream<bf16_tag>(p, a.form, grid, s) : launch_stream<f16_tag>(p, a.form, grid, s);
 }

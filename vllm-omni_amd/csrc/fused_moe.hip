@@ -602,20 +602,25 @@ extern "C" int mi_moe_expert_gemm(void* out, const void* a_rows, const void* wei
       // tokens 154 | 123, 253 193 | 152; 1024 x 384, 128 experts, 512 tokens 26.9 | 22.8, but 1 token 6.9 | 7.7 and 4096 x 1536 20.7 | 21.7.  Up,
       // 64-row tiles: 1536 x 4096, 200 tokens 172 | 143, gated 400 tokens 330 | 289, 384 x 1024 gated 44.2 | 39.8.  32-row tiles of the up
       // forms stay with the ring: gated 5 tokens 131 | 131, 32 tokens 255 | 270, 253 tokens 316 | 314, 384 x 1024 36.4 | 37.3; the
-      // squared relu's alone would gain once most experts are chosen (64 tokens 183 | 151, 1 token 34 | 40).
+      // squared relu's alone would gain once most experts are chosen (64 tokens 183 | 151, 1 token 34 | 40): below, for K of whole 2048s.
       // One round of tiles or less can be behind (the bound on them counts up to 1.75 times as many as there are).  140 sizes, 28 to 50 rows an
       // expert in 64-row tiles, the ring's time as 1: under 512 tiles down 0.77 to 1.22 (1152 x 1024, 8 experts 12.3 | 15.0 us), up 0.81 to 1.40 (448
       // x 768 gated, 64 experts 21.6 | 30.3, 512 x 2048 gated, 8 experts 19.6 | 25.7); past them 0.70 to 0.96 and 0.80 to 0.94, but for up
-      // products of K 2048, weight rows 4 KB apart (1024 x 2048 gated, 64 experts 111 | 121), and a last tile that is half empty (level).  70
+      // products with a last tile that is half empty (level).  70
       // sizes, 1 to 22 rows an expert in 32-row tiles, down: under 192 tiles to 1.19, past them 0.61 to 1.08 (2048 x 1536, 32 experts
       // 35 | 31), half-empty last tiles to 1.21 (384 x 256, 128 experts 9.5 | 11.5).
       const int32_t cols = gated ? 128 : 256;
       const int64_t width = (int64_t)max_tiles * n_out / cols;
       const bool always = e && strcmp(e, "always") == 0;
       const bool fit = tiles_fit(n_out, cols);
+      // With the blocks of K turned (k % 2048 == 0) up forms gain on the stream in 32-row tiles as well, us, ring | stream, both turned: 4096 x 1536, 64
+      // experts, squared relu, 64 tokens, 8 chosen 138 | 126, 120 tokens 146 | 127, gated, 6 chosen, 8 tokens 137 | 130, 32 tokens 253 | 243, 253 tokens 300 | 282;
+      // 2048 x 1024 gated, 30 tokens 88 | 83.  Under 512 tiles 16 tokens 120 | 123, 2048 x 768 gated, 32 tokens 63.9 | 65.4, 4 tokens 23.3 | 25.0 (but squared
+      // relu, 40 tokens 40.8 | 34.6).  64-row tiles: 2048 x 768, 200 tokens (264 tiles) 44.5 | 35.7, gated, 400 tokens 82 | 71.5, 2048 x 1024 gated, 300 tokens 97 | 89.5.
+      const bool turned = k % 2048 == 0, plain = form == MI_MOE_PLAIN;
       const bool stream = always ? rows_per_tile <= 64
-                          : rows_per_tile == 64 ? width >= 512 && (form == MI_MOE_PLAIN || (k != 2048 && fit))
-                                                : rows_per_tile == 32 && form == MI_MOE_PLAIN && width >= 192 && fit;
+                          : rows_per_tile == 64 ? (plain ? width >= 512 : fit && width >= (turned ? 256 : 512))
+                                                : rows_per_tile == 32 && fit && (plain ? width >= 192 : turned && width >= 512);
       const bool tall = rows_per_tile > 64 && (always || tall_fills(max_tiles, n_out, gated));
       int rc = tall ? launch_grouped_tall(ga, s) : stream ? launch_grouped_stream(ga, s) : MI_ERR_UNSUPPORTED;
       if (rc == MI_ERR_UNSUPPORTED) rc = launch_grouped_skinny(ga, s);

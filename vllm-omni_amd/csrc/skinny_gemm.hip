@@ -257,15 +257,17 @@ __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_
         src[i] = reinterpret_cast<const char*>(p.w + (int64_t)n * p.K + 64 * (int64_t)b_lo + 8 * lc);
       }
     }
+    const int first = p.turn ? (int)((uint32_t)wg % (uint32_t)max(n_it, 1)) : 0;
     auto issue = [&](int it, int stage) {
       char* st = smem + stage * C::kStage;
+      const int kk = it + first - (it + first < n_it ? 0 : n_it);
 #pragma unroll
       for (int i = 0; i < C::PPL; ++i) {
         if (l + kV2Loaders * i < C::XI)
-          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)it),
+          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk),
                                            (lds_void*)(st + (l + kV2Loaders * i) * 1024), 16, 0, 0);
         else
-          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)it),
+          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk),
                                            (lds_void*)(st + (l + kV2Loaders * i) * 1024), 16, 0, MI_SKINNY_W_AUX);
       }
     };
@@ -445,6 +447,17 @@ SkinnyPlan skinny_plan(int m, int n, int k, int force_split) {
 namespace mi {
 namespace {
 
+// Whether the weight tiles' k blocks are turned (SkinnyParams::turn).  Workgroups keep step with each other, and with weight rows a multiple of 8192
+// bytes apart all of them then read from the same few channels at a time; begun one block behind its neighbour, each reads elsewhere.  Slices of K
+// do that by themselves unless they begin a multiple of 4096 bytes apart.  As they are | turned, us, cold weights: 33056 x 4096, 1 row 56.2 | 43.0, 64 rows
+// 58.6 | 47.8, 128 rows 63.2 | 55.3, 200 rows 81.2 | 78.3; gated 24576 x 4096, 32 rows 46.8 | 40.5; 15360 x 4096 in two slices, 32 rows 32.9 | 28.6; 4096 x
+// 16384 in eight, 1 row 44.2 | 29.5; experts' 2048 x 768 (rows 4096 bytes apart), 200 tokens, 8 of 64 50.1 | 43.3, 4096 x 1536, 64 tokens 180 | 147.  Not past
+// the line: 6144 x 4096 in five slices, 128 rows 22.4 | 23.6, 15360 x 4096, 200 rows 45.0 | 46.2, 37888 x 3584 45.4 | 45.7; 12288 x 2048 and 2048 x 6144 level.
+// Two blocks apart: 4096 x 16384 38.0, gated 33056 x 4096 46.5.
+int skinny_turn(int k, int split, int mt) {
+  return k % 4096 == 0 && (split == 1 || (mt <= 8 && k % (2048 * split) == 0));
+}
+
 int linear_v2() {   // MI_LINEAR_V2=0: the first-generation kernel at 129-256 rows too (A/B runs; read per call)
   const char* e = getenv("MI_LINEAR_V2");
   return e ? atoi(e) : 1;
@@ -466,6 +479,7 @@ int launch_v2(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
 int launch_skinny(const SkinnyParams& p_in, const SkinnyPlan& pl, bool gated, int dtype, hipStream_t s, bool int8 = false) {
   SkinnyParams p = p_in;
   p.RB = (p.M + 16 * pl.mt - 1) / (16 * pl.mt);
+  p.turn = skinny_turn(p.K, pl.split, pl.mt);
   p.U = pl.tiles * pl.split;
   if (dtype != MI_DTYPE_BF16 && dtype != MI_DTYPE_F16) return MI_ERR_UNSUPPORTED;
   if (pl.mt == 16 && pl.nslab >= 4 && linear_v2()) {
@@ -1040,6 +1054,7 @@ int launch_grouped_skinny(const GroupedGemmArgs& a, hipStream_t s) {
   p.relu_squared = a.form == MI_MOE_RELU_SQUARED;
   p.pair_weights = a.pair_weights;
   p.w_expert_stride = a.weight_expert_stride;
+  p.turn = grouped_turn(a.k);
   p.dbg = 0;
   p.ldx = a.a_row_stride;
   p.ldo = a.out_row_stride;

@@ -28,4 +28,12 @@ int launch_grouped_stream(const GroupedGemmArgs& a, hipStream_t s);
 // Tiles of 128 or 256 rows (tall_gemm.hip); MI_ERR_UNSUPPORTED outside its envelope.
 int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s);
 
+// Experts' weight rows a multiple of 4096 bytes apart: the k blocks of 256 weight rows (128 columns of a gated form) begin with that of their number
+// among all experts' and go round.  One rule for every kernel of the grouped products: their sums keep one order.
+inline bool grouped_turn(int64_t k) { return k % 2048 == 0; }
+__device__ __forceinline__ int grouped_first_block(bool gated, int expert, int col, int n_out, int n_it) {
+  const int unit = gated ? 128 : 256;
+  return (int)((uint32_t)(expert * ((n_out + unit - 1) / unit) + col / unit) % (uint32_t)n_it);
+}
+
 }  // namespace mi

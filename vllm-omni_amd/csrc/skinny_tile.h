@@ -3,6 +3,7 @@
 // (cp_stack.hip) both run it.
 #pragma once
 #include "mfma_attn_common.h"
+#include "skinny_grouped.h"
 
 // experiment switches (csrc/Makefile `make variant VARIANT_DEFS=...`); the defaults are the measured best
 #ifndef MI_SKINNY_W_AUX
@@ -73,6 +74,7 @@ struct SkinnyParams {
   int64_t w_expert_stride;     // elements
   int32_t dbg;            // MI_LINEAR_DBG (timing experiments only): 1 = no DMA, 2 = no fragment reads / MFMAs, 4 = no reduce launch, 8 = no output stores
   int64_t ldx, ldo;
+  int32_t turn = 0;      // 1: a weight tile's k blocks begin with that of the tile's number and go round (skinny_turn); GROUPED: grouped_first_block
 };
 
 // operands as plain vectors (a HIP `uint4` is a struct: its copies between address spaces become memcpys that keep
@@ -219,7 +221,7 @@ __device__ __forceinline__ void skinny_tile(const SkinnyParams& p, const int wg_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint16_t* wbase = p.w;
-  int m0 = 0, wg = wg_linear, row_tile = 0;
+  int m0 = 0, wg = wg_linear, row_tile = 0, expert = 0;
   if constexpr (GROUPED) {
     // the maps were written by the alignment kernel just before this launch: keep their reads off a stale scalar cache
     scalar_cache_acquire();
@@ -235,7 +237,8 @@ __device__ __forceinline__ void skinny_tile(const SkinnyParams& p, const int wg_
       row_tile = blockIdx.y;
       if (row_tile >= p.num_tiles[0]) return;        // whole workgroup, before any barrier
     }
-    wbase += (int64_t)p.tile_expert[row_tile] * p.w_expert_stride;
+    expert = p.tile_expert[row_tile];
+    wbase += (int64_t)expert * p.w_expert_stride;
   } else {
     // More rows than one image holds (16 MT): RB row blocks per (tile, slice).  Workgroup ids go round-robin over the 8
     // XCDs, so the row blocks of one work item are dealt 8 ids apart: id = 8 RB q + 8 rb + j <-> item u = 8 q + j, row
@@ -295,22 +298,32 @@ __device__ __forceinline__ void skinny_tile(const SkinnyParams& p, const int wg_
     // step `it` of the workgroup = k block it % n_it of its tile it / n_it: the x pieces start over with every tile, the
     // weight pieces move on by one tile's rows (a chained launch has whole tiles only: the host checks)
     const int64_t w_tile_bytes = (int64_t)(GATED ? 16 * NSLAB : TR) * p.K * 2;
-    int kk_next = 0;                 // k block of the next step to issue
+    int kk_first = 0, tile_next = tile0;
+    const auto take = [&]() {
+      if (!p.turn || n_it == 0) return;
+      if constexpr (GROUPED) kk_first = grouped_first_block(GATED, expert, tile_next * (GATED ? 16 * NSLAB : TR), p.N, n_it);
+      else kk_first = wg % n_it;
+    };
+    take();
+    int kk_next = 0;                 // k block of the next step to issue, counted from kk_first
     int64_t w_next = 0;              // byte offset of its tile's weight rows
     auto issue = [&](int stage) {
       char* st = smem + stage * kStage;
+      const int kk = kk_next + kk_first - (kk_next + kk_first < n_it ? 0 : n_it);
 #pragma unroll
       for (int i = 0; i < PPL; ++i) {
         if (l + NL * i < XI)
-          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk_next),
+          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk),
                                            (lds_void*)(st + (l + NL * i) * 1024), 16, 0, COH ? kAuxAgent : 0);
         else
-          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk_next + w_next),
+          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk + w_next),
                                            (lds_void*)(st + (l + NL * i) * 1024), 16, 0, MI_SKINNY_W_AUX);
       }
       if (++kk_next == n_it) {
         kk_next = 0;
         w_next += w_tile_bytes;
+        ++tile_next;
+        if constexpr (GROUPED) take();
       }
     };
     const int total = n_it * chain;

@@ -39,6 +39,7 @@ struct TallParams {
   int64_t ldx, ldo, w_expert_stride;
   // DENSE: one weight matrix, all M rows.  The first `whole` tiles are items of their own; each of the others is cut along K into
   // `split` items that leave fp32 sums in part [item][256][256]
+  int32_t turn;      // experts: a tile's k blocks begin with grouped_first_block and go round
   int32_t M, whole, split, group;
   const uint16_t* bias;
   float* part;
@@ -56,6 +57,7 @@ constexpr int kTallStage = 64 * 1024;
 struct TallItem {
   int row0, tile, expert, units;     // units: 64-row units of the row tile that hold live rows
   int kb, n_it;                      // where the item starts along K (bytes) and its 64-wide blocks: an even number
+  int first;                         // the block that it begins with (then round)
   int slab;                          // >= 0: fp32 sums into this slab
   int row[8];
 };
@@ -80,6 +82,7 @@ __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo
   t.kb = 0;
   t.n_it = p.K >> 6;
   t.slab = -1;
+  t.first = 0;
   if constexpr (tall_dense(FORM)) {
     int at = lo + item;
     if (item >= whole) {
@@ -102,6 +105,7 @@ __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo
   t.tile = item - row_tile * p.nx;
   t.row0 = row_tile * p.rpt;
   t.expert = p.tile_expert[row_tile];
+  if (p.turn) t.first = grouped_first_block(tall_gated(FORM), t.expert, t.tile * (tall_gated(FORM) ? kTallN / 2 : kTallN), p.N, t.n_it);
   t.units = 0;
 #pragma unroll
   for (int u = 0; u < 4; ++u)
@@ -112,6 +116,14 @@ __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo
     const int r = t.row0 + (row < p.rpt ? row : 0);
     t.row[i] = p.gather_div > 0 ? p.row_map[r] : r;
   }
+}
+
+// where block i of an item lies along K (bytes)
+template <int FORM>
+__device__ __forceinline__ int tall_block(const TallItem& t, int i) {
+  if constexpr (tall_dense(FORM)) return t.kb + i * 128;
+  const int at = i + t.first;
+  return (at < t.n_it ? at : at - t.n_it) * 128;
 }
 
 // byte offsets of a lane's 8 x pieces
@@ -226,7 +238,7 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     __builtin_amdgcn_s_waitcnt(kLgkm0);
     barrier();                                   // everybody has read this stage
     // (loads spread over the step: a wave that finds the memory pipe's queue full issues no product either)
-    const int kb = KIND == 0 ? t.kb + (it + 2) * 128 : nt.kb + (KIND - 1) * 128;
+    const int kb = KIND == 0 ? tall_block<FORM>(t, it + 2) : tall_block<FORM>(nt, KIND - 1);
     if (KIND == 0 || more) tall_issue_w(wo, wr, kb, cur);
     if (KIND == 2) {
       if (more) tall_issue_x<8>(p, x, kb, cur);
@@ -381,10 +393,10 @@ __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
   tall_rows<FORM>(p, t, x);
   {
     const __amdgpu_buffer_rsrc_t wr = tall_weights<GATED>(p, t);
-    tall_issue_w(wo, wr, t.kb, s0);
-    tall_issue_x<8>(p, x, t.kb, s0);
-    tall_issue_w(wo, wr, t.kb + 128, s1);
-    tall_issue_x<8>(p, x, t.kb + 128, s1);
+    tall_issue_w(wo, wr, tall_block<FORM>(t, 0), s0);
+    tall_issue_x<8>(p, x, tall_block<FORM>(t, 0), s0);
+    tall_issue_w(wo, wr, tall_block<FORM>(t, 1), s1);
+    tall_issue_x<8>(p, x, tall_block<FORM>(t, 1), s1);
   }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   while (true) {
@@ -462,6 +474,7 @@ int launch_grouped_tall(const GroupedGemmArgs& a, hipStream_t s) {
   p.ldx = a.a_row_stride;
   p.ldo = a.out_row_stride;
   p.w_expert_stride = a.weight_expert_stride;
+  p.turn = grouped_turn(a.k);
   const int cols = gated ? kTallN / 2 : kTallN;
   p.nx = (a.n_out + cols - 1) / cols;
   const int64_t work = (int64_t)p.nx * a.max_tiles;
