@@ -20,7 +20,7 @@ def _case(s, nq, nkv, hd, bound, dev, seed=0):
 # launches of more than 256 workgroups: lone waves, two partitions, partitions that merge in their workgroup, a last round that is not full,
 # more rounds than are resident, up to 1024 sequences
 @pytest.mark.parametrize("s,nq,nkv,hd,bound", [(65, 28, 4, 128, 700), (120, 28, 4, 128, 700), (70, 28, 4, 128, 1000), (161, 32, 8, 128, 300), (257, 14, 2, 128, 320),
-                                               (200, 32, 8, 128, 512), (300, 16, 2, 64, 600), (1024, 8, 1, 64, 520), (33, 40, 10, 128, 400)])
+                                               (200, 32, 8, 128, 512), (300, 14, 2, 128, 600), (1024, 8, 1, 128, 520), (33, 40, 10, 128, 400)])
 def test_order(s, nq, nkv, hd, bound):
     from vllm_omni_amd import ops
 
@@ -59,6 +59,7 @@ def test_sizes_that_are_not_ordered():
     lens = lambda n: torch.full((n,), 100, dtype=torch.int32, device=dev)  # noqa: E731
     assert ops.decode_seq_order(lens(64), 28, 4, 128, 16, 2048) is None       # a workgroup a CU
     assert ops.decode_seq_order(lens(256), 28, 4, 128, 16, 256) is None       # short bounds
+    assert ops.decode_seq_order(lens(512), 16, 2, 64, 16, 4096) is None
     assert ops.decode_seq_order(lens(1025), 8, 1, 128, 16, 2048) is None
     assert ops.decode_seq_order(lens(1), 28, 4, 128, 16, 2048) is None
     with pytest.raises(ValueError):

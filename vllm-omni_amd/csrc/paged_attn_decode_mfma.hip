@@ -810,46 +810,49 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
   }
 }
 
-// Places of the sequences, longest first: how many are longer than each (or as long, in front of it), counted by as many of the 1024 threads as
-// there are for a sequence.  Lengths within a sixteenth of each other stay as they are.  Once a step; 120 sequences 3.0 us, 256 5.0, 512 13.
-constexpr int kOrderSeqs = 1024;
+// Places of the sequences, longest first: how many are longer than each (or as long, in front of it).  A workgroup has 128 sequences, eight threads
+// for each.  Lengths within a sixteenth of each other stay as they are.  Once a step; 120 sequences 3.4 us, 256 4.1, 512 5.6, 1024 8.4.
+constexpr int kOrderSeqs = 1024, kOrderEach = 128;
 __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __restrict__ out, const int32_t* __restrict__ seq_lens, int num_seqs,
                                                                   const DecodeOrder o) {
   scalar_cache_acquire();
   __shared__ __attribute__((aligned(16))) int32_t lens[kOrderSeqs];
-  __shared__ int32_t ranks[kOrderSeqs];
+  __shared__ int32_t ranks[kOrderEach];
   __shared__ int32_t least, most;
   const int t = threadIdx.x;
   if (t == 0) least = 0x7fffffff, most = 0;
+  if (t < kOrderEach) ranks[t] = 0;
   lens[t] = t < num_seqs ? seq_lens[t] : -1;      // (no sequence: behind the empty ones)
-  ranks[t] = 0;
   __syncthreads();
-  const int each = (num_seqs + 63) / 64 * 64, parts = kOrderSeqs / each, quads = (num_seqs + 3) / 4;
-  const int i = t % each, part = t / each, len = lens[i];
-  if (part < parts) {
-    int rank = 0;
+  int lo = t < num_seqs ? lens[t] : 0x7fffffff, hi = max(lens[t], 0);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    lo = min(lo, __shfl_xor(lo, d, 64));
+    hi = max(hi, __shfl_xor(hi, d, 64));
+  }
+  if ((t & 63) == 0) {
+    atomicMin(&least, lo);
+    atomicMax(&most, hi);
+  }
+  constexpr int parts = kOrderSeqs / kOrderEach;
+  const int quads = (num_seqs + 3) / 4, part = t / kOrderEach;
+  const int i = min(kOrderEach * (int)blockIdx.x + t % kOrderEach, kOrderSeqs - 1), len = lens[i];
+  int rank = 0;
 #pragma unroll 4
-    for (int j = 4 * (part * quads / parts); j < 4 * ((part + 1) * quads / parts); j += 4) {
-      const int4 l = *reinterpret_cast<const int4*>(lens + j);
-      rank += (l.x > len || (l.x == len && j < i)) + (l.y > len || (l.y == len && j + 1 < i)) + (l.z > len || (l.z == len && j + 2 < i)) +
-              (l.w > len || (l.w == len && j + 3 < i));
-    }
-    atomicAdd(&ranks[i], rank);
+  for (int j = 4 * (part * quads / parts); j < 4 * ((part + 1) * quads / parts); j += 4) {
+    const int4 l = *reinterpret_cast<const int4*>(lens + j);
+    rank += (l.x > len || (l.x == len && j < i)) + (l.y > len || (l.y == len && j + 1 < i)) + (l.z > len || (l.z == len && j + 2 < i)) +
+            (l.w > len || (l.w == len && j + 3 < i));
   }
-  if (t < num_seqs) {
-    atomicMin(&least, lens[t]);
-    atomicMax(&most, lens[t]);
-  }
+  atomicAdd(&ranks[t % kOrderEach], rank);
   __syncthreads();
-  if (t >= num_seqs) return;
-  out[t] = lens[t];
-  if (most - least <= most / 16) {      // nothing to even out
-    out[num_seqs + t] = t;
-    return;
-  }
-  const int rank = ranks[t], round = rank / o.per, first = round * o.per;
-  const int place = round < o.turned && (round & 1) ? first + min(o.per, num_seqs - first) - 1 - (rank - first) : rank;
-  out[num_seqs + place] = t;
+  if (t >= kOrderEach || i >= num_seqs) return;
+  out[i] = len;
+  rank = ranks[t];
+  const int round = rank / o.per, first = round * o.per;
+  const int place = most - least <= most / 16 ? i      // nothing to even out
+                    : round < o.turned && (round & 1) ? first + min(o.per, num_seqs - first) - 1 - (rank - first) : rank;
+  out[num_seqs + place] = i;
 }
 
 // one wave a workgroup, or (group) the partitions of a sequence's head group as the waves of one
@@ -912,19 +915,20 @@ int32_t decode_mfma_turn(int64_t groups, int num_parts) {
 // Contexts of uneven length: a launch of more workgroups than CUs lasts as long as the CU with the largest sum, or as its last arrivals.  Longest
 // first the late ones are short, and with every other round of 256 turned the sums of the rounds that are resident together even out.
 // Not where a CU has one workgroup at most, and partitions of three or more gain nothing (23 x 4 KV heads in 6, 425 to 1700 tokens 15.2 | 16.0 us).
-// Equal lengths cost nothing (256 x 4, 4096 tokens 322 | 322, 300 tokens 29.5 | 29.5; 512 x 2 of 64 dims, 4096 166.0 | 166.5).  As they are | ordered, us:
+// Equal lengths cost nothing (256 x 4, 4096 tokens 322 | 322, 300 tokens 29.5 | 29.5).  As they are | ordered, us:
 // 120 x 4 in 2, 175 to 700 tokens 27.8 | 22.9; 70 x 4 in 2, 100 to 3000 67 | 58; 256 x 4, 1000 to 4096 246 | 231, 75 to 300 23.1 | 22.3; 161 x 8, 300 to
-// 1500 121 | 98; 200 x 8, 750 to 3001 276 | 242; 300 x 8, 500 to 2000 263 | 242; 64 dims: 512 x 2, 1000 to 4096 127 | 121; 300 x 2 in 2, 500 to 2000
-// 46.1 | 38.5.  Longest first alone, no round turned: 120 x 4 25.2, 300 x 2 40.2.  Bounds of up to 256 tokens of 128 dims: not tried, a launch takes 7 to 11 us.
+// 1500 121 | 98; 200 x 8, 750 to 3001 276 | 242; 300 x 8, 500 to 2000 263 | 242.  Longest first alone, no round turned: 120 x 4 25.2.  Heads of 64 dims
+// gain with uneven contexts (512 x 2, 1000 to 4096 127 | 121), but their waves, all resident at once, feel the look-up in front of their loads: a
+// step of 512 equal contexts 6474 | 6515.  Bounds of up to 256 tokens: not tried, a launch takes 7 to 11 us.
 DecodeOrder decode_mfma_order(int num_seqs, int groups_per_seq, int num_parts, bool group_parts, int head_dim, int max_seq_len) {
-  const int ring = head_dim == 128 ? ring_bytes<128> : ring_bytes<64>, waves = group_parts ? num_parts : 1;
+  const int ring = ring_bytes<128>, waves = group_parts ? num_parts : 1;
   const int64_t each = (int64_t)groups_per_seq * (num_parts / waves);      // workgroups of a sequence
-  if (num_seqs < 2 || num_seqs > kOrderSeqs || each * num_seqs <= kCUs || (!group_parts && num_parts > 2) || (int64_t)max_seq_len * head_dim <= 256 * 128)
+  if (head_dim != 128 || max_seq_len <= 256 || num_seqs < 2 || num_seqs > kOrderSeqs || each * num_seqs <= kCUs || (!group_parts && num_parts > 2))
     return {0, 0};
   return {each < kCUs ? (int32_t)(kCUs / each) : 1, kLdsBytes / (ring * waves)};
 }
 int launch_decode_order(int32_t* out, const int32_t* seq_lens, int num_seqs, DecodeOrder order, hipStream_t stream) {
-  hipLaunchKernelGGL(decode_order_kernel, dim3(1), dim3(kOrderSeqs), 0, stream, out, seq_lens, num_seqs, order);
+  hipLaunchKernelGGL(decode_order_kernel, dim3((num_seqs + kOrderEach - 1) / kOrderEach), dim3(kOrderSeqs), 0, stream, out, seq_lens, num_seqs, order);
   return launch_status();
 }
 
