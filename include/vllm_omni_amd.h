@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define MI_ABI_VERSION 6
+#define MI_ABI_VERSION 7
 
 /* dtype enum shared by every entry point */
 enum {
@@ -228,16 +228,15 @@ int mi_rope_cache_attend_block_splitk(void* out, const void* partials, int32_t s
  * context is left out — `out` is then NOT written, unless the partitions merge inside the attention launch (few of
  * them, as the waves of one workgroup).  Never set by the product. */
 #define MI_DECODE_SKIP_MERGE 32
-/* MI_DECODE_SEQ_ORDER: seq_lens is what mi_decode_seq_order wrote for this call's sequences and sizes: their lengths, then the order that the
- * launch takes them in (matrix-core kernel; the others run them as they are).  Speed only: outputs keep their bits. */
-#define MI_DECODE_SEQ_ORDER 64
 #define MI_DECODE_COUNTER_BYTES (1 << 20)
 int64_t mi_paged_attn_decode_workspace_bytes(int32_t num_seqs, int32_t num_q_heads,
                                              int32_t head_dim, int32_t max_seq_len,
                                              int32_t partition_size);
 /* lens_and_order [2 * num_seqs]: a copy of seq_lens, then the order in which a decode launch of these sizes (and flags) should take the
- * sequences: for calls with MI_DECODE_SEQ_ORDER of one step, whose lengths are the same in every layer.  MI_ERR_UNSUPPORTED: such a launch
- * gains nothing from an order (nothing is written). */
+ * sequences: the seq_order of the _ordered calls of one step, whose lengths are the same in every layer.  MI_ERR_UNSUPPORTED: such a launch
+ * gains nothing from an order (nothing is written).
+ * seq_order [num_seqs] of an _ordered call: every number below num_seqs once, or NULL.  Speed only (matrix-core kernel; the others run the
+ * sequences as they are): the lengths are those of seq_lens whatever the order was made of, and outputs keep their bits. */
 int mi_decode_seq_order(int32_t* lens_and_order, const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
                         int32_t head_dim, int32_t block_size, int32_t max_seq_len, int32_t partition_size, int32_t flags, void* stream);
 int mi_paged_attn_decode(void* out, const void* q, const void* k_cache, const void* v_cache,
@@ -249,6 +248,15 @@ int mi_paged_attn_decode(void* out, const void* q, const void* k_cache, const vo
                          int64_t cache_token_stride, int64_t cache_head_stride,
                          int32_t partition_size, void* workspace, int64_t workspace_bytes,
                          int dtype, int out_dtype, int32_t flags, void* stream);
+int mi_paged_attn_decode_ordered(void* out, const void* q, const void* k_cache, const void* v_cache,
+                                 const int32_t* block_table, const int32_t* seq_lens,
+                                 int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                 int32_t head_dim, int32_t block_size, int32_t block_table_stride,
+                                 int32_t max_seq_len, float scale, int64_t q_token_stride,
+                                 int64_t out_token_stride, int64_t cache_block_stride,
+                                 int64_t cache_token_stride, int64_t cache_head_stride,
+                                 int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                 int dtype, int out_dtype, int32_t flags, const int32_t* seq_order, void* stream);
 /* A4 + A7 + A5 in ONE launch for a pure-decode step (round 4): q [S, nq*d], k / v [S, nkv*d] arrive as qkv_proj wrote
  * them (views of one qkv row are fine); every wave rotates its q heads in registers (neox, fp32 table row of
  * positions[s], one rounding — mi_rope_neox_and_cache's arithmetic), and the wave that owns a sequence's last context
@@ -273,6 +281,19 @@ int mi_rope_cache_paged_attn_decode(void* out, const void* q, const void* k, con
                                     int64_t cache_token_stride, int64_t cache_head_stride,
                                     int32_t partition_size, void* workspace, int64_t workspace_bytes,
                                     int dtype, int out_dtype, int32_t flags, void* stream);
+int mi_rope_cache_paged_attn_decode_ordered(void* out, const void* q, const void* k, const void* v,
+                                            const int64_t* positions, const float* cos_sin_cache,
+                                            int32_t max_position, int32_t rot_dim, const void* q_norm_weight,
+                                            const void* k_norm_weight, float norm_eps, void* k_cache, void* v_cache,
+                                            const int64_t* slot_mapping, const int32_t* block_table,
+                                            const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads,
+                                            int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                            int32_t block_table_stride, int32_t max_seq_len, float scale,
+                                            int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride,
+                                            int64_t out_token_stride, int64_t cache_block_stride,
+                                            int64_t cache_token_stride, int64_t cache_head_stride,
+                                            int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                            int dtype, int out_dtype, int32_t flags, const int32_t* seq_order, void* stream);
 
 /* The same launch fed by the fp32 split-K partials [split][num_seqs][(num_q_heads + 2 num_kv_heads) * head_dim] of qkv_proj
  * (mi_linear_partials) and its bias (may be NULL) instead of 16-bit q / k / v rows: bit-identical to mi_linear in front of it. */
@@ -285,6 +306,15 @@ int mi_rope_cache_paged_attn_decode_splitk(void* out, const void* partials, int3
                                            float scale, int64_t out_token_stride, int64_t cache_block_stride, int64_t cache_token_stride,
                                            int64_t cache_head_stride, int32_t partition_size, void* workspace, int64_t workspace_bytes,
                                            int dtype, int out_dtype, int32_t flags, void* stream);
+int mi_rope_cache_paged_attn_decode_splitk_ordered(void* out, const void* partials, int32_t split, const void* qkv_bias,
+                                                   const int64_t* positions, const float* cos_sin_cache, int32_t max_position, int32_t rot_dim,
+                                                   const void* q_norm_weight, const void* k_norm_weight, float norm_eps, void* k_cache,
+                                                   void* v_cache, const int64_t* slot_mapping, const int32_t* block_table,
+                                                   const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
+                                                   int32_t head_dim, int32_t block_size, int32_t block_table_stride, int32_t max_seq_len,
+                                                   float scale, int64_t out_token_stride, int64_t cache_block_stride, int64_t cache_token_stride,
+                                                   int64_t cache_head_stride, int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                                   int dtype, int out_dtype, int32_t flags, const int32_t* seq_order, void* stream);
 /* Partition size the auto heuristic picks: the fewest partitions that leave >= 512 waves (>= 1024 at
  * head_dim <= 64), each of at most 8192 tokens and at least 256, or, from three partitions on, an eighth of
  * max_seq_len and at least 64 (never more than max_seq_len rounded up to 32).  ONE partition (direct output,
@@ -936,7 +966,6 @@ int mi_paged_attn_decode_biased(void* out, const void* q, const void* k_cache, c
                                 int64_t cache_block_stride, int64_t cache_token_stride,
                                 int64_t cache_head_stride, int32_t partition_size, void* workspace,
                                 int64_t workspace_bytes, int dtype, void* stream);
-/* ... with flags: MI_DECODE_SEQ_ORDER or 0 */
 int mi_paged_attn_decode_biased_ordered(void* out, const void* q, const void* k_cache, const void* v_cache,
                                         const int32_t* block_table, const int32_t* seq_lens,
                                         const float* slopes, const float* sinks, float out_scale,
@@ -945,7 +974,7 @@ int mi_paged_attn_decode_biased_ordered(void* out, const void* q, const void* k_
                                         float scale, int64_t q_token_stride, int64_t out_token_stride,
                                         int64_t cache_block_stride, int64_t cache_token_stride,
                                         int64_t cache_head_stride, int32_t partition_size, void* workspace,
-                                        int64_t workspace_bytes, int dtype, int32_t flags, void* stream);
+                                        int64_t workspace_bytes, int dtype, const int32_t* seq_order, void* stream);
 int mi_paged_attn_prefill_biased(void* out, const void* q, const void* k_cache, const void* v_cache,
                                  const int32_t* block_table, const int32_t* seq_lens,
                                  const int32_t* query_start_loc, const float* slopes,

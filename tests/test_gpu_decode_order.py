@@ -97,3 +97,19 @@ def test_lengths_close_to_each_other_stay(lens, kept):
 
     order = ops.decode_seq_order(torch.tensor(lens, dtype=torch.int32, device="cuda"), 28, 4, 128, 16, 700)
     assert torch.equal(order[1].cpu(), torch.arange(120, dtype=torch.int32)) == kept
+
+
+# an order is a matter of speed: one made of other lengths gives the bits of the call's own
+@pytest.mark.parametrize("biased", [False, True])
+def test_an_order_of_other_lengths(biased):
+    from vllm_omni_amd import ops
+
+    dev = torch.device("cuda", 0)
+    s, nq, nkv, hd, bound = 120, 28, 4, 128, 700
+    q, kc, vc, bt, lens = _case(s, nq, nkv, hd, bound, dev)
+    kw = {"slopes": torch.rand(nq, device=dev), "sinks": torch.randn(nq, device=dev)} if biased else {}
+    order = ops.decode_seq_order(lens, nq, nkv, hd, 16, bound)
+    lens = torch.randint(0, bound + 1, (s,), dtype=torch.int32, generator=torch.Generator().manual_seed(9)).to(dev)
+    want = ops.paged_attn_decode(torch.empty_like(q), q, kc, vc, bt, lens, bound, hd ** -0.5, **kw)
+    got = ops.paged_attn_decode(torch.empty_like(q), q, kc, vc, bt, lens, bound, hd ** -0.5, order=order, **kw)
+    assert torch.equal(want.view(torch.int16), got.view(torch.int16))

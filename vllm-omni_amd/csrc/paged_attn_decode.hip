@@ -585,7 +585,7 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
                 int32_t block_size, int32_t block_table_stride, int32_t max_seq_len, float scale, int64_t q_token_stride,
                 int64_t out_token_stride, int64_t cache_block_stride, int64_t cache_token_stride,
                 int64_t cache_head_stride, int32_t partition_size, void* workspace, int64_t workspace_bytes, int dtype,
-                int out_dtype, int32_t flags, void* stream, const RopeFusion* rope, const float* slopes = nullptr,
+                int out_dtype, int32_t flags, void* stream, const int32_t* seq_order, const RopeFusion* rope, const float* slopes = nullptr,
                 const float* sinks = nullptr, float out_scale = 1.f) {
   using namespace mi;
   if (num_seqs == 0) return MI_OK;
@@ -639,7 +639,7 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
   p.group_parts = use_mfma && decode_mfma_groups((int64_t)num_seqs * (num_q_heads / G), num_parts, head_dim, max_seq_len);
   if (p.group_parts) p.part_count = nullptr;
   p.turn = decode_mfma_turn((int64_t)num_seqs * (num_q_heads / G), num_parts);
-  if (use_mfma && (flags & MI_DECODE_SEQ_ORDER)) p.seq_order = seq_lens + num_seqs;
+  if (use_mfma) p.seq_order = seq_order;
   p.num_seqs = num_seqs;
   p.num_q_heads = num_q_heads;
   p.kv_group = kv_group;
@@ -699,6 +699,23 @@ int decode_call(void* out, const void* q, const void* k_cache, const void* v_cac
 }
 }  // namespace
 
+extern "C" int mi_paged_attn_decode_ordered(void* out, const void* q, const void* k_cache,
+                                            const void* v_cache, const int32_t* block_table,
+                                            const int32_t* seq_lens, int32_t num_seqs,
+                                            int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                            int32_t block_size, int32_t block_table_stride,
+                                            int32_t max_seq_len, float scale, int64_t q_token_stride,
+                                            int64_t out_token_stride, int64_t cache_block_stride,
+                                            int64_t cache_token_stride, int64_t cache_head_stride,
+                                            int32_t partition_size, void* workspace,
+                                            int64_t workspace_bytes, int dtype, int out_dtype,
+                                            int32_t flags, const int32_t* seq_order, void* stream) {
+  return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                     block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
+                     cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
+                     workspace_bytes, dtype, out_dtype, flags, stream, seq_order, nullptr);
+}
+
 extern "C" int mi_paged_attn_decode(void* out, const void* q, const void* k_cache,
                                     const void* v_cache, const int32_t* block_table,
                                     const int32_t* seq_lens, int32_t num_seqs,
@@ -710,10 +727,10 @@ extern "C" int mi_paged_attn_decode(void* out, const void* q, const void* k_cach
                                     int32_t partition_size, void* workspace,
                                     int64_t workspace_bytes, int dtype, int out_dtype,
                                     int32_t flags, void* stream) {
-  return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                     block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
-                     cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
-                     workspace_bytes, dtype, out_dtype, flags, stream, nullptr);
+  return mi_paged_attn_decode_ordered(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                                      block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
+                                      cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace, workspace_bytes,
+                                      dtype, out_dtype, flags, nullptr, stream);
 }
 
 extern "C" int mi_decode_seq_order(int32_t* lens_and_order, const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
@@ -738,12 +755,13 @@ extern "C" int mi_paged_attn_decode_biased_ordered(void* out, const void* q, con
                                                    int32_t max_seq_len, float scale, int64_t q_token_stride,
                                                    int64_t out_token_stride, int64_t cache_block_stride,
                                                    int64_t cache_token_stride, int64_t cache_head_stride, int32_t partition_size,
-                                                   void* workspace, int64_t workspace_bytes, int dtype, int32_t flags, void* stream) {
+                                                   void* workspace, int64_t workspace_bytes, int dtype, const int32_t* seq_order,
+                                                   void* stream) {
   return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
                      block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
                      cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
-                     workspace_bytes, dtype, dtype, MI_DECODE_PACKED_PV | MI_DECODE_NONTEMPORAL | (flags & MI_DECODE_SEQ_ORDER), stream, nullptr, slopes,
-                     sinks, out_scale);
+                     workspace_bytes, dtype, dtype, MI_DECODE_PACKED_PV | MI_DECODE_NONTEMPORAL, stream, seq_order, nullptr, slopes, sinks,
+                     out_scale);
 }
 
 extern "C" int mi_paged_attn_decode_biased(void* out, const void* q, const void* k_cache, const void* v_cache,
@@ -757,7 +775,35 @@ extern "C" int mi_paged_attn_decode_biased(void* out, const void* q, const void*
   return mi_paged_attn_decode_biased_ordered(out, q, k_cache, v_cache, block_table, seq_lens, slopes, sinks, out_scale, num_seqs, num_q_heads,
                                              num_kv_heads, head_dim, block_size, block_table_stride, max_seq_len, scale, q_token_stride,
                                              out_token_stride, cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
-                                             workspace_bytes, dtype, 0, stream);
+                                             workspace_bytes, dtype, nullptr, stream);
+}
+
+extern "C" int mi_rope_cache_paged_attn_decode_ordered(void* out, const void* q, const void* k, const void* v,
+                                                       const int64_t* positions, const float* cos_sin_cache,
+                                                       int32_t max_position, int32_t rot_dim, const void* q_norm_weight,
+                                                       const void* k_norm_weight, float norm_eps, void* k_cache, void* v_cache,
+                                                       const int64_t* slot_mapping, const int32_t* block_table,
+                                                       const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads,
+                                                       int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                                       int32_t block_table_stride, int32_t max_seq_len, float scale,
+                                                       int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride,
+                                                       int64_t out_token_stride, int64_t cache_block_stride,
+                                                       int64_t cache_token_stride, int64_t cache_head_stride,
+                                                       int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                                       int dtype, int out_dtype, int32_t flags, const int32_t* seq_order, void* stream) {
+  if (num_seqs == 0) return MI_OK;
+  if (!k || !v || !positions || !cos_sin_cache || !slot_mapping || max_position <= 0) return MI_ERR_INVALID_ARG;
+  if (rot_dim != head_dim) return MI_ERR_UNSUPPORTED;   // partial rotary: use the two launches
+  if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return MI_ERR_INVALID_ARG;
+  if (((uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight) & 15) return MI_ERR_INVALID_ARG;
+  if (k_token_stride % 8 || v_token_stride % 8 || (((uintptr_t)k | (uintptr_t)v | (uintptr_t)cos_sin_cache) & 15))
+    return MI_ERR_INVALID_ARG;
+  const RopeFusion rf{k, v, positions, slot_mapping, cos_sin_cache, max_position, k_token_stride, v_token_stride,
+                      q_norm_weight, k_norm_weight, norm_eps, nullptr, 0, nullptr};
+  return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                     block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
+                     cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
+                     workspace_bytes, dtype, out_dtype, flags, stream, seq_order, &rf);
 }
 
 extern "C" int mi_rope_cache_paged_attn_decode(void* out, const void* q, const void* k, const void* v,
@@ -773,19 +819,38 @@ extern "C" int mi_rope_cache_paged_attn_decode(void* out, const void* q, const v
                                                int64_t cache_token_stride, int64_t cache_head_stride,
                                                int32_t partition_size, void* workspace, int64_t workspace_bytes,
                                                int dtype, int out_dtype, int32_t flags, void* stream) {
+  return mi_rope_cache_paged_attn_decode_ordered(out, q, k, v, positions, cos_sin_cache, max_position, rot_dim, q_norm_weight,
+                                                 k_norm_weight, norm_eps, k_cache, v_cache, slot_mapping, block_table, seq_lens, num_seqs,
+                                                 num_q_heads, num_kv_heads, head_dim, block_size, block_table_stride, max_seq_len, scale,
+                                                 q_token_stride, k_token_stride, v_token_stride, out_token_stride, cache_block_stride,
+                                                 cache_token_stride, cache_head_stride, partition_size, workspace, workspace_bytes, dtype,
+                                                 out_dtype, flags, nullptr, stream);
+}
+
+extern "C" int mi_rope_cache_paged_attn_decode_splitk_ordered(void* out, const void* partials, int32_t split, const void* qkv_bias,
+                                                              const int64_t* positions, const float* cos_sin_cache,
+                                                              int32_t max_position, int32_t rot_dim, const void* q_norm_weight,
+                                                              const void* k_norm_weight, float norm_eps, void* k_cache, void* v_cache,
+                                                              const int64_t* slot_mapping, const int32_t* block_table,
+                                                              const int32_t* seq_lens, int32_t num_seqs, int32_t num_q_heads,
+                                                              int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                                              int32_t block_table_stride, int32_t max_seq_len, float scale,
+                                                              int64_t out_token_stride, int64_t cache_block_stride,
+                                                              int64_t cache_token_stride, int64_t cache_head_stride,
+                                                              int32_t partition_size, void* workspace, int64_t workspace_bytes,
+                                                              int dtype, int out_dtype, int32_t flags, const int32_t* seq_order, void* stream) {
   if (num_seqs == 0) return MI_OK;
-  if (!k || !v || !positions || !cos_sin_cache || !slot_mapping || max_position <= 0) return MI_ERR_INVALID_ARG;
-  if (rot_dim != head_dim) return MI_ERR_UNSUPPORTED;   // partial rotary: use the two launches
+  if (!partials || !positions || !cos_sin_cache || !slot_mapping || max_position <= 0 || split < 1) return MI_ERR_INVALID_ARG;
+  if (rot_dim != head_dim) return MI_ERR_UNSUPPORTED;
   if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return MI_ERR_INVALID_ARG;
-  if (((uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight) & 15) return MI_ERR_INVALID_ARG;
-  if (k_token_stride % 8 || v_token_stride % 8 || (((uintptr_t)k | (uintptr_t)v | (uintptr_t)cos_sin_cache) & 15))
+  if (((uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight | (uintptr_t)partials | (uintptr_t)qkv_bias | (uintptr_t)cos_sin_cache) & 15)
     return MI_ERR_INVALID_ARG;
-  const RopeFusion rf{k, v, positions, slot_mapping, cos_sin_cache, max_position, k_token_stride, v_token_stride,
-                      q_norm_weight, k_norm_weight, norm_eps, nullptr, 0, nullptr};
-  return decode_call(out, q, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                     block_size, block_table_stride, max_seq_len, scale, q_token_stride, out_token_stride,
-                     cache_block_stride, cache_token_stride, cache_head_stride, partition_size, workspace,
-                     workspace_bytes, dtype, out_dtype, flags, stream, &rf);
+  const RopeFusion rf{nullptr, nullptr, positions, slot_mapping, cos_sin_cache, max_position, 0, 0, q_norm_weight, k_norm_weight,
+                      norm_eps, static_cast<const float*>(partials), split, qkv_bias};
+  return decode_call(out, partials, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                     block_size, block_table_stride, max_seq_len, scale, 0, out_token_stride, cache_block_stride,
+                     cache_token_stride, cache_head_stride, partition_size, workspace, workspace_bytes, dtype, out_dtype, flags,
+                     stream, seq_order, &rf);
 }
 
 extern "C" int mi_rope_cache_paged_attn_decode_splitk(void* out, const void* partials, int32_t split, const void* qkv_bias,
@@ -800,16 +865,10 @@ extern "C" int mi_rope_cache_paged_attn_decode_splitk(void* out, const void* par
                                                       int64_t cache_token_stride, int64_t cache_head_stride,
                                                       int32_t partition_size, void* workspace, int64_t workspace_bytes,
                                                       int dtype, int out_dtype, int32_t flags, void* stream) {
-  if (num_seqs == 0) return MI_OK;
-  if (!partials || !positions || !cos_sin_cache || !slot_mapping || max_position <= 0 || split < 1) return MI_ERR_INVALID_ARG;
-  if (rot_dim != head_dim) return MI_ERR_UNSUPPORTED;
-  if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return MI_ERR_INVALID_ARG;
-  if (((uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight | (uintptr_t)partials | (uintptr_t)qkv_bias | (uintptr_t)cos_sin_cache) & 15)
-    return MI_ERR_INVALID_ARG;
-  const RopeFusion rf{nullptr, nullptr, positions, slot_mapping, cos_sin_cache, max_position, 0, 0, q_norm_weight, k_norm_weight,
-                      norm_eps, static_cast<const float*>(partials), split, qkv_bias};
-  return decode_call(out, partials, k_cache, v_cache, block_table, seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                     block_size, block_table_stride, max_seq_len, scale, 0, out_token_stride, cache_block_stride,
-                     cache_token_stride, cache_head_stride, partition_size, workspace, workspace_bytes, dtype, out_dtype, flags,
-                     stream, &rf);
+  return mi_rope_cache_paged_attn_decode_splitk_ordered(out, partials, split, qkv_bias, positions, cos_sin_cache, max_position, rot_dim,
+                                                        q_norm_weight, k_norm_weight, norm_eps, k_cache, v_cache, slot_mapping, block_table,
+                                                        seq_lens, num_seqs, num_q_heads, num_kv_heads, head_dim, block_size,
+                                                        block_table_stride, max_seq_len, scale, out_token_stride, cache_block_stride,
+                                                        cache_token_stride, cache_head_stride, partition_size, workspace, workspace_bytes,
+                                                        dtype, out_dtype, flags, nullptr, stream);
 }

@@ -19,7 +19,7 @@ MI_DTYPE_F16, MI_DTYPE_BF16, MI_DTYPE_F32 = 0, 1, 2
 MI_OK = 0
 MI_ERR_INVALID_ARG, MI_ERR_UNSUPPORTED, MI_ERR_WORKSPACE = -1, -2, -3
 MI_ERR_LAUNCH, MI_ERR_EXHAUSTED, MI_ERR_STATE = -4, -5, -6
-ABI_VERSION = 6
+ABI_VERSION = 7
 MI_LINEAR_PLAN_FULL, MI_LINEAR_PLAN_PARTIALS, MI_LINEAR_PLAN_GATED = 0, 1, 2
 MI_LINEAR_COUNTER_BYTES = 16 << 10
 MI_DECODE_PACKED_PV = 1
@@ -28,7 +28,6 @@ MI_DECODE_NONTEMPORAL = 4
 MI_DECODE_ROUNDED_P = 8
 MI_DECODE_FUSED_MERGE = 16
 MI_DECODE_SKIP_MERGE = 32
-MI_DECODE_SEQ_ORDER = 64
 MI_DECODE_COUNTER_BYTES = 1 << 20
 MI_ALLREDUCE_MAX_RANKS, MI_ALLREDUCE_HANDLE_BYTES = 8, 64
 
@@ -121,13 +120,24 @@ SIGNATURES = {
                                       c_int32, c_int32, c_int32, c_float, c_int64, c_int64,
                                       c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int,
                                       c_int, c_int32, _P]),
+    "mi_paged_attn_decode_ordered": (c_int, [_P, _P, _P, _P, _P, _P, c_int32, c_int32, c_int32, c_int32,
+                                              c_int32, c_int32, c_int32, c_float, c_int64, c_int64,
+                                              c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int,
+                                              c_int, c_int32, _P, _P]),
     "mi_rope_cache_paged_attn_decode": (c_int, [_P, _P, _P, _P, _P, _P, c_int32, c_int32, _P, _P, c_float, _P, _P, _P, _P, _P, c_int32, c_int32,
                                                  c_int32, c_int32, c_int32, c_int32, c_int32, c_float, c_int64, c_int64,
                                                  c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int,
                                                  c_int, c_int32, _P]),
+    "mi_rope_cache_paged_attn_decode_ordered": (c_int, [_P, _P, _P, _P, _P, _P, c_int32, c_int32, _P, _P, c_float, _P, _P, _P, _P, _P, c_int32, c_int32,
+                                                         c_int32, c_int32, c_int32, c_int32, c_int32, c_float, c_int64, c_int64,
+                                                         c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int,
+                                                         c_int, c_int32, _P, _P]),
     "mi_rope_cache_paged_attn_decode_splitk": (c_int, [_P, _P, c_int32, _P, _P, _P, c_int32, c_int32, _P, _P, c_float, _P, _P, _P, _P, _P,
                                                         c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_float, c_int64,
                                                         c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, c_int, c_int32, _P]),
+    "mi_rope_cache_paged_attn_decode_splitk_ordered": (c_int, [_P, _P, c_int32, _P, _P, _P, c_int32, c_int32, _P, _P, c_float, _P, _P, _P, _P, _P,
+                                                                c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_float, c_int64,
+                                                                c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, c_int, c_int32, _P, _P]),
     "mi_paged_attn_prefill": (c_int, [_P, _P, _P, _P, _P, _P, _P, c_int32, c_int32, c_int32,
                                        c_int32, c_int32, c_int32, c_int32, c_int32, c_float,
                                        c_int64, c_int64, c_int64, c_int64, c_int64, c_int, _P]),
@@ -214,7 +224,7 @@ SIGNATURES = {
     "mi_paged_attn_decode_biased": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_float, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
                                             c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, _P]),
     "mi_paged_attn_decode_biased_ordered": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_float, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
-                                                    c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, c_int32, _P]),
+                                                    c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int32, _P, c_int64, c_int, _P, _P]),
     "mi_decode_seq_order": (c_int, [_P, _P, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, _P]),
     "mi_paged_attn_prefill_biased": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, c_float, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32,
                                              c_int32, c_int32, c_float, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int32,

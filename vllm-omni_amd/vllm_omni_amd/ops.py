@@ -375,7 +375,7 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     wave of each (sequence, head group) instead of a second kernel — same bits.  Returns ``out``.
     ``slopes`` / ``sinks`` (fp32 [nq]): a distance bias (score - slope * (position - key position)) and one more term
     exp(sink) of the softmax's denominator, and the output times ``out_scale``; bf16 and the default mode only.
-    ``order``: ``decode_seq_order`` of these lengths and sizes (speed only: same bits).
+    ``order``: ``decode_seq_order`` of these sequences (speed only: the lengths are ``seq_lens``'s whatever it was made of, and the bits stay).
     """
     _gpu(out, q, k_cache, v_cache, block_table, seq_lens, workspace, slopes, sinks, order)
     nb, bs, hkv, d = k_cache.shape
@@ -397,7 +397,7 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         fused_merge = DECODE_FUSED_MERGE and ready
     elif fused_merge and not ready:
         raise ValueError("fused_merge needs a workspace from ops.new_decode_workspace (zeroed arrival counters)")
-    lens, ordered = _ordered_lens(seq_lens, order, s)
+    seq_order = _seq_order(order, s)
     if slopes is None and sinks is None and out_scale != 1.0:
         raise ValueError("out_scale goes with a distance bias or a sink")
     if slopes is not None or sinks is not None:
@@ -405,12 +405,12 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         if force_valu or rounded_p or packed_pv is False or out.dtype != q.dtype:
             raise ValueError("a distance bias or a sink runs in the default mode only")
         check("mi_paged_attn_decode_biased_ordered", lib.mi_paged_attn_decode_biased_ordered(
-            _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(lens), _p(slopes), _p(sinks), float(out_scale), s, nq, hkv, d, bs,
+            _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(seq_lens), _p(slopes), _p(sinks), float(out_scale), s, nq, hkv, d, bs,
             block_table.stride(0), int(max_seq_len), float(scale), q.stride(0), out.stride(0), cb, ct, ch, int(partition_size),
-            _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(q.dtype), ordered, _stream()))
+            _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(q.dtype), _p(seq_order), _stream()))
         return out
-    check("mi_paged_attn_decode", lib.mi_paged_attn_decode(
-        _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(lens), s, nq, hkv, d, bs,
+    check("mi_paged_attn_decode_ordered", lib.mi_paged_attn_decode_ordered(
+        _p(out), _p(q), _p(k_cache), _p(v_cache), _p(block_table), _p(seq_lens), s, nq, hkv, d, bs,
         block_table.stride(0), int(max_seq_len), float(scale), q.stride(0), out.stride(0), cb, ct, ch,
         int(partition_size), _p(workspace),
         workspace.numel() * workspace.element_size() if workspace is not None else 0,
@@ -419,18 +419,17 @@ def paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         | (_C.MI_DECODE_FORCE_VALU if force_valu else 0)
         | (_C.MI_DECODE_ROUNDED_P if rounded_p else 0)
         | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0)
-        | ordered
         | (_C.MI_DECODE_SKIP_MERGE if _skip_merge else 0)   # bench.py's kernel-only timing; never set by the product
         | (_C.MI_DECODE_NONTEMPORAL if (DECODE_NONTEMPORAL if nontemporal is None else nontemporal) else 0),
-        _stream()))
+        _p(seq_order), _stream()))
     return out
 
 
 def decode_seq_order(seq_lens: torch.Tensor, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int, max_seq_len: int,
                      partition_size: int = 0) -> Optional[torch.Tensor]:
     """int32 [2, S] on the device: the lengths, and the order in which the decode attention launches of one step (the default mode, these
-    sizes) should take the sequences — longest first.  For their ``order`` as long as ``seq_lens`` holds these values.  None where a
-    launch gains nothing from it."""
+    sizes) should take the sequences — longest first.  For their ``order``; one of other lengths costs speed alone.  None where a launch
+    gains nothing from it."""
     _gpu(seq_lens)
     _i32(seq_lens)
     s = seq_lens.numel()
@@ -446,13 +445,13 @@ def decode_seq_order(seq_lens: torch.Tensor, num_q_heads: int, num_kv_heads: int
     return out
 
 
-def _ordered_lens(seq_lens: torch.Tensor, order: Optional[torch.Tensor], s: int):
-    """(what a decode launch of s sequences reads as their lengths, its flag)"""
+def _seq_order(order: Optional[torch.Tensor], s: int) -> Optional[torch.Tensor]:
+    """the row of ``decode_seq_order`` that a decode launch of s sequences reads"""
     if order is None:
-        return seq_lens, 0
+        return None
     if order.dtype != torch.int32 or tuple(order.shape) != (2, s) or not order.is_contiguous():
         raise ValueError("order: decode_seq_order of this call's sequences")
-    return order, _C.MI_DECODE_SEQ_ORDER
+    return order[1]
 
 
 def rope_decode_fusable(q: torch.Tensor, k_cache: torch.Tensor, positions: torch.Tensor, rot_dim: int,
@@ -498,15 +497,15 @@ def rope_cache_paged_attn_decode(out: torch.Tensor, q: torch.Tensor, k: torch.Te
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = new_decode_workspace(need, q.device)
     fused_merge = DECODE_FUSED_MERGE and _decode_ws_ready(workspace)
-    lens, ordered = _ordered_lens(seq_lens, order, s)
-    check("mi_rope_cache_paged_attn_decode", lib.mi_rope_cache_paged_attn_decode(
+    seq_order = _seq_order(order, s)
+    check("mi_rope_cache_paged_attn_decode_ordered", lib.mi_rope_cache_paged_attn_decode_ordered(
         _p(out), _p(q), _p(k), _p(v), _p(positions), _p(cos_sin_cache), max_pos, rot_dim, _p(q_norm_weight),
         _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache),
-        _p(slot_mapping), _p(block_table), _p(lens), s, nq, hkv, d, bs, block_table.stride(0), int(max_seq_len),
+        _p(slot_mapping), _p(block_table), _p(seq_lens), s, nq, hkv, d, bs, block_table.stride(0), int(max_seq_len),
         float(scale), q.stride(0), k.stride(0), v.stride(0), out.stride(0), cb, ct, ch, int(partition_size), _p(workspace),
         workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(q.dtype), _dt(out.dtype),
-        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | ordered | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0)
-        | (_C.MI_DECODE_SKIP_MERGE if _skip_merge else 0), _stream()))
+        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0)
+        | (_C.MI_DECODE_SKIP_MERGE if _skip_merge else 0), _p(seq_order), _stream()))
     return out
 
 
@@ -545,13 +544,13 @@ def rope_cache_paged_attn_decode_splitk(part: "SplitKPartials", num_q_heads: int
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = new_decode_workspace(need, part.device)
     fused_merge = DECODE_FUSED_MERGE and _decode_ws_ready(workspace)
-    lens, ordered = _ordered_lens(seq_lens, order, s)
-    check("mi_rope_cache_paged_attn_decode_splitk", lib.mi_rope_cache_paged_attn_decode_splitk(
+    seq_order = _seq_order(order, s)
+    check("mi_rope_cache_paged_attn_decode_splitk_ordered", lib.mi_rope_cache_paged_attn_decode_splitk_ordered(
         _p(out), _p(part.part), part.split, _p(part.bias), _p(positions), _p(cos_sin_cache), max_pos, rot_dim, _p(q_norm_weight),
-        _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache), _p(slot_mapping), _p(block_table), _p(lens), s, num_q_heads,
+        _p(k_norm_weight), float(norm_eps), _p(k_cache), _p(v_cache), _p(slot_mapping), _p(block_table), _p(seq_lens), s, num_q_heads,
         hkv, d, bs, block_table.stride(0), int(max_seq_len), float(scale), out.stride(0), cb, ct, ch, int(partition_size),
         _p(workspace), workspace.numel() * workspace.element_size() if workspace is not None else 0, _dt(part.dtype), _dt(out.dtype),
-        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | ordered | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0), _stream()))
+        _C.MI_DECODE_PACKED_PV | _C.MI_DECODE_NONTEMPORAL | (_C.MI_DECODE_FUSED_MERGE if fused_merge else 0), _p(seq_order), _stream()))
     return out
 
 
