@@ -113,3 +113,23 @@ def test_an_order_of_other_lengths(biased):
     want = ops.paged_attn_decode(torch.empty_like(q), q, kc, vc, bt, lens, bound, hd ** -0.5, **kw)
     got = ops.paged_attn_decode(torch.empty_like(q), q, kc, vc, bt, lens, bound, hd ** -0.5, order=order, **kw)
     assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
+# lengths below zero are empty sequences: the order is a permutation all the same, and nothing is written behind it
+@pytest.mark.parametrize("s", [65, 67, 120, 129, 1023])
+def test_lengths_below_zero(s):
+    from vllm_omni_amd import _C, ops
+
+    dev = torch.device("cuda", 0)
+    lens = torch.randint(-3, 700, (s,), dtype=torch.int32, generator=torch.Generator().manual_seed(s))
+    lens[:8] = torch.tensor([-2, -1, 0, -7, -(2 ** 31), 700, -2, -3])
+    lens = lens.to(dev)
+    room = torch.full((2 * s + 64,), 12345, dtype=torch.int32, device=dev)
+    code = _C.lib.mi_decode_seq_order(room.data_ptr(), lens.data_ptr(), s, 28, 4, 128, 16, 700, 0, _C.MI_DECODE_PACKED_PV,
+                                      torch.cuda.current_stream().cuda_stream)
+    assert code == _C.MI_OK
+    assert torch.equal(room[:s], lens)
+    assert torch.equal(room[s:2 * s].sort().values, torch.arange(s, dtype=torch.int32, device=dev))
+    assert (room[2 * s:] == 12345).all()
+    order = ops.decode_seq_order(lens, 28, 4, 128, 16, 700)
+    assert torch.equal(order.view(-1), room[:2 * s])

@@ -822,9 +822,10 @@ __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __res
   const int t = threadIdx.x;
   if (t == 0) least = 0x7fffffff, most = 0;
   if (t < kOrderEach) ranks[t] = 0;
-  lens[t] = t < num_seqs ? seq_lens[t] : -1;      // (no sequence: behind the empty ones)
+  // (no sequence: behind the empty ones, and those are of any length <= 0: ranks stay below num_seqs)
+  lens[t] = t < num_seqs ? max(seq_lens[t], 0) : -1;
   __syncthreads();
-  int lo = t < num_seqs ? lens[t] : 0x7fffffff, hi = max(lens[t], 0);
+  int lo = t < num_seqs ? lens[t] : 0x7fffffff, hi = lens[t];
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
     lo = min(lo, __shfl_xor(lo, d, 64));
@@ -837,6 +838,7 @@ __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __res
   constexpr int parts = kOrderSeqs / kOrderEach;
   const int quads = (num_seqs + 3) / 4, part = t / kOrderEach;
   const int i = min(kOrderEach * (int)blockIdx.x + t % kOrderEach, kOrderSeqs - 1), len = lens[i];
+  const int32_t given = i < num_seqs ? seq_lens[i] : 0;
   int rank = 0;
 #pragma unroll 4
   for (int j = 4 * (part * quads / parts); j < 4 * ((part + 1) * quads / parts); j += 4) {
@@ -847,7 +849,7 @@ __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __res
   atomicAdd(&ranks[t % kOrderEach], rank);
   __syncthreads();
   if (t >= kOrderEach || i >= num_seqs) return;
-  out[i] = len;
+  out[i] = given;
   rank = ranks[t];
   const int round = rank / o.per, first = round * o.per;
   const int place = most - least <= most / 16 ? i      // nothing to even out
