@@ -133,3 +133,14 @@ def test_lengths_below_zero(s):
     assert (room[2 * s:] == 12345).all()
     order = ops.decode_seq_order(lens, 28, 4, 128, 16, 700)
     assert torch.equal(order.view(-1), room[:2 * s])
+
+
+# the empty rows that fill a captured step up do not count as short contexts
+@pytest.mark.parametrize("lens,kept", [([700] * 117 + [0] * 3, True), ([0] * 5 + [660] * 60 + [700] * 50 + [0] * 5, True), ([0] * 120, True),
+                                       ([600] * 60 + [700] * 57 + [0] * 3, False), ([0] * 7 + [1] + [700] * 112, False)])
+def test_empty_rows_do_not_count(lens, kept):
+    from vllm_omni_amd import ops
+
+    order = ops.decode_seq_order(torch.tensor(lens, dtype=torch.int32, device="cuda"), 28, 4, 128, 16, 700)
+    assert torch.equal(order[1].cpu(), torch.arange(120, dtype=torch.int32)) == kept
+    assert torch.equal(order[1].cpu().sort().values, torch.arange(120, dtype=torch.int32))

@@ -811,7 +811,8 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
 }
 
 // Places of the sequences, longest first: how many are longer than each (or as long, in front of it).  A workgroup has 128 sequences, eight threads
-// for each.  Lengths within a sixteenth of each other stay as they are.  Once a step; 120 sequences 3.4 us, 256 4.1, 512 5.6, 1024 8.4.
+// for each.  Lengths within a sixteenth of each other, empty ones aside (the rows that fill a batch up), stay as they are.  Once a step; 120
+// sequences 3.4 us, 256 4.1, 512 5.6, 1024 8.4.
 constexpr int kOrderSeqs = 1024, kOrderEach = 128;
 __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __restrict__ out, const int32_t* __restrict__ seq_lens, int num_seqs,
                                                                   const DecodeOrder o) {
@@ -825,7 +826,7 @@ __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __res
   // (no sequence: behind the empty ones, and those are of any length <= 0: ranks stay below num_seqs)
   lens[t] = t < num_seqs ? max(seq_lens[t], 0) : -1;
   __syncthreads();
-  int lo = t < num_seqs ? lens[t] : 0x7fffffff, hi = lens[t];
+  int lo = lens[t] > 0 ? lens[t] : 0x7fffffff, hi = lens[t];
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
     lo = min(lo, __shfl_xor(lo, d, 64));
