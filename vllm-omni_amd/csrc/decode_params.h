@@ -49,8 +49,8 @@ struct DecodeParams {
   int32_t num_slabs = 0;
   int64_t slab_stride = 0, slab_row = 0;
   bool group_parts = false;   // matrix-core kernel: the partitions are the waves of a workgroup and merge there
-  const int32_t* seq_order = nullptr;   // ... [num_seqs]: the sequence of every place in the launch (decode_seq_order), nullptr: as they are
   int32_t turn = 0;           // ... lone waves: the order of a head group's partitions moves by one every so many waves (0: it does not)
+  const int32_t* seq_order = nullptr;   // ... [num_seqs]: the sequence of every place in the launch (mi_decode_seq_order), nullptr: as they are
 };
 
 // paged_attn_decode_mfma.hip

@@ -153,8 +153,9 @@ __device__ __forceinline__ lds_char* ring_base() {
     return (lds_char*)ring;
   }
 }
+// ORDER: the sequences are taken in p.seq_order.  A form of its own: the look-up stands in front of a wave's loads.
 template <typename Tag, int HD, int AUX, bool SPLIT, int NS, bool ROPE = false, bool NORM = false, bool BIAS = false, bool GROUP = false,
-          bool PART = false>
+          bool PART = false, bool ORDER = false>
 __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void decode_mfma_kernel(const DecodeParams p, const int gh) {
   scalar_cache_acquire();
   using E = Elem<Tag>;
@@ -174,8 +175,8 @@ __global__ __launch_bounds__(GROUP ? 64 * group_parts_max<HD> : 64, 2) void deco
   // lone waves: a head group's partitions side by side, turned where decode_mfma_turn says so
   const int part = GROUP ? wid : (p.turn ? wave + wave / p.turn : wave) % p.num_parts;
   const int hw = (wave / p.num_parts) % (p.num_q_heads / gh);
-  const int place = wave / (p.num_parts * (p.num_q_heads / gh));
-  const int seq = p.seq_order ? p.seq_order[place] : place;
+  int seq = wave / (p.num_parts * (p.num_q_heads / gh));
+  if constexpr (ORDER) seq = p.seq_order[seq];
   const int qh0 = hw * gh;
   const int kvh = qh0 / p.kv_group;
 
@@ -859,23 +860,31 @@ __global__ __launch_bounds__(kOrderSeqs) void decode_order_kernel(int32_t* __res
 }
 
 // one wave a workgroup, or (group) the partitions of a sequence's head group as the waves of one
-template <typename Tag, int HD, int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool BIAS = false, bool PART = false>
-int launch_form(const DecodeParams& p, int gh, hipStream_t stream) {
+template <typename Tag, int HD, int AUX, bool SPLIT, bool ROPE, bool NORM, bool BIAS, bool PART, bool ORDER>
+int launch_order_form(const DecodeParams& p, int gh, hipStream_t stream) {
   constexpr int NS = HD == 128 ? 2 : MI_DECODE_NS64, ring = ring_bytes<HD>;
   static_assert(ring >= (16 * HD + 32) * 4, "a wave's partial takes its ring's place");
   const int64_t groups = (int64_t)p.num_seqs * (p.num_q_heads / gh);
   if (groups * p.num_parts > INT32_MAX) return MI_ERR_UNSUPPORTED;
   if (p.group_parts) {
-    auto kern = decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, true, PART>;
+    auto kern = decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, true, PART, ORDER>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        group_parts_max<HD> * ring);
     if (attr != hipSuccess) return MI_ERR_LAUNCH;
     hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(64 * p.num_parts), p.num_parts * ring, stream, p, gh);
   } else {
-    hipLaunchKernelGGL((decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, false, PART>), dim3((unsigned)(groups * p.num_parts)), dim3(64), 0,
-                       stream, p, gh);
+    hipLaunchKernelGGL((decode_mfma_kernel<Tag, HD, AUX, SPLIT, NS, ROPE, NORM, BIAS, false, PART, ORDER>), dim3((unsigned)(groups * p.num_parts)),
+                       dim3(64), 0, stream, p, gh);
   }
   return launch_status();
+}
+// (an order changes speed alone: heads of 64 dims, which decode_mfma_order leaves out, and the measurement forms have no use for one)
+template <typename Tag, int HD, int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool BIAS = false, bool PART = false>
+int launch_form(const DecodeParams& p, int gh, hipStream_t stream) {
+  if constexpr (HD == 128 && AUX == 2 && SPLIT) {
+    if (p.seq_order) return launch_order_form<Tag, HD, AUX, SPLIT, ROPE, NORM, BIAS, PART, true>(p, gh, stream);
+  }
+  return launch_order_form<Tag, HD, AUX, SPLIT, ROPE, NORM, BIAS, PART, false>(p, gh, stream);
 }
 template <int AUX, bool SPLIT, bool ROPE = false, bool NORM = false, bool PART = false>
 int launch_types(const DecodeParams& p, int gh, int head_dim, int dtype, hipStream_t stream) {
