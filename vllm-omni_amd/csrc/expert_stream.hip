@@ -34,7 +34,7 @@ struct StreamParams {
   int32_t N, K;
   int32_t rpt, gather_div;      // rows per tile; > 0: source row = pair index / gather_div, else the row itself
   int32_t nx;                   // weight tiles of a row tile
-  int32_t turn;                 // a tile's k blocks begin with grouped_first_block and go round
+  int32_t turn;                 // the TURN form: a tile's k blocks begin with grouped_first_block and go round
   uint32_t div_magic;           // 2^32 / gather_div, rounded up: exact for pair indices below 2^28
   uint32_t map_bytes;
   const int32_t* row_map;       // [max_rows] pair index or -1; the pairs of a tile in front
@@ -80,7 +80,7 @@ __device__ __forceinline__ void lds_read_frags(uint32_t w0, uint32_t w1, uint32_
       : "memory");
 }
 
-template <typename Tag, int FORM>
+template <typename Tag, int FORM, bool TURN>
 __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParams p) {
   scalar_cache_acquire();
   using E = Elem<Tag>;
@@ -157,13 +157,13 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
     const StreamRange r = stream_range(lt.col, lt.cut, p.N, p.K, GATED);
     wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w + (int64_t)lt.expert * p.w_expert_stride + r.first), 0, (int)r.bytes, 0x00020000);
     pieces = r.pieces;
-    if (p.turn) w_first = xn_first = grouped_first_block(GATED, lt.expert, lt.col, p.N, n_it);
+    if constexpr (TURN) w_first = xn_first = grouped_first_block(GATED, lt.expert, lt.col, p.N, n_it);
     ++n_loaded;
     if (item + n_loaded * per < items) load_map(item + n_loaded * per, n_loaded % 3);
   };
   int w_it = 0, w_slot = 0, x_it = 0, x_slot = 0;
   const auto issue_w = [&]() {
-    const int kb = 128 * (w_it + w_first - (w_it + w_first < n_it ? 0 : n_it));
+    const int kb = 128 * (TURN ? w_it + w_first - (w_it + w_first < n_it ? 0 : n_it) : w_it);
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(lds + w_slot * kWStage + (wid + 4 * i) * 1024), 16, i < pieces ? wo[i] : kDead,
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
     }
   };
   const auto issue_x = [&]() {
-    const int kb = 128 * (x_it + x_first - (x_it + x_first < n_it ? 0 : n_it));
+    const int kb = 128 * (TURN ? x_it + x_first - (x_it + x_first < n_it ? 0 : n_it) : x_it);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(x_r, (lds_void*)(lds + kXRing + x_slot * kXStage + (wid + 4 * i) * 1024), 16, xo[i], kb, 0, 0);
@@ -311,13 +311,17 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
   __builtin_amdgcn_s_waitcnt(stream_vmcnt(0));      // no load may land in this LDS once it is another workgroup's
 }
 
-template <typename Tag, int FORM>
-int launch_stream_form(const StreamParams& p, const dim3 grid, hipStream_t s) {
-  auto kern = expert_stream_kernel<Tag, FORM>;
+template <typename Tag, int FORM, bool TURN>
+int launch_stream_turn(const StreamParams& p, const dim3 grid, hipStream_t s) {
+  auto kern = expert_stream_kernel<Tag, FORM, TURN>;
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kStreamLds);
   if (attr != hipSuccess) return MI_ERR_LAUNCH;
   hipLaunchKernelGGL(kern, grid, dim3(256), kStreamLds, s, p);
   return launch_status();
+}
+template <typename Tag, int FORM>
+int launch_stream_form(const StreamParams& p, const dim3 grid, hipStream_t s) {
+  return p.turn ? launch_stream_turn<Tag, FORM, true>(p, grid, s) : launch_stream_turn<Tag, FORM, false>(p, grid, s);
 }
 template <typename Tag>
 int launch_stream(const StreamParams& p, int form, const dim3 grid, hipStream_t s) {

@@ -34,10 +34,10 @@
 namespace mi {
 namespace {
 
-template <typename Tag, typename OT, int NSLAB, int MT, int MH, int NL, bool GATED, bool GROUPED = false, int NST = 3>
+template <typename Tag, typename OT, int NSLAB, int MT, int MH, int NL, bool GATED, bool GROUPED = false, int NST = 3, bool TURN = false>
 __global__ __launch_bounds__(64 * (NSLAB * MH + NL)) void skinny_gemm_kernel(const SkinnyParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  skinny_tile<Tag, OT, NSLAB, MT, MH, NL, GATED, GROUPED, NST>(p, (int)blockIdx.x, smem);
+  skinny_tile<Tag, OT, NSLAB, MT, MH, NL, GATED, GROUPED, NST, false, TURN>(p, (int)blockIdx.x, smem);
 }
 
 // ======================================================================================================= v2 (129-256 rows)
@@ -211,7 +211,7 @@ struct V2 {
   }
 };
 
-template <typename Tag, typename OT, int G, int G0, bool GATED>
+template <typename Tag, typename OT, int G, int G0, bool GATED, bool TURN>
 __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_v2_kernel(const SkinnyParams p) {
   using C = V2<Tag, OT, G, G0, GATED>;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -257,10 +257,11 @@ __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_
         src[i] = reinterpret_cast<const char*>(p.w + (int64_t)n * p.K + 64 * (int64_t)b_lo + 8 * lc);
       }
     }
-    const int first = p.turn ? (int)((uint32_t)wg % (uint32_t)max(n_it, 1)) : 0;
+    int kk = 0;      // TURN: k block of the next step to issue
+    if constexpr (TURN) kk = (int)((uint32_t)wg % (uint32_t)max(n_it, 1));
     auto issue = [&](int it, int stage) {
       char* st = smem + stage * C::kStage;
-      const int kk = it + first - (it + first < n_it ? 0 : n_it);
+      if constexpr (!TURN) kk = it;
 #pragma unroll
       for (int i = 0; i < C::PPL; ++i) {
         if (l + kV2Loaders * i < C::XI)
@@ -269,6 +270,9 @@ __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_
         else
           __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk),
                                            (lds_void*)(st + (l + kV2Loaders * i) * 1024), 16, 0, MI_SKINNY_W_AUX);
+      }
+      if constexpr (TURN) {
+        if (++kk == n_it) kk = 0;
       }
     };
     const uint32_t full0 = lds0 + C::kFlags, free0 = lds0 + C::kFlags + C::NST * 16;
@@ -463,15 +467,20 @@ int linear_v2() {   // MI_LINEAR_V2=0: the first-generation kernel at 129-256 ro
   return e ? atoi(e) : 1;
 }
 
-template <typename Tag, typename OT, int G, int G0, bool GATED>
-int launch_v2(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
+template <typename Tag, typename OT, int G, int G0, bool GATED, bool TURN>
+int launch_v2_turn(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
   using C = V2<Tag, OT, G, G0, GATED>;
-  auto kern = skinny_gemm_v2_kernel<Tag, OT, G, G0, GATED>;
+  auto kern = skinny_gemm_v2_kernel<Tag, OT, G, G0, GATED, TURN>;
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
   if (attr != hipSuccess) return MI_ERR_LAUNCH;
   hipLaunchKernelGGL(kern, grid, dim3(64 * (kV2Consumers + kV2Loaders)), C::kLds, s, p);
   return launch_status();
+}
+
+template <typename Tag, typename OT, int G, int G0, bool GATED>
+int launch_v2(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
+  return p.turn ? launch_v2_turn<Tag, OT, G, G0, GATED, true>(p, grid, s) : launch_v2_turn<Tag, OT, G, G0, GATED, false>(p, grid, s);
 }
 
 // `dtype`: the type of the 16-bit OUTPUT (and of the operands, unless `int8`: then x / w are int8 rows and the sums
@@ -576,17 +585,21 @@ int launch_skinny(const SkinnyParams& p_in, const SkinnyPlan& pl, bool gated, in
 
 // MT: 16-row m-tiles of a tile's row image: 4 (<= 64 token rows per tile: decode batches), 8 / 16 (128 / 256 rows: what
 // tall_gemm.hip does not take)
-template <typename Tag, bool GATED, int MT>
-int launch_grouped_t(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
+template <typename Tag, bool GATED, int MT, bool TURN>
+int launch_grouped_turn(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
   constexpr int MH = MT == 4 ? 1 : 2;
   constexpr int nst = MT == 4 ? MI_SKINNY_GROUPED_NST : 3;
-  auto kern = skinny_gemm_kernel<Tag, Tag, 4, MT, MH, 4, GATED, true, nst>;
+  auto kern = skinny_gemm_kernel<Tag, Tag, 4, MT, MH, 4, GATED, true, nst, TURN>;
   constexpr int lds = nst * (MT * 2048 + 4 * 4096);
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return MI_ERR_LAUNCH;
   hipLaunchKernelGGL(kern, grid, dim3(64 * (4 * MH + 4)), lds, s, p);
   return launch_status();
+}
+template <typename Tag, bool GATED, int MT>
+int launch_grouped_t(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
+  return p.turn ? launch_grouped_turn<Tag, GATED, MT, true>(p, grid, s) : launch_grouped_turn<Tag, GATED, MT, false>(p, grid, s);
 }
 template <typename Tag, bool GATED>
 int launch_grouped_rows(const SkinnyParams& p, const dim3 grid, int rpt, hipStream_t s) {

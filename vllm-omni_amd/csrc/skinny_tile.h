@@ -74,7 +74,9 @@ struct SkinnyParams {
   int64_t w_expert_stride;     // elements
   int32_t dbg;            // MI_LINEAR_DBG (timing experiments only): 1 = no DMA, 2 = no fragment reads / MFMAs, 4 = no reduce launch, 8 = no output stores
   int64_t ldx, ldo;
-  int32_t turn = 0;      // 1: a weight tile's k blocks begin with that of the tile's number and go round (skinny_turn); GROUPED: grouped_first_block
+  // 1: a work item's k blocks begin with that of its number (tile x slices + slice) and go round (skinny_turn).  GROUPED: the TURN form, in which
+  // a weight tile's do with grouped_first_block
+  int32_t turn = 0;
 };
 
 // operands as plain vectors (a HIP `uint4` is a struct: its copies between address spaces become memcpys that keep
@@ -197,7 +199,7 @@ __device__ __forceinline__ float glu_value(const SkinnyParams& p, float gt, floa
 // NST: stages of the LDS ring; NST - 1 steps are in flight ahead of the consumers (three everywhere: MI_SKINNY_NST4).
 // COH: the tile is one stage of a producer / consumer chain INSIDE one launch (csrc/cp_stack.hip): x is read and every output
 // written at device scope (sc1: past the XCD's L2), so that a grid barrier — not a kernel boundary — can stand between them.
-template <typename Tag, typename OT, int NSLAB, int MT, int MH, int NL, bool GATED, bool GROUPED = false, int NST = 3, bool COH = false>
+template <typename Tag, typename OT, int NSLAB, int MT, int MH, int NL, bool GATED, bool GROUPED = false, int NST = 3, bool COH = false, bool TURN = false>
 __device__ __forceinline__ void skinny_tile(const SkinnyParams& p, const int wg_linear, char* const smem) {
   // One pipeline step = one 64-wide k block.  A stage of the LDS ring is one image of 128-byte rows: the 16 MT rows of
   // x, then the tile's 32 NSLAB weight rows; 16-byte chunk c of row r sits at chunk c ^ ((r >> 1) & 7).  The image is
@@ -298,32 +300,36 @@ __device__ __forceinline__ void skinny_tile(const SkinnyParams& p, const int wg_
     // step `it` of the workgroup = k block it % n_it of its tile it / n_it: the x pieces start over with every tile, the
     // weight pieces move on by one tile's rows (a chained launch has whole tiles only: the host checks)
     const int64_t w_tile_bytes = (int64_t)(GATED ? 16 * NSLAB : TR) * p.K * 2;
-    int kk_first = 0, tile_next = tile0;
-    const auto take = [&]() {
-      if (!p.turn || n_it == 0) return;
-      if constexpr (GROUPED) kk_first = grouped_first_block(GATED, expert, tile_next * (GATED ? 16 * NSLAB : TR), p.N, n_it);
-      else kk_first = wg % n_it;
-    };
-    take();
-    int kk_next = 0;                 // k block of the next step to issue, counted from kk_first
+    // (launches that are not turned pay nothing for it: with a wrap of its own at every step gated 10368 x 3584, 1 row, took 19.1 us, so 18.3; experts'
+    // 1024 x 384 up, 1 token 11.25 | 10.9)
+    int kk_first = 0, tile_next = tile0;      // TURN: the block that a tile begins with, and the next step's tile
+    const auto take = [&]() { kk_first = grouped_first_block(GATED, expert, tile_next * (GATED ? 16 * NSLAB : TR), p.N, n_it); };
+    if constexpr (TURN) take();
+    else if (!GROUPED && p.turn && n_it > 0) kk_first = wg % n_it;
+    int kk_next = kk_first;          // k block of the next step to issue
     int64_t w_next = 0;              // byte offset of its tile's weight rows
     auto issue = [&](int stage) {
       char* st = smem + stage * kStage;
-      const int kk = kk_next + kk_first - (kk_next + kk_first < n_it ? 0 : n_it);
 #pragma unroll
       for (int i = 0; i < PPL; ++i) {
         if (l + NL * i < XI)
-          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk),
+          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk_next),
                                            (lds_void*)(st + (l + NL * i) * 1024), 16, 0, COH ? kAuxAgent : 0);
         else
-          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk + w_next),
+          __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk_next + w_next),
                                            (lds_void*)(st + (l + NL * i) * 1024), 16, 0, MI_SKINNY_W_AUX);
       }
       if (++kk_next == n_it) {
         kk_next = 0;
-        w_next += w_tile_bytes;
-        ++tile_next;
-        if constexpr (GROUPED) take();
+        if constexpr (GROUPED && !TURN) w_next += w_tile_bytes;
+      }
+      if constexpr (TURN) {
+        if (kk_next == kk_first) {
+          w_next += w_tile_bytes;
+          ++tile_next;
+          take();
+          kk_next = kk_first;
+        }
       }
     };
     const int total = n_it * chain;

@@ -37,9 +37,9 @@ struct TallParams {
   const int32_t* num_tiles;     // [1]
   const float* pair_weights;    // RELU_SQUARED: the sums of a pair's row times this, in front of the activation
   int64_t ldx, ldo, w_expert_stride;
+  int32_t turn;      // the TURN form: experts whose tiles' k blocks begin with grouped_first_block and go round
   // DENSE: one weight matrix, all M rows.  The first `whole` tiles are items of their own; each of the others is cut along K into
   // `split` items that leave fp32 sums in part [item][256][256]
-  int32_t turn;      // experts: a tile's k blocks begin with grouped_first_block and go round
   int32_t M, whole, split, group;
   const uint16_t* bias;
   float* part;
@@ -57,7 +57,7 @@ constexpr int kTallStage = 64 * 1024;
 struct TallItem {
   int row0, tile, expert, units;     // units: 64-row units of the row tile that hold live rows
   int kb, n_it;                      // where the item starts along K (bytes) and its 64-wide blocks: an even number
-  int first;                         // the block that it begins with (then round)
+  int first;                         // TURN: the block that it begins with (then round)
   int slab;                          // >= 0: fp32 sums into this slab
   int row[8];
 };
@@ -76,13 +76,12 @@ __device__ __forceinline__ int tall_items(const TallParams& p, bool dense, int x
   return whole;
 }
 
-template <int FORM>
+template <int FORM, bool TURN>
 __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo, int whole, int tail, TallItem& t) {
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   t.kb = 0;
   t.n_it = p.K >> 6;
   t.slab = -1;
-  t.first = 0;
   if constexpr (tall_dense(FORM)) {
     int at = lo + item;
     if (item >= whole) {
@@ -105,7 +104,7 @@ __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo
   t.tile = item - row_tile * p.nx;
   t.row0 = row_tile * p.rpt;
   t.expert = p.tile_expert[row_tile];
-  if (p.turn) t.first = grouped_first_block(tall_gated(FORM), t.expert, t.tile * (tall_gated(FORM) ? kTallN / 2 : kTallN), p.N, t.n_it);
+  if constexpr (TURN) t.first = grouped_first_block(tall_gated(FORM), t.expert, t.tile * (tall_gated(FORM) ? kTallN / 2 : kTallN), p.N, t.n_it);
   t.units = 0;
 #pragma unroll
   for (int u = 0; u < 4; ++u)
@@ -119,9 +118,9 @@ __device__ __forceinline__ void tall_fetch(const TallParams& p, int item, int lo
 }
 
 // where block i of an item lies along K (bytes)
-template <int FORM>
+template <bool TURN>
 __device__ __forceinline__ int tall_block(const TallItem& t, int i) {
-  if constexpr (tall_dense(FORM)) return t.kb + i * 128;
+  if constexpr (!TURN) return t.kb + i * 128;
   const int at = i + t.first;
   return (at < t.n_it ? at : at - t.n_it) * 128;
 }
@@ -173,7 +172,7 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int kLgkm0 = 0xC07F;     // lgkmcnt(0), any vmcnt
 
 // A tile of 64 HM rows x 256 weight rows.  Four waves: 2 (rows) x 2 (weight rows), each 32 HM x 128.
-template <typename Tag, int FORM, int HM>
+template <typename Tag, int FORM, bool TURN, int HM>
 __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s1, char* so, const TallItem& t, uint32_t (&x)[8],
                                           const uint32_t (&wo)[8], const TallItem& nt, bool more) {
   using E = Elem<Tag>;
@@ -238,7 +237,7 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     __builtin_amdgcn_s_waitcnt(kLgkm0);
     barrier();                                   // everybody has read this stage
     // (loads spread over the step: a wave that finds the memory pipe's queue full issues no product either)
-    const int kb = KIND == 0 ? tall_block<FORM>(t, it + 2) : tall_block<FORM>(nt, KIND - 1);
+    const int kb = KIND == 0 ? tall_block<TURN>(t, it + 2) : tall_block<TURN>(nt, KIND - 1);
     if (KIND == 0 || more) tall_issue_w(wo, wr, kb, cur);
     if (KIND == 2) {
       if (more) tall_issue_x<8>(p, x, kb, cur);
@@ -368,7 +367,7 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
   else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 }
 
-template <typename Tag, int FORM>
+template <typename Tag, int FORM, bool TURN = false>
 __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
   scalar_cache_acquire();
   constexpr bool GATED = tall_gated(FORM);
@@ -389,14 +388,14 @@ __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
     wo[i] = (uint32_t)n * (uint32_t)(2 * p.K) + 16 * ((lane & 7) ^ ((row >> 1) & 7));
   }
   TallItem t, nt;
-  tall_fetch<FORM>(p, item, lo, whole, tail, t);
+  tall_fetch<FORM, TURN>(p, item, lo, whole, tail, t);
   tall_rows<FORM>(p, t, x);
   {
     const __amdgpu_buffer_rsrc_t wr = tall_weights<GATED>(p, t);
-    tall_issue_w(wo, wr, tall_block<FORM>(t, 0), s0);
-    tall_issue_x<8>(p, x, tall_block<FORM>(t, 0), s0);
-    tall_issue_w(wo, wr, tall_block<FORM>(t, 1), s1);
-    tall_issue_x<8>(p, x, tall_block<FORM>(t, 1), s1);
+    tall_issue_w(wo, wr, tall_block<TURN>(t, 0), s0);
+    tall_issue_x<8>(p, x, tall_block<TURN>(t, 0), s0);
+    tall_issue_w(wo, wr, tall_block<TURN>(t, 1), s1);
+    tall_issue_x<8>(p, x, tall_block<TURN>(t, 1), s1);
   }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   while (true) {
@@ -406,11 +405,11 @@ __global__ __launch_bounds__(256, 1) void tall_gemm_kernel(const TallParams p) {
     item += stride;
     const bool more = item < items;
     nt = t;
-    if (more) tall_fetch<FORM>(p, item, lo, whole, tail, nt);
-    if (t.units >= 4) tall_tile<Tag, FORM, 4>(p, s0, s1, so, t, x, wo, nt, more);
-    else if (t.units == 3) tall_tile<Tag, FORM, 3>(p, s0, s1, so, t, x, wo, nt, more);
-    else if (t.units == 2) tall_tile<Tag, FORM, 2>(p, s0, s1, so, t, x, wo, nt, more);
-    else tall_tile<Tag, FORM, 1>(p, s0, s1, so, t, x, wo, nt, more);
+    if (more) tall_fetch<FORM, TURN>(p, item, lo, whole, tail, nt);
+    if (t.units >= 4) tall_tile<Tag, FORM, TURN, 4>(p, s0, s1, so, t, x, wo, nt, more);
+    else if (t.units == 3) tall_tile<Tag, FORM, TURN, 3>(p, s0, s1, so, t, x, wo, nt, more);
+    else if (t.units == 2) tall_tile<Tag, FORM, TURN, 2>(p, s0, s1, so, t, x, wo, nt, more);
+    else tall_tile<Tag, FORM, TURN, 1>(p, s0, s1, so, t, x, wo, nt, more);
     if (!more) break;
     t = nt;
   }
@@ -441,12 +440,16 @@ __global__ __launch_bounds__(256) void tall_reduce_kernel(const TallParams p) {
       make_uint4(E::pack(v0[0], v0[1]), E::pack(v0[2], v0[3]), E::pack(v1[0], v1[1]), E::pack(v1[2], v1[3]));
 }
 
+template <typename Tag, bool TURN>
+int launch_tall_form(const TallParams& p, int form, const dim3 grid, hipStream_t s) {
+  if (form == MI_MOE_GATED) hipLaunchKernelGGL((tall_gemm_kernel<Tag, MI_MOE_GATED, TURN>), grid, dim3(256), 0, s, p);
+  else if (form == MI_MOE_PLAIN) hipLaunchKernelGGL((tall_gemm_kernel<Tag, MI_MOE_PLAIN, TURN>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((tall_gemm_kernel<Tag, MI_MOE_RELU_SQUARED, TURN>), grid, dim3(256), 0, s, p);
+  return launch_status();
+}
 template <typename Tag>
 int launch_tall(const TallParams& p, int form, const dim3 grid, hipStream_t s) {
-  if (form == MI_MOE_GATED) hipLaunchKernelGGL((tall_gemm_kernel<Tag, MI_MOE_GATED>), grid, dim3(256), 0, s, p);
-  else if (form == MI_MOE_PLAIN) hipLaunchKernelGGL((tall_gemm_kernel<Tag, MI_MOE_PLAIN>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((tall_gemm_kernel<Tag, MI_MOE_RELU_SQUARED>), grid, dim3(256), 0, s, p);
-  return launch_status();
+  return p.turn ? launch_tall_form<Tag, true>(p, form, grid, s) : launch_tall_form<Tag, false>(p, form, grid, s);
 }
 
 }  // namespace
