@@ -451,15 +451,22 @@ SkinnyPlan skinny_plan(int m, int n, int k, int force_split) {
 namespace mi {
 namespace {
 
-// Whether the weight tiles' k blocks are turned (SkinnyParams::turn).  Workgroups keep step with each other, and with weight rows a multiple of 8192
-// bytes apart all of them then read from the same few channels at a time; begun one block behind its neighbour, each reads elsewhere.  Slices of K
-// do that by themselves unless they begin a multiple of 4096 bytes apart.  As they are | turned, us, cold weights: 33056 x 4096, 1 row 56.2 | 43.0, 64 rows
-// 58.6 | 47.8, 128 rows 63.2 | 55.3, 200 rows 81.2 | 78.3; gated 24576 x 4096, 32 rows 46.8 | 40.5; 15360 x 4096 in two slices, 32 rows 32.9 | 28.6; 4096 x
-// 16384 in eight, 1 row 44.2 | 29.5; experts' 2048 x 768 (rows 4096 bytes apart), 200 tokens, 8 of 64 50.1 | 43.3, 4096 x 1536, 64 tokens 180 | 147.  Not past
-// the line: 6144 x 4096 in five slices, 128 rows 22.4 | 23.6, 15360 x 4096, 200 rows 45.0 | 46.2, 37888 x 3584 45.4 | 45.7; 12288 x 2048 and 2048 x 6144 level.
-// Two blocks apart: 4096 x 16384 38.0, gated 33056 x 4096 46.5.
-int skinny_turn(int k, int split, int mt) {
-  return k % 4096 == 0 && (split == 1 || (mt <= 8 && k % (2048 * split) == 0));
+// Whether the k blocks are turned (SkinnyParams::turn).  Workgroups keep step with each other, and with weight rows a multiple of 8192 bytes apart
+// all of them then read from the same few channels at a time; begun one block behind its neighbour, each reads elsewhere.  Slices of K do that by
+// themselves unless they begin a multiple of 4096 bytes apart.  As they are | turned, us, cold weights: 33056 x 4096, 1 row 56.7 | 44.6, 64 rows 58.3 |
+// 45.2, 128 rows 63.1 | 54.3, 256 rows 81.2 | 79.2; gated 24576 x 4096, 32 rows 44.0 | 38.3; 15360 x 4096 in two slices, 32 rows 30.3 | 28.5; 4096 x
+// 16384 in eight, 1 row 44.2 | 29.5; experts' 2048 x 768 (rows 4096 bytes apart), 200 tokens, 8 of 64 43.8 | 35.6.  Not past the line: 6144 x 4096 in
+// five slices, 128 rows 22.4 | 23.6, 15360 x 4096, 200 rows 45.0 | 46.2, 37888 x 3584 45.4 | 45.7; 12288 x 2048 and 2048 x 6144 level.  Two blocks
+// apart: 4096 x 16384 38.0, gated 33056 x 4096 46.5.
+// Where x is most of what a workgroup takes in, its blocks come best while all workgroups ask for the same ones.  So gated tiles of under 64
+// columns are turned up to 128 rows, and of K 4096 up to 64 rows and past 192 tiles: gated 8192 x 4096, 64 rows 24.9 | 26.8, 12288 x 4096
+// 27.0 | 29.0, 128 rows 31.7 | 34.8, 15360 x 4096, 128 rows 33.7 | 35.5, 12288 x 12288, 256 rows 133 | 179; but 14336 x 4096, 32 rows 26.5 | 24.1,
+// 14336 x 8192, 64 rows 56.4 | 45.9, 128 rows 62.5 | 57.3.  And two slices of K 4096 in 128-row images past 112 tiles: 12288 x 4096, 128
+// rows 32.5 | 33.2, but 14336 x 4096 36.2 | 35.5.
+int skinny_turn(int m, int k, const SkinnyPlan& pl, bool gated) {
+  if (k % 4096 || (pl.split > 1 && (pl.mt > 8 || k % (2048 * pl.split)))) return 0;
+  if (gated && pl.nslab < 4) return m <= 128 && (k > 4096 || (m <= 64 && pl.tiles > 192));
+  return k > 4096 || pl.split == 1 || pl.mt <= 4 || pl.tiles >= 112;
 }
 
 int linear_v2() {   // MI_LINEAR_V2=0: the first-generation kernel at 129-256 rows too (A/B runs; read per call)
@@ -488,7 +495,7 @@ int launch_v2(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
 int launch_skinny(const SkinnyParams& p_in, const SkinnyPlan& pl, bool gated, int dtype, hipStream_t s, bool int8 = false) {
   SkinnyParams p = p_in;
   p.RB = (p.M + 16 * pl.mt - 1) / (16 * pl.mt);
-  p.turn = skinny_turn(p.K, pl.split, pl.mt);
+  p.turn = skinny_turn(p.M, p.K, pl, gated);
   p.U = pl.tiles * pl.split;
   if (dtype != MI_DTYPE_BF16 && dtype != MI_DTYPE_F16) return MI_ERR_UNSUPPORTED;
   if (pl.mt == 16 && pl.nslab >= 4 && linear_v2()) {
