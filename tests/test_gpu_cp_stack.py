@@ -156,3 +156,11 @@ def test_stack_refuses_what_it_was_not_built_for(dev):
     with pytest.raises(ValueError):
         stack.decode(torch.empty(5, H, dtype=torch.bfloat16, device=dev), torch.zeros(5, H, dtype=torch.bfloat16, device=dev),
                      torch.arange(1, 6, dtype=torch.int32, device=dev), 3)
+
+
+# down_proj of rows 16 KB apart in four slices: its launch turns the k blocks of its weight tiles, and so does the phase
+def test_stack_matches_turned_launches(dev, monkeypatch):
+    import sys
+
+    monkeypatch.setattr(sys.modules[__name__], "INTER", 8192)
+    test_stack_matches_the_chain_of_launches(dev, 512, 1, 16, torch.bfloat16)

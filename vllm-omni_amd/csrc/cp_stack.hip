@@ -359,6 +359,7 @@ __device__ __forceinline__ void cp_linear_phase(const uint16_t* x, const uint16_
   q.N = N;
   q.K = K;
   q.S = GATED ? 1 : S;
+  q.turn = !GATED && skinny_in_step(K, S);      // (a gated phase's K is at most 1024)
   q.RB = (M + 63) / 64;
   const int tiles = GATED ? (N + 16 * NSLAB - 1) / (16 * NSLAB) : (N + 32 * NSLAB - 1) / (32 * NSLAB);
   q.U = tiles * q.S;

@@ -464,7 +464,7 @@ namespace {
 // 14336 x 8192, 64 rows 56.4 | 45.9, 128 rows 62.5 | 57.3.  And two slices of K 4096 in 128-row images past 112 tiles: 12288 x 4096, 128
 // rows 32.5 | 33.2, but 14336 x 4096 36.2 | 35.5.
 int skinny_turn(int m, int k, const SkinnyPlan& pl, bool gated) {
-  if (k % 4096 || (pl.split > 1 && (pl.mt > 8 || k % (2048 * pl.split)))) return 0;
+  if (!skinny_in_step(k, pl.split) || (pl.split > 1 && pl.mt > 8)) return 0;
   if (gated && pl.nslab < 4) return m <= 128 && (k > 4096 || (m <= 64 && pl.tiles > 192));
   return k > 4096 || pl.split == 1 || pl.mt <= 4 || pl.tiles >= 112;
 }

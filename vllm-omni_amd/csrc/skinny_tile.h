@@ -79,6 +79,9 @@ struct SkinnyParams {
   int32_t turn = 0;
 };
 
+// Slices of K that begin a multiple of 4096 bytes apart, of weight rows a multiple of 8192: what skinny_turn turns (of 64-row images always)
+__host__ __device__ __forceinline__ bool skinny_in_step(int k, int split) { return k % 4096 == 0 && (split == 1 || k % (2048 * split) == 0); }
+
 // operands as plain vectors (a HIP `uint4` is a struct: its copies between address spaces become memcpys that keep
 // the staging array in scratch)
 template <typename Tag>
