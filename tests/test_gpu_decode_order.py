@@ -144,3 +144,127 @@ def test_empty_rows_do_not_count(lens, kept):
     order = ops.decode_seq_order(torch.tensor(lens, dtype=torch.int32, device="cuda"), 28, 4, 128, 16, 700)
     assert torch.equal(order[1].cpu(), torch.arange(120, dtype=torch.int32)) == kept
     assert torch.equal(order[1].cpu().sort().values, torch.arange(120, dtype=torch.int32))
+
+
+def _step(s, nq, nkv, bound, dtype, dev):
+    """a decode step's rows: uneven contexts with this step's token in them, empty rows with slot -1, blocks of their own"""
+    g = torch.Generator().manual_seed(s + bound)
+    lens = torch.randint(0, bound + 1, (s,), generator=g, dtype=torch.int32)
+    lens[0], lens[1], lens[s // 2], lens[s - 1] = bound, 1, 0, 0
+    cols = (bound + 15) // 16
+    table = (torch.randperm(s * cols, generator=g) + 1).view(s, cols).to(torch.int32)
+    at = (lens.long() - 1).clamp(min=0)
+    slots = torch.where(lens > 0, table[torch.arange(s), at // 16].long() * 16 + at % 16, -1)
+    gd = torch.Generator(device=dev).manual_seed(s)
+    kv = torch.randn(2, s * cols + 1, 16, nkv, 128, generator=gd, device=dev).to(dtype)
+    rows = (nq + 2 * nkv) * 128
+    norms = [(1 + 0.1 * torch.randn(128, generator=gd, device=dev)).to(dtype) for _ in range(2)]
+    slabs = torch.randn(3, s, rows, generator=gd, device=dev)
+    return lens.to(dev), table.to(dev), at.to(dev), slots.to(dev), kv, norms, slabs, torch.randn(rows, generator=gd, device=dev).to(dtype)
+
+
+# the launches of a pure-decode step, which rotate, norm and write the token's cache row as well: outputs and caches
+@pytest.mark.parametrize("slabs", [False, True], ids=["rows", "slabs"])
+@pytest.mark.parametrize("norm", [False, True], ids=["plain", "qk-norm"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("s,nq,nkv,bound", [(120, 28, 4, 700), (70, 28, 4, 1000), (161, 32, 8, 300), (257, 14, 2, 320)])
+def test_steps_that_write_the_cache(s, nq, nkv, bound, dtype, norm, slabs):
+    from vllm_omni_amd import ops
+    from vllm_omni_amd.layers import build_cos_sin_cache
+
+    dev = torch.device("cuda", 0)
+    lens, table, pos, slots, kv, norms, part, bias = _step(s, nq, nkv, bound, dtype, dev)
+    order = ops.decode_seq_order(lens, nq, nkv, 128, 16, bound)
+    assert order is not None and not torch.equal(order[1], torch.arange(s, dtype=torch.int32, device=dev))
+    csc = build_cos_sin_cache(128, 2048, 1e6, device=dev)
+    kw = dict(zip(("q_norm_weight", "k_norm_weight"), norms)) if norm else {}
+    qkv = part[0].to(dtype)
+    got = []
+    for o in (None, order):
+        cache = kv.clone()
+        if slabs:
+            p = ops.SplitKPartials(part, 3, s, qkv.shape[1], bias, dtype, (s,), dev, None)
+            out = ops.rope_cache_paged_attn_decode_splitk(p, nq, nkv, 128, pos, csc, cache[0], cache[1], slots, table, lens, bound, 128 ** -0.5,
+                                                          order=o, **kw)
+        else:
+            q, k, v = qkv.split([nq * 128, nkv * 128, nkv * 128], -1)
+            out = torch.full((s, nq * 128), 7.0 if o is None else 9.0, dtype=dtype, device=dev)
+            ops.rope_cache_paged_attn_decode(out, q, k, v, pos, csc, cache[0], cache[1], slots, table, lens, bound, 128 ** -0.5, order=o, **kw)
+        got.append((out.view(torch.int16), cache.view(torch.int16)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert not torch.equal(got[1][1], kv.view(torch.int16))
+
+
+# partitions that merge behind their last arrival, by counters of (sequence, head group)
+def test_fused_merge():
+    from vllm_omni_amd import ops
+
+    dev = torch.device("cuda", 0)
+    s, nq, nkv, hd, bound = 70, 28, 4, 128, 1000
+    q, kc, vc, bt, lens = _case(s, nq, nkv, hd, bound, dev)
+    order = ops.decode_seq_order(lens, nq, nkv, hd, 16, bound)
+    assert order is not None and -(-bound // ops.decode_auto_partition(s, nkv, bound, 16, head_dim=hd)) == 2
+    want = ops.paged_attn_decode(torch.empty_like(q), q, kc, vc, bt, lens, bound, hd ** -0.5, fused_merge=False)
+    ws = ops.new_decode_workspace(ops.decode_workspace_bytes(s, nq, hd, bound, ops.decode_auto_partition(s, nkv, bound, 16, head_dim=hd)), dev)
+    for _ in range(2):      # the counters are back at zero
+        got = ops.paged_attn_decode(torch.empty_like(q), q, kc, vc, bt, lens, bound, hd ** -0.5, workspace=ws, fused_merge=True, order=order)
+        assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
+# whole steps through the runner: 67 requests of uneven length, captured (filled up to 72 rows) and eager, with and without an order
+@pytest.mark.parametrize("eager", [False, True], ids=["captured", "eager"])
+@pytest.mark.parametrize("qk_norm", [False, True], ids=["plain", "qk-norm"])
+def test_runner_steps(eager, qk_norm, monkeypatch):
+    from vllm_omni_amd import ops
+    from vllm_omni_amd.model_runner import GPUARModelRunner
+    from vllm_omni_amd.sched_output import CachedRequestData, NewRequestData, SamplingParams, SchedulerOutput
+    from vllm_omni_amd.talker import TalkerConfig
+
+    dev = torch.device("cuda", 0)
+    n, longest, steps = 67, 330, 4
+    ctx = torch.randint(1, longest - steps, (n,), generator=torch.Generator().manual_seed(2)).tolist()
+    per = (longest + 15) // 16
+    made, real = [], ops.decode_seq_order
+
+    def passes(ordered):
+        def spy(*a, **k):
+            o = real(*a, **k) if ordered else None
+            made.append(o)
+            return o
+
+        monkeypatch.setattr(ops, "decode_seq_order", spy)
+        c = TalkerConfig.from_json("mini_talker")
+        c.mrope_section, c.head_dim, c.num_attention_heads, c.num_key_value_heads, c.qk_norm = None, 128, 8, 4, qk_norm
+        r = GPUARModelRunner(c, dev, torch.bfloat16, max_num_reqs=128, max_model_len=longest, max_num_batched_tokens=128, block_size=16,
+                             enforce_eager=eager, seed=0)
+        r.load_model()
+        r.initialize_kv_cache(n * per + 1)
+        g = torch.Generator(device=dev).manual_seed(7)
+        for kv in r.kv_caches:
+            for x in kv:
+                x.copy_(torch.randn(x.shape, generator=g, device=dev))
+        ids, out = [f"r{i}" for i in range(n)], []
+        for step in range(steps):
+            sched = {i: 1 for i in ids}
+            if step == 0:
+                so = SchedulerOutput(scheduled_new_reqs=[NewRequestData(i, list(range(k + 1)), SamplingParams(temperature=0.0),
+                                                                        (list(range(1 + j * per, 1 + (j + 1) * per)),), k)
+                                                         for j, (i, k) in enumerate(zip(ids, ctx))],
+                                     num_scheduled_tokens=sched, total_num_scheduled_tokens=n)
+            else:
+                so = SchedulerOutput(scheduled_cached_reqs=CachedRequestData(req_ids=ids, new_token_ids=[], new_block_ids=[None] * n,
+                                                                             num_computed_tokens=[k + step for k in ctx], num_output_tokens=[step] * n),
+                                     num_scheduled_tokens=sched, total_num_scheduled_tokens=n)
+            r.execute_model(so)
+            st = r.execute_model_state
+            out += [st.logits[:n].clone(), st.hidden_states[:n].clone()]
+            out.append(torch.tensor(r.sample_tokens().sampled_token_ids))
+        return out + [x[1:].clone() for kv in r.kv_caches for x in kv]
+
+    want = passes(False)
+    made.clear()
+    got = passes(True)
+    assert made and all(o is not None for o in made)
+    assert len(made) == (steps if eager else 3)      # one a forward pass whatever its layers: two to warm up and the captured one
+    for a, b in zip(want, got):
+        assert torch.equal(a, b)
