@@ -72,3 +72,87 @@ def test_experts(h, i, e, top, t, act, monkeypatch):
         got = r.part[rows].double()
         # activations are stored in bf16 in front of the second product
         assert (got - want).norm() / want.norm() < 2 ** -7
+
+
+# where gated tiles of under 64 columns begin to be turned, and end: 192 tiles and more of K 4096 to 64 rows, longer K to 128
+@pytest.mark.parametrize("inter,k,rows", [(6144, 4096, (64,)), (7168, 4096, (1, 64, 65)), (3584, 4096, (32, 65)), (4096, 8192, (128, 129)), (2048, 12288, (16, 200))])
+def test_gated_lines(inter, k, rows):
+    from vllm_omni_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(inter + k)
+    w = _draw(2 * inter, k, g=g)
+    c = torch.randint(0, inter, (257,), generator=g, device=DEV)
+    for m in rows:
+        x = _draw(m, k, g=g)
+        gate, up = ((x.double() @ w[c + o].double().t()).to(w.dtype).double() for o in (0, inter))
+        ref, got = torch.nn.functional.silu(gate) * up, ops.linear_silu_mul(x, w)[:, c].double()
+        scale = ref.norm() / ref.numel() ** 0.5      # (as in test_linear)
+        assert ((got - ref).norm() / ref.norm()) < 2 ** -7 and ((got - ref).abs() / (ref.abs() + scale)).max() < 2 ** -5
+
+
+# 32-bit slabs and the launches behind them: the bits of the linear, and the squared relu's sums
+@pytest.mark.parametrize("n,k", [(15360, 4096), (8192, 8192), (4096, 16384)])
+@pytest.mark.parametrize("m", [1, 64, 128, 200])
+def test_slabs(n, k, m):
+    from vllm_omni_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    x, w, b = _draw(m, k, g=g), _draw(n, k, g=g), _draw(n, g=g)
+    part = ops.linear_partials(x, w, b)
+    got = part.materialize()
+    assert torch.equal(got, ops.linear(x, w, b))
+    cols = torch.randint(0, n, (257,), generator=g, device=DEV)
+    want = x.double() @ w[cols].double().t()
+    _close(got[:, cols], want + b[cols].double())
+    _close(ops.linear_relu_squared(x, w)[:, cols], torch.relu(want) ** 2)
+
+
+# int8: K counts pairs of bytes, so rows of 8192 and 16384 bytes are turned; integer sums have one value whatever their order
+@pytest.mark.parametrize("n,k", [(33056, 8192), (10368, 8192), (4112, 8192), (4096, 16384)])
+@pytest.mark.parametrize("m", [1, 64, 128, 200, 300])
+def test_int8(n, k, m):
+    from vllm_omni_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    xq, wq = (torch.randint(-128, 128, s, generator=g, device=DEV, dtype=torch.int32).to(torch.int8) for s in ((m, k), (n, k)))
+    xs, ws = torch.rand(m, generator=g, device=DEV) * 0.05 + 1e-3, torch.rand(n, generator=g, device=DEV) * 0.01 + 1e-4
+    b = _draw(n, g=g)
+    got = ops.int8_linear_q(xq, xs, wq, ws, b, torch.bfloat16)
+    assert torch.equal(got, ops.int8_gemm_dequant(xq, xs, wq, ws, b, torch.bfloat16))
+    cols = torch.randint(0, n, (129,), generator=g, device=DEV)
+    want = (xq.double() @ wq[cols].double().t()) * xs[:, None].double() * ws[cols].double() + b[cols].double()
+    _close(got[:, cols], want)
+
+
+@pytest.mark.parametrize("inter,k,m", [(16528, 8192, 1), (16528, 8192, 64), (12288, 8192, 200), (5184, 16384, 128), (2048, 8192, 300)])
+def test_int8_gated(inter, k, m):
+    from vllm_omni_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(inter + m)
+    x = _draw(m, k, g=g)
+    wq, ws = ops.dynamic_int8_quant(_draw(2 * inter, k, g=g) * 0.05)
+    gt, up = ops.int8_gemm_dequant(*ops.dynamic_int8_quant(x), wq, ws, None, torch.bfloat16).float().split(inter, -1)
+    want, got = torch.nn.functional.silu(gt) * up, ops.int8_linear_silu_mul(x, wq, ws).float()
+    # both round the two integer products to 16 bits first: one more rounding, and the error of the fast exponential (far below it)
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -7 + 1e-6).all()
+
+
+# every row by itself: rounding of the gate, the activations and the results is about 2^-8 of a row's norm
+@pytest.mark.parametrize("h,i,e,top,t", [(4096, 1536, 64, 8, 64), (4096, 1536, 64, 8, 200), (2048, 768, 64, 8, 200), (4096, 256, 16, 4, 60), (4096, 512, 8, 4, 700)])
+@pytest.mark.parametrize("act", ["silu_gated", "relu_squared"])
+def test_every_row_of_the_experts(h, i, e, top, t, act):
+    from vllm_omni_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(h + t)
+    ups = 2 if act == "silu_gated" else 1
+    x = _draw(t, h, g=g)
+    wu, wd = _draw(e, ups * i, h, g=g) * h ** -0.5, _draw(e, h, i, g=g) * i ** -0.5
+    ids = torch.rand(t, e, generator=g, device=DEV).argsort(-1)[:, :top].int().contiguous()
+    r = ops.moe_expert_rows(x, ids, torch.rand(t, top, generator=g, device=DEV), wu, wd, act)
+    got = r.part[r.row_of_pair.long()].view(t, top, h).double()
+    for j in range(e):
+        tok, place = (ids == j).nonzero(as_tuple=True)
+        u = x[tok].double() @ wu[j].double().t()
+        mid = torch.nn.functional.silu(u[:, :i]) * u[:, i:] if ups == 2 else torch.relu(u) ** 2
+        want = mid @ wd[j].double().t()
+        assert ((got[tok, place] - want).norm(dim=-1) <= want.norm(dim=-1) * 2 ** -7).all(), j
