@@ -13,6 +13,9 @@
 //     that waits for a place in it issues no products either (16 in a row 0.96, spread 1.42 PFLOP/s at 65536 x 8192 x 4096).
 //   * A workgroup stays and takes its XCD's items in turn; the next item's first two stages are on their way through the last two
 //     steps, and its places are fetched a whole item ahead.  Results turn in LDS and leave as 256-byte row segments.
+//   * Experts' weight rows a multiple of 4096 bytes apart: the k blocks of a tile begin where those of the other grouped kernels do
+//     (skinny_grouped.h; one order of sums).  Up, relu squared, 4096 x 1536, 1000 tokens, 8 chosen 191 | 186 us, gated, 6 chosen 313 | 294, 2048
+//     x 768, 1000 tokens 57 | 50; from 2048 tokens on 0.99 to 1.01 of the time without.
 //   * A row tile's live rows are counted in units of 64: four code paths, so that an expert's last tile costs what it holds.
 // Experts' both products, 4096 x 1536, 64 experts, 8 chosen (relu squared): 8192 rows 2176 -> 1603 us, 1024 rows 877 -> 400 us;
 // gated, 6 chosen: 8192 rows 2289 -> 1819 us, 1365 rows 1213 -> 533 us; 1024 x 384, 128 experts, 8 chosen: 2048 rows 199 -> 113 us
@@ -222,9 +225,17 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr int A = NM * 5 / 8, B = NM / 4;      // where the two barriers of a step stand among its 2 NM products
+  int ahead = TURN ? tall_block<TURN>(t, 2) : 0;      // where the next step's loads lie along K
   // KIND 0: a step in the middle; 1, 2: the last two, which load the next item's first two
   auto step = [&](auto kind, int it, char* cur, char* nxt) __attribute__((always_inline)) {
     constexpr int KIND = decltype(kind)::value;
+    int kb = KIND == 0 ? t.kb + (it + 2) * 128 : tall_block<TURN>(nt, KIND - 1);
+    if constexpr (TURN && KIND == 0) {
+      // (here, among the products: behind the barrier, in front of the loads, it costs 1 to 2 % of a launch that the matrix cores hold)
+      kb = ahead;
+      ahead = ahead + 128 == 128 * n_it ? 0 : ahead + 128;
+      asm volatile("" : "+s"(kb), "+s"(ahead));
+    }
     read(1, cur);
     mul(0, 0, A);
 #pragma unroll
@@ -237,7 +248,6 @@ __device__ __forceinline__ void tall_tile(const TallParams& p, char* s0, char* s
     __builtin_amdgcn_s_waitcnt(kLgkm0);
     barrier();                                   // everybody has read this stage
     // (loads spread over the step: a wave that finds the memory pipe's queue full issues no product either)
-    const int kb = KIND == 0 ? tall_block<TURN>(t, it + 2) : tall_block<TURN>(nt, KIND - 1);
     if (KIND == 0 || more) tall_issue_w(wo, wr, kb, cur);
     if (KIND == 2) {
       if (more) tall_issue_x<8>(p, x, kb, cur);
