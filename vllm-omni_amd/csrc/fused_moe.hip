@@ -601,8 +601,7 @@ extern "C" int mi_moe_expert_gemm(void* out, const void* a_rows, const void* wei
       // chip.  Cold weights, us, ring | stream.  Down: 4096 x 1536, 64 experts, 8 chosen, 7 tokens 107 | 88, 64 157 | 129, 200 177 | 142, 6 chosen, 32
       // tokens 154 | 123, 253 193 | 152; 1024 x 384, 128 experts, 512 tokens 26.9 | 22.8, but 1 token 6.9 | 7.7 and 4096 x 1536 20.7 | 21.7.  Up,
       // 64-row tiles: 1536 x 4096, 200 tokens 172 | 143, gated 400 tokens 330 | 289, 384 x 1024 gated 44.2 | 39.8.  32-row tiles of the up
-      // forms stay with the ring: gated 5 tokens 131 | 131, 32 tokens 255 | 270, 253 tokens 316 | 314, 384 x 1024 36.4 | 37.3; the
-      // squared relu's alone would gain once most experts are chosen (64 tokens 183 | 151, 1 token 34 | 40): below, for K of whole 2048s.
+      // forms stay with the ring where K is no multiple of 2048 (gated 384 x 1024 36.4 | 37.3).
       // One round of tiles or less can be behind (the bound on them counts up to 1.75 times as many as there are).  140 sizes, 28 to 50 rows an
       // expert in 64-row tiles, the ring's time as 1: under 512 tiles down 0.77 to 1.22 (1152 x 1024, 8 experts 12.3 | 15.0 us), up 0.81 to 1.40 (448
       // x 768 gated, 64 experts 21.6 | 30.3, 512 x 2048 gated, 8 experts 19.6 | 25.7); past them 0.70 to 0.96 and 0.80 to 0.94, but for up

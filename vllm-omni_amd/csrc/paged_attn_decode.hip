@@ -738,7 +738,6 @@ extern "C" int mi_decode_seq_order(int32_t* lens_and_order, const int32_t* seq_l
   using namespace mi;
   if (!lens_and_order || !seq_lens || num_seqs <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || max_seq_len <= 0 || num_q_heads % num_kv_heads != 0)
     return MI_ERR_INVALID_ARG;
-  if (head_dim != 64 && head_dim != 128) return MI_ERR_UNSUPPORTED;
   const int32_t ps = mi_paged_attn_decode_effective_partition(num_seqs, num_kv_heads, max_seq_len, head_dim, block_size, partition_size, flags);
   if (!(flags & MI_DECODE_PACKED_PV) || (flags & MI_DECODE_FORCE_VALU) || block_size < 16 || ps <= 0 || ps % 32) return MI_ERR_UNSUPPORTED;
   const int parts = (max_seq_len + ps - 1) / ps, groups = num_q_heads / heads_per_wave(num_q_heads / num_kv_heads, 16);

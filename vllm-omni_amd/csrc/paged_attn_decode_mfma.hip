@@ -926,12 +926,14 @@ int32_t decode_mfma_turn(int64_t groups, int num_parts) {
 
 // Contexts of uneven length: a launch of more workgroups than CUs lasts as long as the CU with the largest sum, or as its last arrivals.  Longest
 // first the late ones are short, and with every other round of 256 turned the sums of the rounds that are resident together even out.
-// Not where a CU has one workgroup at most, and partitions of three or more gain nothing (23 x 4 KV heads in 6, 425 to 1700 tokens 15.2 | 16.0 us).
-// Equal lengths cost nothing (256 x 4, 4096 tokens 322 | 322, 300 tokens 29.5 | 29.5).  As they are | ordered, us:
-// 120 x 4 in 2, 175 to 700 tokens 27.8 | 22.9; 70 x 4 in 2, 100 to 3000 67 | 58; 256 x 4, 1000 to 4096 246 | 231, 75 to 300 23.1 | 22.3; 161 x 8, 300 to
-// 1500 121 | 98; 200 x 8, 750 to 3001 276 | 242; 300 x 8, 500 to 2000 263 | 242.  Longest first alone, no round turned: 120 x 4 25.2.  Heads of 64 dims
-// gain with uneven contexts (512 x 2, 1000 to 4096 127 | 121), but their waves, all resident at once, feel the look-up in front of their loads: a
-// step of 512 equal contexts 6474 | 6515.  Bounds of up to 256 tokens: not tried, a launch takes 7 to 11 us.
+// Not where a CU has one workgroup at most, and partitions of three or more gain nothing (23 x 4 KV heads in 6, 425 to 1700 tokens 15.2 | 16.0 us):
+// so not at bounds above 16384 tokens either, however short the contexts (a captured step's bound is the longest context its server allows).
+// Equal lengths stay as they are and pay for the look-up alone, 0 to 0.5 us a launch (65 x 4 in 2, 300 tokens 15.7 | 15.9; 161 x 8 44.2 | 44.6; 256 x 4, 3000
+// tokens 235 | 235).  As they are | ordered, us: 120 x 4 in 2, 175 to 700 tokens 28.0 | 23.2, at a bound of 8192 39.8 | 35.0; 65 x 4 in 2, 50 to 8000
+// 150 | 124; 256 x 4, 750 to 3001 173 | 162, 20 to 250 (bound 2048) 18.8 | 17.8; 161 x 8, 175 to 700 61 | 52; 200 x 8, 750 to 3001 278 | 243; 300 x 8 403 |
+// 364; 1000 x 1, 50 to 8000 (bound 16384, in 2) 523 | 379.  Longest first alone, no round turned: 120 x 4 25.2.  Heads of 64 dims gain with uneven contexts
+// (512 x 2, 1000 to 4096 127 | 121), but their waves, all resident at once, feel the look-up in front of their loads: a step of 512 equal contexts
+// 6474 | 6515.  Bounds of up to 256 tokens: not tried, a launch takes 7 to 11 us.
 DecodeOrder decode_mfma_order(int num_seqs, int groups_per_seq, int num_parts, bool group_parts, int head_dim, int max_seq_len) {
   const int ring = ring_bytes<128>, waves = group_parts ? num_parts : 1;
   const int64_t each = (int64_t)groups_per_seq * (num_parts / waves);      // workgroups of a sequence

@@ -211,7 +211,7 @@ struct V2 {
   }
 };
 
-template <typename Tag, typename OT, int G, int G0, bool GATED, bool TURN>
+template <typename Tag, typename OT, int G, int G0, bool GATED>
 __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_v2_kernel(const SkinnyParams p) {
   using C = V2<Tag, OT, G, G0, GATED>;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -257,11 +257,12 @@ __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_
         src[i] = reinterpret_cast<const char*>(p.w + (int64_t)n * p.K + 64 * (int64_t)b_lo + 8 * lc);
       }
     }
-    int kk = 0;      // TURN: k block of the next step to issue
-    if constexpr (TURN) kk = (int)((uint32_t)wg % (uint32_t)max(n_it, 1));
+    // (one form for turned launches and others: with k blocks counted by themselves, and with a form without the wrap, hipcc's code was 1 to 2 %
+    // slower, 37888 x 3584, 256 rows 73.9 | 74.7, gated 72.1 | 73.6 us)
+    const int first = p.turn ? (int)((uint32_t)wg % (uint32_t)max(n_it, 1)) : 0;
     auto issue = [&](int it, int stage) {
       char* st = smem + stage * C::kStage;
-      if constexpr (!TURN) kk = it;
+      const int kk = it + first - (it + first < n_it ? 0 : n_it);
 #pragma unroll
       for (int i = 0; i < C::PPL; ++i) {
         if (l + kV2Loaders * i < C::XI)
@@ -270,9 +271,6 @@ __global__ __launch_bounds__(64 * (kV2Consumers + kV2Loaders)) void skinny_gemm_
         else
           __builtin_amdgcn_global_load_lds((gbl_void*)(src[i] + 128 * (int64_t)kk),
                                            (lds_void*)(st + (l + kV2Loaders * i) * 1024), 16, 0, MI_SKINNY_W_AUX);
-      }
-      if constexpr (TURN) {
-        if (++kk == n_it) kk = 0;
       }
     };
     const uint32_t full0 = lds0 + C::kFlags, free0 = lds0 + C::kFlags + C::NST * 16;
@@ -474,20 +472,15 @@ int linear_v2() {   // MI_LINEAR_V2=0: the first-generation kernel at 129-256 ro
   return e ? atoi(e) : 1;
 }
 
-template <typename Tag, typename OT, int G, int G0, bool GATED, bool TURN>
-int launch_v2_turn(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
+template <typename Tag, typename OT, int G, int G0, bool GATED>
+int launch_v2(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
   using C = V2<Tag, OT, G, G0, GATED>;
-  auto kern = skinny_gemm_v2_kernel<Tag, OT, G, G0, GATED, TURN>;
+  auto kern = skinny_gemm_v2_kernel<Tag, OT, G, G0, GATED>;
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
   if (attr != hipSuccess) return MI_ERR_LAUNCH;
   hipLaunchKernelGGL(kern, grid, dim3(64 * (kV2Consumers + kV2Loaders)), C::kLds, s, p);
   return launch_status();
-}
-
-template <typename Tag, typename OT, int G, int G0, bool GATED>
-int launch_v2(const SkinnyParams& p, const dim3 grid, hipStream_t s) {
-  return p.turn ? launch_v2_turn<Tag, OT, G, G0, GATED, true>(p, grid, s) : launch_v2_turn<Tag, OT, G, G0, GATED, false>(p, grid, s);
 }
 
 // `dtype`: the type of the 16-bit OUTPUT (and of the operands, unless `int8`: then x / w are int8 rows and the sums

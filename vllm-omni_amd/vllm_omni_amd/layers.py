@@ -498,9 +498,11 @@ def _narrow_kernel_wins(m: int, n: int, k: int) -> bool:
     # 33 to 128 rows of a K that splits into few slices (narrow_plan in skinny_gemm.hip), timed at 30 widths and five K between 3584 and 4096.
     # Library | kernel, us, cold weights: 4608 x 3584, 64 rows 18.9 | 14.4, 128 rows 22.9 | 18.8; 5120 x 4096 17.4 | 15.5 and 25.0 | 19.7; 4096 x
     # 4096 15.0 | 14.1 and 24.5 | 17.7; 6144 x 4096 18.0 | 17.3 and 25.8 | 23.6 (worst: 4352 x 4096, 72 rows 3 % behind).  Wider weights run on the
-    # wide tile and lose: 7296 x 4096, 64 rows 18.5 | 20.5, 8192 x 4096 19.2 | 22.7, 12288 x 4096 25.7 | 29.3, 12288 x 3584, 128 rows 29.0 | 33.3 -
-    # but for what is past 8192 columns, where the library's time steps up and the kernel's does not: 8320 x 4096, 64 rows 0.83 of it, 10368 x 4096
-    # 26.8 | 22.9 and 31.1 | 28.4 (K 3584 is 3 to 5 % behind at 112 rows).  K 3072 is level (6144 x 3072, 128 rows 21.1 | 21.6), K 2048 behind
+    # wide tile and lose: 7296 x 4096, 64 rows 18.7 | 21.5, 8192 x 4096 19.9 | 23.0, 12288 x 4096 26.1 | 27.5, 12288 x 3584, 128 rows 31.4 | 34.6 -
+    # but for what is past 8192 columns, where the library's time steps up and the kernel's does not: 8320 x 4096, 64 rows 0.80 of it, 10368 x 4096
+    # 28.0 | 23.6 and 30.5 | 27.4 (K 3584 is 3 to 5 % behind at 112 rows).  Past 10496 columns both fall apart by size (11264 x 4096, 64 and 128 rows 29.5 | 26.7
+    # and 30.9 | 32.7, 15360 28.0 | 30.5 and 33.2 | 36.5, 20480 43.4 | 35.1 and 43.8 | 44.4, 33056 71 | 45 and 70 | 55): the library's, not swept
+    # finely enough for a line.  K 3072 is level (6144 x 3072, 128 rows 21.3 | 22.6), K 2048 behind
     # (8192 x 2048, 64 rows 13.6 | 15.0), and at 256 rows whole decode steps are behind, 1.5 to 3 %
     # The split-K reduce (+ bias) of qkv_proj (4608 x 3584) inside the decode attention launch, both launches, us, library | kernel and its
     # reduce | this: 64 x 2048 tokens 68.6 | 64.1 | 61.9, 120 x up to 700 47.7 | 47.2 | 46.1, 128 x 2048 113 | 111 | 107; up to 32 rows the wait
