@@ -74,8 +74,8 @@ def test_experts(h, i, e, top, t, act, monkeypatch):
         assert (got - want).norm() / want.norm() < 2 ** -7
 
 
-# where gated tiles of under 64 columns begin to be turned, and end: 192 tiles and more of K 4096 to 64 rows, longer K to 128
-@pytest.mark.parametrize("inter,k,rows", [(6144, 4096, (64,)), (7168, 4096, (1, 64, 65)), (3584, 4096, (32, 65)), (4096, 8192, (128, 129)), (2048, 12288, (16, 200))])
+# where gated tiles of under 64 columns begin to be turned, and end: 209 to 249 tiles of K 4096 to 64 rows, longer K to 128 and 224
+@pytest.mark.parametrize("inter,k,rows", [(6656, 4096, (64,)), (6688, 4096, (33, 64, 65)), (7968, 4096, (1, 64)), (8000, 4096, (64,)), (3584, 4096, (32, 65)), (4096, 8192, (128, 224, 225)), (2048, 12288, (16, 128, 129))])
 def test_gated_lines(inter, k, rows):
     from vllm_omni_amd import ops
 

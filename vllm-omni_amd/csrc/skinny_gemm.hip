@@ -457,13 +457,15 @@ namespace {
 // five slices, 128 rows 22.4 | 23.6, 15360 x 4096, 200 rows 45.0 | 46.2, 37888 x 3584 45.4 | 45.7; 12288 x 2048 and 2048 x 6144 level.  Two blocks
 // apart: 4096 x 16384 38.0, gated 33056 x 4096 46.5.
 // Where x is most of what a workgroup takes in, its blocks come best while all workgroups ask for the same ones.  So gated tiles of under 64
-// columns are turned up to 128 rows, and of K 4096 up to 64 rows and past 192 tiles: gated 8192 x 4096, 64 rows 24.9 | 26.8, 12288 x 4096
-// 27.0 | 29.0, 128 rows 31.7 | 34.8, 15360 x 4096, 128 rows 33.7 | 35.5, 12288 x 12288, 256 rows 133 | 179; but 14336 x 4096, 32 rows 26.5 | 24.1,
-// 14336 x 8192, 64 rows 56.4 | 45.9, 128 rows 62.5 | 57.3.  And two slices of K 4096 in 128-row images past 112 tiles: 12288 x 4096, 128
-// rows 32.5 | 33.2, but 14336 x 4096 36.2 | 35.5.
+// columns are turned up to 128 rows, K of whole 8192s up to 224, and K 4096 up to 64 rows and at 209 to 249 tiles: gated 8192 x 4096, 64 rows
+// 24.9 | 26.8, 12288 x 4096 27.0 | 29.0, 128 rows 31.7 | 34.8, 15360 x 4096, 128 rows 33.7 | 35.5, 12288 x 12288, 144 rows 116 | 114, 256 133 |
+// 182, 8192 x 8192, 256 rows 82.5 | 83.8, 12672 x 4096 (198 tiles), 32 rows 23.6 | 25.0, 16256 x 4096 (254), 64 rows 31.6 | 34.9; but 13440 x 4096
+// (210), 32 rows 27.2 | 24.0, 14336 x 8192, 64 rows 56.4 | 45.9, 208 rows 87.8 | 84.8.  Under 209 tiles the times as they are go up and down by 15 % with
+// the number of tiles (162 tiles 23.3 | 22.1, 168 22.9 | 22.4, 198 as above).  And two slices of K 4096 in 128-row images past 112 tiles: 12288 x 4096,
+// 128 rows 32.5 | 33.2, but 14336 x 4096 36.2 | 35.5.
 int skinny_turn(int m, int k, const SkinnyPlan& pl, bool gated) {
   if (!skinny_in_step(k, pl.split) || (pl.split > 1 && pl.mt > 8)) return 0;
-  if (gated && pl.nslab < 4) return m <= 128 && (k > 4096 || (m <= 64 && pl.tiles > 192));
+  if (gated && pl.nslab < 4) return k > 4096 ? m <= (k % 8192 ? 128 : 224) : m <= 64 && pl.tiles > 208 && pl.tiles < 250;
   return k > 4096 || pl.split == 1 || pl.mt <= 4 || pl.tiles >= 112;
 }
 
