@@ -34,7 +34,7 @@ struct StreamParams {
   int32_t N, K;
   int32_t rpt, gather_div;      // rows per tile; > 0: source row = pair index / gather_div, else the row itself
   int32_t nx;                   // weight tiles of a row tile
-  int32_t turn;                 // the TURN form: a tile's k blocks begin with grouped_first_block and go round
+  int32_t turn;                 // a tile's k blocks begin with grouped_first_block and go round
   uint32_t div_magic;           // 2^32 / gather_div, rounded up: exact for pair indices below 2^28
   uint32_t map_bytes;
   const int32_t* row_map;       // [max_rows] pair index or -1; the pairs of a tile in front
@@ -80,7 +80,7 @@ __device__ __forceinline__ void lds_read_frags(uint32_t w0, uint32_t w1, uint32_
       : "memory");
 }
 
-template <typename Tag, int FORM, bool TURN>
+template <typename Tag, int FORM>
 __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParams p) {
   scalar_cache_acquire();
   using E = Elem<Tag>;
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
   StreamItem lt;
   __amdgpu_buffer_rsrc_t wr = x_r;
   uint32_t xo[2], xn[2];
-  int w_first = 0, x_first = 0, xn_first = 0;      // the blocks that the tiles begin with
+  int w_first = 0, x_first = 0, xn_first = 0;      // where the tiles begin along K (bytes)
   int pieces = 0, n_loaded = 0;      // n_loaded: tiles taken up so far
   const auto take = [&]() {
     const int i = item + n_loaded * per;
@@ -157,34 +157,36 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
     const StreamRange r = stream_range(lt.col, lt.cut, p.N, p.K, GATED);
     wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.w + (int64_t)lt.expert * p.w_expert_stride + r.first), 0, (int)r.bytes, 0x00020000);
     pieces = r.pieces;
-    if constexpr (TURN) w_first = xn_first = grouped_first_block(GATED, lt.expert, lt.col, p.N, n_it);
+    if (p.turn) w_first = xn_first = 128 * grouped_first_block(GATED, lt.expert, lt.col, p.N, n_it);
     ++n_loaded;
     if (item + n_loaded * per < items) load_map(item + n_loaded * per, n_loaded % 3);
   };
-  int w_it = 0, w_slot = 0, x_it = 0, x_slot = 0;
+  int w_slot = 0, x_slot = 0;
+  // the next blocks (bytes along K), counted from where their tile begins: with a sum of both in every block the plain form spilled twice as many
+  // scalars (1024 x 384, 1 token, down 6.41 | 6.47 us)
+  int w_at = 0, x_at = 0;
   const auto issue_w = [&]() {
-    const int kb = 128 * (TURN ? w_it + w_first - (w_it + w_first < n_it ? 0 : n_it) : w_it);
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(lds + w_slot * kWStage + (wid + 4 * i) * 1024), 16, i < pieces ? wo[i] : kDead,
-                                               kb, 0, MI_SKINNY_W_AUX);
+                                               w_at, 0, MI_SKINNY_W_AUX);
     w_slot = (w_slot + 1) & 3;
-    if (++w_it == n_it) {
-      w_it = 0;
+    w_at = w_at + 128 == 128 * n_it ? 0 : w_at + 128;
+    if (w_at == w_first) {
       take();
+      w_at = w_first;
     }
   };
   const auto issue_x = [&]() {
-    const int kb = 128 * (TURN ? x_it + x_first - (x_it + x_first < n_it ? 0 : n_it) : x_it);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_r, (lds_void*)(lds + kXRing + x_slot * kXStage + (wid + 4 * i) * 1024), 16, xo[i], kb, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_r, (lds_void*)(lds + kXRing + x_slot * kXStage + (wid + 4 * i) * 1024), 16, xo[i], x_at, 0, 0);
     x_slot = x_slot == 2 ? 0 : x_slot + 1;
-    if (++x_it == n_it) {
-      x_it = 0;
+    x_at = x_at + 128 == 128 * n_it ? 0 : x_at + 128;
+    if (x_at == x_first) {
       xo[0] = xn[0];
       xo[1] = xn[1];
-      x_first = xn_first;
+      x_at = x_first = xn_first;
     }
   };
 
@@ -193,7 +195,8 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
   take();
   xo[0] = xn[0];
   xo[1] = xn[1];
-  x_first = xn_first;
+  x_at = x_first = xn_first;
+  w_at = w_first;
   StreamItem t = lt;
   issue_w();
   issue_x();
@@ -311,17 +314,13 @@ __global__ __launch_bounds__(256, 1) void expert_stream_kernel(const StreamParam
   __builtin_amdgcn_s_waitcnt(stream_vmcnt(0));      // no load may land in this LDS once it is another workgroup's
 }
 
-template <typename Tag, int FORM, bool TURN>
-int launch_stream_turn(const StreamParams& p, const dim3 grid, hipStream_t s) {
-  auto kern = expert_stream_kernel<Tag, FORM, TURN>;
+template <typename Tag, int FORM>
+int launch_stream_form(const StreamParams& p, const dim3 grid, hipStream_t s) {
+  auto kern = expert_stream_kernel<Tag, FORM>;
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kStreamLds);
   if (attr != hipSuccess) return MI_ERR_LAUNCH;
   hipLaunchKernelGGL(kern, grid, dim3(256), kStreamLds, s, p);
   return launch_status();
-}
-template <typename Tag, int FORM>
-int launch_stream_form(const StreamParams& p, const dim3 grid, hipStream_t s) {
-  return p.turn ? launch_stream_turn<Tag, FORM, true>(p, grid, s) : launch_stream_turn<Tag, FORM, false>(p, grid, s);
 }
 template <typename Tag>
 int launch_stream(const StreamParams& p, int form, const dim3 grid, hipStream_t s) {
